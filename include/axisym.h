@@ -396,25 +396,22 @@ axs_status axs_rigid_stepper_reset_scalars(axs_rigid_stepper* st, void* stream);
  * -> phi pinned to the sphere of eta where phi > -3 dx -> narrow-band
  * reinit (as axs_reinit_distance_f64) -> chi = smooth Heaviside(phi,
  * moll_zone) -> least-squares extrapolation of eta on the doubled grid
- * (sweeps until one fits nothing: lsq_sweeps queued launches, a longer
- * loop finished by one workgroup) -> solid stress
+ * (sweeps until one fits nothing) -> solid stress
  * blended by chi -> omega += dt curl(div sigma) -> ENO3 -> RK2.  FP64.
  * The caller owns the state buffers ((nr, nz) doubles; scalars
  * AXS_RIGID_SCALARS doubles: t, dt, dt/dx, nu dt/2, nu dt, max|u|, step
- * counter, sweeps used in the last step, steps whose loop outran the
- * lsq_sweeps queued launches and was finished by the one-workgroup tail;
+ * counter, sweeps used in the last step, steps whose loop took lsq_sweeps
+ * sweeps or more (0 with lsq_grow);
  * r (nr), z (nz), kill_wz (2 kill_width), kill_wr (kill_width)); the
  * stepper owns its scratch.  nz must equal 2 nr (the extrapolation uses z
  * as both axes of the doubled grid, as the reference does). */
 typedef struct axs_soft_stepper axs_soft_stepper;
 typedef struct {
   int nr, nz, kill_width;
-  int lsq_sweeps;        /* extrapolation sweeps queued per step as launches */
+  int lsq_sweeps;        /* steps whose extrapolation takes this many sweeps or more are
+                            counted in the scalars; the loop always runs to its end */
   int reinit_iterations; /* < 0: 2 ceil(reinit_band / dx) + 8 */
-  int lsq_grow;          /* nonzero: graph runs raise lsq_sweeps to the most sweeps a step
-                            has needed so far + 4, rounded up to 4 (at most 4096), as they
-                            learn it (read back without blocking; the graphs are captured
-                            again); eager runs keep it */
+  int lsq_grow;          /* nonzero: count no step */
   double dx, nu, G, rho_f, CFL, eps;
   double r_ball, z_cm, r_cm;               /* phi pin: r_ball - |eta - (z_cm, r_cm)| */
   double moll_zone, extrap_zone, reinit_band;
@@ -449,8 +446,7 @@ axs_status axs_soft_stepper_run(axs_soft_stepper* st, int nsteps, int use_graph,
  * gives the same bits alone and in any mix.  Cases join (add) and leave
  * (remove) between runs; both wait for the device to finish queued work.
  * The configuration and buffers are those of axs_soft_stepper_create
- * (lsq_sweeps and lsq_grow are the batch's: the queue starts at 12 sweeps
- * and grows as in lsq_grow); the buffers must stay valid until the case is
+ * (lsq_sweeps and lsq_grow are not used); the buffers must stay valid until the case is
  * removed.  At most 1024 cases; nz up to 4096 (nr up to 2048). */
 typedef struct axs_soft_batch axs_soft_batch;
 axs_status axs_soft_batch_create(int max_cases, axs_soft_batch** out);
@@ -483,8 +479,9 @@ axs_status axs_soft_batch_remove(axs_soft_batch* b, int case_id);
 /* Queues nsteps steps of every case on `stream` (use_graph: captured after
  * each change of the case set, replayed). */
 axs_status axs_soft_batch_run(axs_soft_batch* b, int nsteps, int use_graph, void* stream);
-/* Cases, extrapolation sweeps queued per step, graph launches and captures
- * so far (any pointer may be null). */
+/* Cases, the most extrapolation sweeps a step has taken + 4 rounded up to 4
+ * (at least 12), graph launches and captures so far (any pointer may be
+ * null). */
 axs_status axs_soft_batch_info(const axs_soft_batch* b, int* ncase, int* queued_sweeps,
                                int64_t* graph_launches, int64_t* captures);
 axs_status axs_soft_batch_destroy(axs_soft_batch* b);

@@ -30,34 +30,110 @@ __device__ __forceinline__ short lsq_start_code(short positional_sum, short tota
   return short(short(2 * code - short(6)) / short(2));
 }
 
-// least_squares.hpp:10-59 for 3 coefficients and 2 right-hand sides.
-__device__ void lsq_gauss_3x2(double A[3][5], double sol[2][3]) {
-  for (int i = 0; i < 3; i++) {
-    int max_row = i;
-    double max_element = fabs(A[i][i]);
-    for (int k = i + 1; k < 3; k++) {
-      if (fabs(A[k][i]) > max_element) {
-        max_element = fabs(A[k][i]);
-        max_row = k;
-      }
-    }
-    for (int k = i; k < 5; k++) {
-      double tmp = A[max_row][k];
-      A[max_row][k] = A[i][k];
-      A[i][k] = tmp;
-    }
-    for (int k = i + 1; k < 3; k++) {
-      double c = -A[k][i] / A[i][i];
-      A[k][i] = 0.0;
-      for (int j = i + 1; j < 5; j++) A[k][j] += c * A[i][j];
-    }
+template <typename V>
+__device__ __forceinline__ void lsq_swap(bool take, V& a, V& b) {
+  const V t = a;
+  a = take ? b : a;
+  b = take ? t : b;
+}
+
+// least_squares.hpp:10-59 for 3 coefficients and 2 right-hand sides, split
+// into what depends on the known cells alone (the elimination of the normal
+// matrix with its pivots) and what depends on the values (the right-hand
+// sides); the two parts together run the reference's operations in its
+// order.  Rows are exchanged by selects: a row index known only at run time
+// would send the matrix to scratch memory.
+struct LsqFactor {
+  // multipliers of rows 1 and 2 (after the first exchange) and of row 2
+  // (after the second), then the upper triangle
+  double c1, c2, c3, u00, u01, u02, u11, u12, u22;
+  int m0;  // row exchanged with row 0
+  int m1;  // rows 1 and 2 exchanged (0 or 1)
+};
+
+__device__ __forceinline__ LsqFactor lsq_factor_3x3(double a00, double a01, double a02,
+                                                    double a10, double a11, double a12,
+                                                    double a20, double a21, double a22) {
+  LsqFactor f;
+  f.m0 = 0;
+  double best = fabs(a00);
+  if (fabs(a10) > best) {
+    best = fabs(a10);
+    f.m0 = 1;
   }
-  for (int comp = 0; comp < 2; ++comp) {
-    for (int i = 2; i >= 0; --i) {
-      sol[comp][i] = A[i][3 + comp] / A[i][i];
-      for (int k = i - 1; k >= 0; --k) A[k][3 + comp] -= A[k][i] * sol[comp][i];
-    }
+  if (fabs(a20) > best) f.m0 = 2;
+  lsq_swap(f.m0 == 1, a00, a10);
+  lsq_swap(f.m0 == 1, a01, a11);
+  lsq_swap(f.m0 == 1, a02, a12);
+  lsq_swap(f.m0 == 2, a00, a20);
+  lsq_swap(f.m0 == 2, a01, a21);
+  lsq_swap(f.m0 == 2, a02, a22);
+  f.c1 = -a10 / a00;
+  a11 += f.c1 * a01;
+  a12 += f.c1 * a02;
+  f.c2 = -a20 / a00;
+  a21 += f.c2 * a01;
+  a22 += f.c2 * a02;
+  f.m1 = fabs(a21) > fabs(a11) ? 1 : 0;
+  lsq_swap(f.m1 == 1, a11, a21);
+  lsq_swap(f.m1 == 1, a12, a22);
+  f.c3 = -a21 / a11;
+  a22 += f.c3 * a12;
+  f.u00 = a00;
+  f.u01 = a01;
+  f.u02 = a02;
+  f.u11 = a11;
+  f.u12 = a12;
+  f.u22 = a22;
+  return f;
+}
+
+// The fit's value at (px, py) for one right-hand side (b0, b1, b2).
+__device__ __forceinline__ double lsq_eval(const LsqFactor& f, double b0, double b1, double b2,
+                                           double px, double py) {
+  lsq_swap(f.m0 == 1, b0, b1);
+  lsq_swap(f.m0 == 2, b0, b2);
+  b1 += f.c1 * b0;
+  b2 += f.c2 * b0;
+  lsq_swap(f.m1 == 1, b1, b2);
+  b2 += f.c3 * b1;
+  const double s2 = b2 / f.u22;
+  b1 -= f.u12 * s2;
+  b0 -= f.u02 * s2;
+  const double s1 = b1 / f.u11;
+  b0 -= f.u01 * s1;
+  const double s0 = b0 / f.u00;
+  double e = 0.0;
+  e += s0 * 1.0;
+  e += s1 * (1.0 * px);
+  e += s2 * (1.0 * py);
+  return e;
+}
+
+// Normal matrix of the window at (s_y, s_x) from its cells' flags m (row
+// major, 0 or 1), factored.
+__device__ __forceinline__ LsqFactor lsq_window_factor(const double m[9],
+                                                       const double* __restrict__ gx,
+                                                       const double* __restrict__ gy, int n0,
+                                                       int n1, int s_y, int s_x) {
+  double L1[9], L2[9];
+#pragma unroll
+  for (int n = 0; n < 9; ++n) {
+    const int jl = s_y + n / 3, il = s_x + n % 3;
+    L1[n] = m[n] * ((il >= 0 && il < n1) ? gx[il] : 0.0);
+    L2[n] = m[n] * ((jl >= 0 && jl < n0) ? gy[jl] : 0.0);
   }
+  double b00 = 0.0, b01 = 0.0, b02 = 0.0, b11 = 0.0, b12 = 0.0, b22 = 0.0;
+#pragma unroll
+  for (int q = 0; q < 9; ++q) {
+    b00 += m[q] * m[q];
+    b01 += m[q] * L1[q];
+    b02 += m[q] * L2[q];
+    b11 += L1[q] * L1[q];
+    b12 += L1[q] * L2[q];
+    b22 += L2[q] * L2[q];
+  }
+  return lsq_factor_3x3(b00, b01, b02, b01, b11, b12, b02, b12, b22);
 }
 
 // Fit of cell (j, i) from the known cells around it
@@ -70,7 +146,9 @@ __device__ __forceinline__ bool lsq_fit_cell(const int16_t* __restrict__ cur,
                                              const double* __restrict__ gy, int n0, int n1,
                                              int j, int i, double& vx, double& vy) {
   short local_sum = 0, lx = 0, ly = 0;
+#pragma unroll
   for (int jl = -1; jl <= 1; ++jl)
+#pragma unroll
     for (int il = -1; il <= 1; ++il) {
       const short f = lsq_flag(cur, n0, n1, j + jl, i + il);
       local_sum += (jl == 0 && il == 0) ? short(0) : f;
@@ -80,54 +158,38 @@ __device__ __forceinline__ bool lsq_fit_cell(const int16_t* __restrict__ cur,
   if (!local_sum) return false;
   const int s_x = i + lsq_start_code(lx, local_sum);
   const int s_y = j + lsq_start_code(ly, local_sum);
-  double L0[9], L1[9], L2[9], r0[9], r1[9];
-  int n = 0;
-  for (int jl = s_y; jl < s_y + 3; ++jl) {
-    for (int il = s_x; il < s_x + 3; ++il, ++n) {
-      const bool in = (jl >= 0 && jl < n0 && il >= 0 && il < n1);
-      const double m = in ? double(cur[(int64_t)jl * n1 + il]) : 0.0;
-      const double xv = in ? gx[il] : 0.0;
-      const double yv = in ? gy[jl] : 0.0;
-      L0[n] = m;
-      L1[n] = m * xv;
-      L2[n] = m * yv;
-      const int64_t g = (int64_t)jl * n1 + il;
-      r0[n] = m * (in ? ex[g] : 0.0);
-      r1[n] = m * (in ? ey[g] : 0.0);
-    }
+  double m[9], r0[9], r1[9];
+#pragma unroll
+  for (int n = 0; n < 9; ++n) {
+    const int jl = s_y + n / 3, il = s_x + n % 3;
+    const bool in = (jl >= 0 && jl < n0 && il >= 0 && il < n1);
+    const int64_t g = (int64_t)jl * n1 + il;
+    m[n] = in ? double(cur[g]) : 0.0;
+    r0[n] = m[n] * (in ? ex[g] : 0.0);
+    r1[n] = m[n] * (in ? ey[g] : 0.0);
   }
-  const double* Ls[3] = {L0, L1, L2};
-  double B[3][5];
-  for (int a = 0; a < 3; ++a)
-    for (int b = 0; b < 3; ++b) {
-      double s = 0.0;
-      for (int q = 0; q < 9; ++q) s += Ls[a][q] * Ls[b][q];
-      B[a][b] = s;
-    }
-  for (int a = 0; a < 3; ++a) {
-    double s = 0.0;
-    for (int q = 0; q < 9; ++q) s += Ls[a][q] * r0[q];
-    B[a][3] = s;
-    s = 0.0;
-    for (int q = 0; q < 9; ++q) s += Ls[a][q] * r1[q];
-    B[a][4] = s;
+  const LsqFactor f = lsq_window_factor(m, gx, gy, n0, n1, s_y, s_x);
+  double bx[3] = {0.0, 0.0, 0.0}, by[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int n = 0; n < 9; ++n) {
+    const int jl = s_y + n / 3, il = s_x + n % 3;
+    const double l1 = m[n] * ((il >= 0 && il < n1) ? gx[il] : 0.0);
+    const double l2 = m[n] * ((jl >= 0 && jl < n0) ? gy[jl] : 0.0);
+    bx[0] += m[n] * r0[n];
+    bx[1] += l1 * r0[n];
+    bx[2] += l2 * r0[n];
+    by[0] += m[n] * r1[n];
+    by[1] += l1 * r1[n];
+    by[2] += l2 * r1[n];
   }
-  double sol[2][3];
-  lsq_gauss_3x2(B, sol);
-  const double px = gx[i], py = gy[j];
-  const double E[3] = {1.0, 1.0 * px, 1.0 * py};
-  double e = 0.0;
-  for (int q = 0; q < 3; ++q) e += sol[0][q] * E[q];
-  vx = e;
-  e = 0.0;
-  for (int q = 0; q < 3; ++q) e += sol[1][q] * E[q];
-  vy = e;
+  vx = lsq_eval(f, bx[0], bx[1], bx[2], gx[i], gy[j]);
+  vy = lsq_eval(f, by[0], by[1], by[2], gx[i], gy[j]);
   return true;
 }
 
 // One sweep, phase 1: select + fit.  pend[c] = 1 when cell c is extrapolated
 // this sweep (new values in nx/ny), else 0.
-__global__ void lsq_fit_kernel(const int16_t* __restrict__ cur, const int16_t* __restrict__ tgt,
+__global__ void __launch_bounds__(256) lsq_fit_kernel(const int16_t* __restrict__ cur, const int16_t* __restrict__ tgt,
                                const double* __restrict__ ex, const double* __restrict__ ey,
                                const double* __restrict__ gx, const double* __restrict__ gy,
                                int n0, int n1, double* __restrict__ nx, double* __restrict__ ny,
@@ -150,36 +212,6 @@ __global__ void lsq_fit_kernel(const int16_t* __restrict__ cur, const int16_t* _
   atomicAdd(counter, 1u);
 }
 
-// The same sweep over a list of cells (the ones with current ^ target set
-// when the list was made; entries that became known are skipped by the same
-// test).  pend is indexed by list entry.
-__global__ void lsq_fit_list_kernel(const int16_t* __restrict__ cur,
-                                    const int16_t* __restrict__ tgt,
-                                    const double* __restrict__ ex, const double* __restrict__ ey,
-                                    const double* __restrict__ gx, const double* __restrict__ gy,
-                                    int n0, int n1, const int* __restrict__ list,
-                                    const unsigned* __restrict__ count, double* __restrict__ nx,
-                                    double* __restrict__ ny, int8_t* __restrict__ pend,
-                                    unsigned* __restrict__ counter,
-                                    const unsigned* __restrict__ prev_counter) {
-  if (prev_counter && *prev_counter == 0u) return;
-  const int nl = (int)*count;
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nl; k += gridDim.x * blockDim.x) {
-    const int c = list[k];
-    int8_t p = 0;
-    if (cur[c] ^ tgt[c]) {
-      double vx, vy;
-      if (lsq_fit_cell(cur, ex, ey, gx, gy, n0, n1, c / n1, c % n1, vx, vy)) {
-        nx[c] = vx;
-        ny[c] = vy;
-        p = 1;
-        atomicAdd(counter, 1u);
-      }
-    }
-    pend[k] = p;
-  }
-}
-
 // Phase 2: commit values and flags of the cells fitted in phase 1.
 __global__ void lsq_commit_kernel(int16_t* __restrict__ cur, double* __restrict__ ex,
                                   double* __restrict__ ey, const double* __restrict__ nx,
@@ -193,267 +225,23 @@ __global__ void lsq_commit_kernel(int16_t* __restrict__ cur, double* __restrict_
   cur[c] = 1;
 }
 
-__global__ void lsq_commit_list_kernel(int16_t* __restrict__ cur, double* __restrict__ ex,
-                                       double* __restrict__ ey, const double* __restrict__ nx,
-                                       const double* __restrict__ ny,
-                                       const int8_t* __restrict__ pend,
-                                       const int* __restrict__ list,
-                                       const unsigned* __restrict__ count,
-                                       const unsigned* __restrict__ counter) {
-  if (*counter == 0u) return;
-  const int nl = (int)*count;
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nl; k += gridDim.x * blockDim.x) {
-    if (!pend[k]) continue;
-    const int c = list[k];
-    ex[c] = nx[c];
-    ey[c] = ny[c];
-    cur[c] = 1;
-  }
-}
-
-// Cells with current ^ target set, in any order (the set is what matters:
-// a sweep's fits read only the previous sweep's state); *count must be zero.
-__global__ void lsq_list_kernel(const int16_t* __restrict__ cur, const int16_t* __restrict__ tgt,
-                                int64_t n, int* __restrict__ list, unsigned* __restrict__ count) {
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  list_append(c < n && (cur[c] ^ tgt[c]), (int)c, list, count);
-}
-
-__global__ void lsq_sweep_pingpong_kernel(
-    const int16_t* __restrict__ cur_in, const double* __restrict__ ex_in,
-    const double* __restrict__ ey_in, int16_t* __restrict__ cur_out, double* __restrict__ ex_out,
-    double* __restrict__ ey_out, const int16_t* __restrict__ tgt, const double* __restrict__ gx,
-    const double* __restrict__ gy, int n0, int n1, const int* __restrict__ list,
-    const unsigned* __restrict__ count, unsigned* __restrict__ counter,
-    const unsigned* __restrict__ prev_counter) {
-  if (prev_counter && *prev_counter == 0u) return;  // the reference loop has ended
-  const int nl = (int)*count;
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nl; k += gridDim.x * blockDim.x) {
-    const int c = list[k];
-    double vx, vy;
-    if ((cur_in[c] ^ tgt[c]) &&
-        lsq_fit_cell(cur_in, ex_in, ey_in, gx, gy, n0, n1, c / n1, c % n1, vx, vy)) {
-      ex_out[c] = vx;
-      ey_out[c] = vy;
-      cur_out[c] = 1;
-      atomicAdd(counter, 1u);
-    } else {
-      ex_out[c] = ex_in[c];
-      ey_out[c] = ey_in[c];
-      cur_out[c] = cur_in[c];
-    }
-  }
-}
-
-__device__ void lsq_sweep_tail_body(
-    int16_t* __restrict__ cur_a, double* __restrict__ ex_a, double* __restrict__ ey_a,
-    int16_t* __restrict__ cur_b, double* __restrict__ ex_b, double* __restrict__ ey_b,
-    const int16_t* __restrict__ tgt, const double* __restrict__ gx, const double* __restrict__ gy,
-    int n0, int n1, const int* __restrict__ list, const unsigned* __restrict__ count,
-    unsigned* __restrict__ counters, int sweeps, int* __restrict__ tail, int cap) {
-  // unknown cells (u) and cells fitted by the previous sweep (f), read from
-  // index `par` and written to index par ^ 1 of each
-  int* ul[2] = {tail, tail + cap};
-  int* fl[2] = {tail + 2 * (int64_t)cap, tail + 3 * (int64_t)cap};
-  __shared__ unsigned nu[2], nf[2];
-  if (counters[sweeps - 1] == 0u) {  // the loop ended within the queued sweeps
-    if (threadIdx.x == 0) counters[sweeps] = 0u;
-    return;
-  }
-  // sweep sweeps-1 wrote the second set when sweeps-1 is even: the result
-  // must end there
-  const bool home_b = ((sweeps - 1) & 1) == 0;
-  int16_t* ci = home_b ? cur_b : cur_a;
-  double* xi = home_b ? ex_b : ex_a;
-  double* yi = home_b ? ey_b : ey_a;
-  int16_t* co = home_b ? cur_a : cur_b;
-  double* xo = home_b ? ex_a : ex_b;
-  double* yo = home_b ? ey_a : ey_b;
-  const int nl = (int)*count;
-  unsigned ran = 0;
-  for (;;) {
-    const int par = ran & 1, nxt = par ^ 1;
-    if (threadIdx.x == 0) {
-      nu[nxt] = 0u;
-      nf[nxt] = 0u;
-    }
-    __syncthreads();
-    if (ran == 0) {
-      // the whole list: fit, or copy through (the two sets differ on the
-      // cells the last queued sweep fitted)
-      for (int k = threadIdx.x; k < nl; k += blockDim.x) {
-        const int c = list[k];
-        double vx, vy;
-        const bool unknown = ci[c] ^ tgt[c];
-        if (unknown && lsq_fit_cell(ci, xi, yi, gx, gy, n0, n1, c / n1, c % n1, vx, vy)) {
-          xo[c] = vx;
-          yo[c] = vy;
-          co[c] = 1;
-          fl[nxt][atomicAdd(&nf[nxt], 1u)] = c;
-        } else {
-          xo[c] = xi[c];
-          yo[c] = yi[c];
-          co[c] = ci[c];
-          if (unknown) ul[nxt][atomicAdd(&nu[nxt], 1u)] = c;
-        }
-      }
-    } else {
-      // cells fitted by the previous sweep: into this sweep's output set
-      const int nfp = (int)nf[par];
-      for (int k = threadIdx.x; k < nfp; k += blockDim.x) {
-        const int c = fl[par][k];
-        xo[c] = xi[c];
-        yo[c] = yi[c];
-        co[c] = ci[c];
-      }
-      // cells still unknown (equal, flag 0, in both sets): fit or keep
-      const int nup = (int)nu[par];
-      for (int k = threadIdx.x; k < nup; k += blockDim.x) {
-        const int c = ul[par][k];
-        double vx, vy;
-        if (lsq_fit_cell(ci, xi, yi, gx, gy, n0, n1, c / n1, c % n1, vx, vy)) {
-          xo[c] = vx;
-          yo[c] = vy;
-          co[c] = 1;
-          fl[nxt][atomicAdd(&nf[nxt], 1u)] = c;
-        } else {
-          ul[nxt][atomicAdd(&nu[nxt], 1u)] = c;
-        }
-      }
-    }
-    __syncthreads();
-    ++ran;
-    int16_t* tc = ci;
-    ci = co;
-    co = tc;
-    double* t = xi;
-    xi = xo;
-    xo = t;
-    t = yi;
-    yi = yo;
-    yo = t;
-    // the same values for every thread; with current flags inside target
-    // ones every sweep but the last fills a listed cell, so the second
-    // test only bounds the loop for flags that break that rule
-    if (nf[nxt] == 0u || ran > (unsigned)nl) break;
-  }
-  // the last sweep fitted nothing and copied the previous sweep's fits
-  // across: both sets now hold every fit, the home set included
-  if (threadIdx.x == 0) counters[sweeps] = ran;
-}
-
-__global__ void __launch_bounds__(512) lsq_sweep_tail_kernel(
-    int16_t* __restrict__ cur_a, double* __restrict__ ex_a, double* __restrict__ ey_a,
-    int16_t* __restrict__ cur_b, double* __restrict__ ex_b, double* __restrict__ ey_b,
-    const int16_t* __restrict__ tgt, const double* __restrict__ gx, const double* __restrict__ gy,
-    int n0, int n1, const int* __restrict__ list, const unsigned* __restrict__ count,
-    unsigned* __restrict__ counters, int sweeps, int* __restrict__ tail, int cap) {
-  lsq_sweep_tail_body(cur_a, ex_a, ey_a, cur_b, ex_b, ey_b, tgt, gx, gy, n0, n1, list, count,
-                      counters, sweeps, tail, cap);
-}
-
-// ------------------------------------------------------------ soft batches
-// The doubled (2 nr, nz) grid of every case, z serving as both axes'
-// coordinates as in the single-case step; each case has its own list,
-// counters and tail lists.
-
-template <typename B>
-__global__ void soft_batch_lsq_list_kernel(const SoftCaseT<B>* __restrict__ cs,
-                                           const uint32_t* __restrict__ blocks) {
-  const SoftBlock b = soft_block(blocks);  // a row of the doubled grid
-  const SoftCaseT<B>& C = cs[b.c];
-  // the doubled row's physical row (both halves mirror it); outside the
-  // step's zone every flag is 0 (the whole workgroup leaves together)
-  if (!zone_row(C, b.i >= C.nr ? b.i - C.nr : C.nr - 1 - b.i)) return;
-  const int j = b.j;
-  const int64_t c = (int64_t)b.i * C.nz + j;
-  list_append(j < C.nz && (C.cur[c] ^ C.tgt[c]), (int)c, C.lw.list, C.lw.count);
-}
-
-// Ping-pong sweep q over each case's list (blockIdx.y = case): sweep q reads
-// the first set (cur, e1d, e2d) when q is even.
-template <typename B>
-__global__ void soft_batch_lsq_sweep_kernel(const SoftCaseT<B>* __restrict__ cs, int q) {
-  const SoftCaseT<B>& C = cs[blockIdx.y];
-  const LsqWork& w = C.lw;
-  if (q > 0 && w.counters[q - 1] == 0u) return;  // the reference loop has ended
-  const bool odd = q & 1;
-  const int16_t* cur_in = odd ? w.cur2 : C.cur;
-  const double* ex_in = odd ? w.ex2 : C.e1d;
-  const double* ey_in = odd ? w.ey2 : C.e2d;
-  int16_t* cur_out = odd ? C.cur : w.cur2;
-  double* ex_out = odd ? C.e1d : w.ex2;
-  double* ey_out = odd ? C.e2d : w.ey2;
-  const int n0 = 2 * C.nr, n1 = C.nz;
-  const int nl = (int)*w.count;
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nl; k += gridDim.x * blockDim.x) {
-    const int c = w.list[k];
-    double vx, vy;
-    if ((cur_in[c] ^ C.tgt[c]) &&
-        lsq_fit_cell(cur_in, ex_in, ey_in, C.z, C.z, n0, n1, c / n1, c % n1, vx, vy)) {
-      ex_out[c] = vx;
-      ey_out[c] = vy;
-      cur_out[c] = 1;
-      atomicAdd(w.counters + q, 1u);
-    } else {
-      ex_out[c] = ex_in[c];
-      ey_out[c] = ey_in[c];
-      cur_out[c] = cur_in[c];
-    }
-  }
-}
-
-template <typename B>
-__global__ void __launch_bounds__(512) soft_batch_lsq_tail_kernel(
-    const SoftCaseT<B>* __restrict__ cs, int sweeps) {
-  const SoftCaseT<B>& C = cs[blockIdx.x];
-  const LsqWork& w = C.lw;
-  lsq_sweep_tail_body(C.cur, C.e1d, C.e2d, w.cur2, w.ex2, w.ey2, C.tgt, C.z, C.z, 2 * C.nr, C.nz,
-                      w.list, w.count, w.counters, sweeps, w.tail, w.cap);
-}
-
-template <typename B>
-hipError_t launch_soft_batch_lsq_list(const SoftCaseT<B>* cases, const SoftBatchDims& d,
-                                      hipStream_t s) {
-  soft_batch_lsq_list_kernel<B><<<d.ndbl_blocks, 256, 0, s>>>(cases, d.dbl_blocks);
-  return hipGetLastError();
-}
-
-template <typename B>
-hipError_t launch_soft_batch_lsq_sweep(const SoftCaseT<B>* cases, const SoftBatchDims& d, int sweep,
-                                       hipStream_t s) {
-  constexpr int kBlocksPerCase = 64;  // a case's band: up to ~16k cells, one per thread
-  soft_batch_lsq_sweep_kernel<B><<<dim3(kBlocksPerCase, d.ncase), 256, 0, s>>>(cases, sweep);
-  return hipGetLastError();
-}
-
-template <typename B>
-hipError_t launch_soft_batch_lsq_tail(const SoftCaseT<B>* cases, const SoftBatchDims& d, int sweeps,
-                                      hipStream_t s) {
-  soft_batch_lsq_tail_kernel<B><<<d.ncase, 512, 0, s>>>(cases, sweeps);
-  return hipGetLastError();
-}
-
-template hipError_t launch_soft_batch_lsq_list<double>(const SoftCaseT<double>*,
-                                                       const SoftBatchDims&, hipStream_t);
-template hipError_t launch_soft_batch_lsq_list<float>(const SoftCaseT<float>*,
-                                                      const SoftBatchDims&, hipStream_t);
-template hipError_t launch_soft_batch_lsq_sweep<double>(const SoftCaseT<double>*,
-                                                        const SoftBatchDims&, int, hipStream_t);
-template hipError_t launch_soft_batch_lsq_sweep<float>(const SoftCaseT<float>*,
-                                                       const SoftBatchDims&, int, hipStream_t);
-template hipError_t launch_soft_batch_lsq_tail<double>(const SoftCaseT<double>*,
-                                                       const SoftBatchDims&, int, hipStream_t);
-template hipError_t launch_soft_batch_lsq_tail<float>(const SoftCaseT<float>*,
-                                                      const SoftBatchDims&, int, hipStream_t);
-
 __global__ void fill_u32_kernel(unsigned* p, int n, unsigned v) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k < n) p[k] = v;
 }
 
-hipError_t launch_lsq_sweep(int16_t* cur, const int16_t* tgt, double* ex, double* ey,
-                            const double* gx, const double* gy, int n0, int n1, LsqWork w,
+// Scratch of the drop-in entry point's sweeps.
+struct LsqSweepWork {
+  double* nx;          // fitted eta_x of this sweep, (n0, n1)
+  double* ny;          // fitted eta_y of this sweep, (n0, n1)
+  int8_t* pend;        // 1 where a cell was fitted this sweep
+  unsigned* counters;  // cells fitted per sweep (one slot per sweep)
+};
+
+// One sweep (fit + commit).  Sweep `sweep` exits at once when
+// counters[sweep - 1] is zero, so many sweeps can be queued without a sync.
+static hipError_t launch_lsq_sweep(int16_t* cur, const int16_t* tgt, double* ex, double* ey,
+                            const double* gx, const double* gy, int n0, int n1, const LsqSweepWork& w,
                             int sweep, hipStream_t s) {
   dim3 grid(ceil_div(n1, 256), n0);
   lsq_fit_kernel<<<grid, 256, 0, s>>>(cur, tgt, ex, ey, gx, gy, n0, n1, w.nx, w.ny, w.pend,
@@ -467,50 +255,469 @@ hipError_t launch_lsq_sweep(int16_t* cur, const int16_t* tgt, double* ex, double
   return hipGetLastError();
 }
 
-hipError_t launch_lsq_list(const int16_t* cur, const int16_t* tgt, int64_t n, LsqWork w,
-                           hipStream_t s) {
-  lsq_list_kernel<<<ceil_div(n, 256), 256, 0, s>>>(cur, tgt, n, w.list, w.count);
-  return hipGetLastError();
-}
-
-hipError_t launch_lsq_sweep_list(int16_t* cur, const int16_t* tgt, double* ex, double* ey,
-                                 const double* gx, const double* gy, int n0, int n1, LsqWork w,
-                                 int sweep, hipStream_t s) {
-  constexpr int kBlocks = 128;  // the band's cells, strided (a few thousand here)
-  lsq_fit_list_kernel<<<kBlocks, 256, 0, s>>>(cur, tgt, ex, ey, gx, gy, n0, n1, w.list, w.count,
-                                              w.nx, w.ny, w.pend, w.counters + sweep,
-                                              sweep > 0 ? w.counters + sweep - 1 : nullptr);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  lsq_commit_list_kernel<<<kBlocks, 256, 0, s>>>(cur, ex, ey, w.nx, w.ny, w.pend, w.list, w.count,
-                                                 w.counters + sweep);
-  return hipGetLastError();
-}
-
-hipError_t launch_lsq_sweep_pingpong(const int16_t* cur_in, const double* ex_in,
-                                     const double* ey_in, int16_t* cur_out, double* ex_out,
-                                     double* ey_out, const int16_t* tgt, const double* gx,
-                                     const double* gy, int n0, int n1, LsqWork w, int sweep,
-                                     hipStream_t s) {
-  constexpr int kBlocks = 128;
-  lsq_sweep_pingpong_kernel<<<kBlocks, 256, 0, s>>>(
-      cur_in, ex_in, ey_in, cur_out, ex_out, ey_out, tgt, gx, gy, n0, n1, w.list, w.count,
-      w.counters + sweep, sweep > 0 ? w.counters + sweep - 1 : nullptr);
-  return hipGetLastError();
-}
-
-hipError_t launch_lsq_sweep_tail(int16_t* cur, double* ex, double* ey, const int16_t* tgt,
-                                 const double* gx, const double* gy, int n0, int n1, LsqWork w,
-                                 int sweeps, hipStream_t s) {
-  lsq_sweep_tail_kernel<<<1, 512, 0, s>>>(cur, ex, ey, w.cur2, w.ex2, w.ey2, tgt, gx, gy, n0, n1,
-                                           w.list, w.count, w.counters, sweeps, w.tail, w.cap);
-  return hipGetLastError();
-}
-
-hipError_t launch_fill_u32(unsigned* p, int n, unsigned v, hipStream_t s) {
+static hipError_t launch_fill_u32(unsigned* p, int n, unsigned v, hipStream_t s) {
   fill_u32_kernel<<<ceil_div(n, 256), 256, 0, s>>>(p, n, v);
   return hipGetLastError();
 }
+
+// -------------------------------------------------- soft steps: by fronts
+//
+// In the soft steps every known cell is a target (known: phi > 0, target:
+// phi > -extrap_zone), so a sweep of the reference fits exactly the unknown
+// target cells next to a cell known before it: the sweep that fits a cell
+// is its 8-neighbour distance from the known set within the target set,
+// whatever the values are.  The loop then splits into three launches:
+//   levels  one workgroup per case walks the fronts on bit rows in LDS and
+//           lists the cells front by front;
+//   factor  one thread per listed cell: its window, the cells of it known
+//           before its front, and the factored normal matrix, none of which
+//           depends on the values;
+//   solve   one workgroup per case and component takes the fronts in order
+//           (a block barrier between them): window values in, right-hand
+//           side, back substitution, value out.
+// One launch per sweep was bound by a fit's latency (flags, window, a 3 x 3
+// elimination with nine divisions, its pivoted rows in scratch memory): 17
+// us a sweep for twelve cases of 130 to 490 rows, paid for every queued
+// sweep.  Now a front pays only the value-dependent part: on those cases 125
+// us a step (levels 46, factor 19, solve 61) instead of 273, and 52 instead
+// of 163 for one 256 x 128 case (19, 10, 24).  The solve pass is bound by the
+// rate of its gathers (nine window values per cell, each lane another line:
+// about a line per cycle from the CU's L1), so the two components run on two
+// CUs; the levels pass by the list stores and barriers of each front.
+// Every fit runs the same operations in the same order as lsq_fit_cell on
+// the flags and values its sweep saw, so the results are the same bits.
+
+// The fronts' known-cell bit rows in LDS: words of 32 cells, at most
+// kLsqOwn per thread.
+constexpr int kLsqThreads = 1024, kLsqOwn = 7;
+constexpr int kLsqLdsWords = kLsqThreads * kLsqOwn;  // 28 KiB
+
+// 8-neighbour dilation at word (row, c) of `known` (rows x wc words).
+__device__ __forceinline__ unsigned lsq_dilate(const unsigned* known, int row, int c, int rows,
+                                               int wc) {
+  unsigned d = 0u;
+#pragma unroll
+  for (int rr = -1; rr <= 1; ++rr) {
+    const int r = row + rr;
+    if (r < 0 || r >= rows) continue;
+    const unsigned* k = known + (r * wc + c);
+    const unsigned m = k[0];
+    d |= m | (m << 1) | (m >> 1);
+    if (c > 0) d |= k[-1] >> 31;
+    if (c + 1 < wc) d |= k[1] << 31;
+  }
+  return d;
+}
+
+// Lists the cells of `bits`, whose lowest is cell `base`, as front `level`.
+__device__ __forceinline__ void lsq_emit(const LsqWork& w, unsigned bits, unsigned base, int level,
+                                         unsigned* s_n) {
+  // the counter's address made to look divergent: on a uniform address the
+  // compiler adds the lanes up one by one in a loop before its one atomic
+  int zero;
+  asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+  unsigned pos = atomicAdd(s_n + zero, (unsigned)__popc(bits));
+  while (bits) {
+    const unsigned cell = base + (unsigned)__ffs((int)bits) - 1u;
+    bits &= bits - 1u;
+    w.list[pos++] = LsqEntry{(int)cell, level};
+    w.lev[cell] = level;
+  }
+}
+
+// Block barrier that orders LDS accesses alone: the global stores of a
+// front's list entries stay in flight (nothing in the walk reads them), where
+// __syncthreads would wait for each front's to land.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// The fronts of one case, by one workgroup of kLsqThreads.  zone[1]: the
+// last physical row with a target cell (-1: none); the doubled rows with
+// target cells are nr - 1 - zone[1] .. nr + zone[1].
+__device__ __forceinline__ void lsq_levels_body(const LsqWork& w, int nr, int nz,
+                                                const int* __restrict__ zone) {
+  __shared__ unsigned sk[kLsqLdsWords];
+  __shared__ int s_w0, s_w1;
+  __shared__ unsigned s_n;
+  const int tid = threadIdx.x;
+  const int z1 = zone[1];
+  const int W = (nz + 31) / 32, r0 = nr - 1 - z1, rows = 2 * (z1 + 1);
+  if (tid == 0) {
+    s_w0 = W;
+    s_w1 = -1;
+    s_n = 0u;
+  }
+  __syncthreads();
+  // word columns with target cells
+  int lo = W, hi = -1;
+  for (int q = tid; q < rows * W; q += kLsqThreads) {
+    const int r = (int)((unsigned)q / (unsigned)W), c = q - r * W;
+    if (w.tb[(int64_t)(r0 + r) * w.wstride + c]) {
+      lo = min(lo, c);
+      hi = max(hi, c);
+    }
+  }
+  if (hi >= 0) {
+    atomicMin(&s_w0, lo);
+    atomicMax(&s_w1, hi);
+  }
+  __syncthreads();
+  const int w0 = s_w0, wc = max(0, s_w1 - s_w0 + 1), nw = rows * wc;
+  unsigned n = 0u;
+  int level = 0;
+  // A front's cells join the known ones only after every thread has read
+  // the known words (first barrier), and are read by the next front after
+  // all have joined (second barrier); s_n moves between the second and the
+  // first alone, so every thread reads the same count and leaves together.
+  if (nw <= kLsqLdsWords) {
+    const int own = (nw + kLsqThreads - 1) / kLsqThreads;  // uniform
+    unsigned todo[kLsqOwn], f[kLsqOwn];
+    int rc[kLsqOwn];  // row << 16 | column (rows <= 8192)
+#pragma unroll
+    for (int u = 0; u < kLsqOwn; ++u) {
+      todo[u] = 0u;
+      rc[u] = 0;
+      const int q = tid + u * kLsqThreads;
+      if (u < own && q < nw) {
+        const int r = (int)((unsigned)q / (unsigned)wc), c = q - r * wc;
+        const int64_t g = (int64_t)(r0 + r) * w.wstride + w0 + c;
+        const unsigned k = w.kb[g];
+        rc[u] = r << 16 | c;
+        sk[q] = k;
+        todo[u] = w.tb[g] & ~k;
+      }
+    }
+    lds_barrier();
+    for (;;) {
+#pragma unroll
+      for (int u = 0; u < kLsqOwn; ++u) {
+        f[u] = 0u;
+        if (u >= own || !todo[u]) continue;
+        const int r = rc[u] >> 16, c = rc[u] & 0xffff;
+        f[u] = lsq_dilate(sk, r, c, rows, wc) & todo[u];
+        if (f[u])
+          lsq_emit(w, f[u], (unsigned)(r0 + r) * (unsigned)nz + (unsigned)(w0 + c) * 32u, level + 1,
+                   &s_n);
+      }
+      lds_barrier();
+      const unsigned now = s_n;
+      if (now == n) break;
+      n = now;
+      ++level;
+      if (tid == 0) w.off[level] = (int)n;
+#pragma unroll
+      for (int u = 0; u < kLsqOwn; ++u) {
+        if (u >= own || !f[u]) continue;
+        sk[tid + u * kLsqThreads] |= f[u];
+        todo[u] &= ~f[u];
+      }
+      lds_barrier();
+    }
+  } else {
+    // a box too large for LDS: the same walk on the case's global words
+    // (todo and f words are each read and written by one thread only)
+    for (int q = tid; q < nw; q += kLsqThreads) {
+      const int r = q / wc;
+      const int64_t g = (int64_t)(r0 + r) * w.wstride + w0 + (q - r * wc);
+      const unsigned k = w.kb[g];
+      w.kw[q] = k;
+      w.tw[q] = w.tb[g] & ~k;
+    }
+    __syncthreads();
+    for (;;) {
+      for (int q = tid; q < nw; q += kLsqThreads) {
+        const unsigned todo = w.tw[q];
+        if (!todo) continue;
+        const int r = q / wc, c = q - r * wc;
+        const unsigned f = lsq_dilate(w.kw, r, c, rows, wc) & todo;
+        w.fw[q] = f;
+        if (f)
+          lsq_emit(w, f, (unsigned)(r0 + r) * (unsigned)nz + (unsigned)(w0 + c) * 32u, level + 1,
+                   &s_n);
+      }
+      __syncthreads();
+      const unsigned now = s_n;
+      if (now == n) break;
+      n = now;
+      ++level;
+      if (tid == 0) w.off[level] = (int)n;
+      for (int q = tid; q < nw; q += kLsqThreads) {
+        const unsigned todo = w.tw[q];
+        if (!todo) continue;
+        const unsigned f = w.fw[q];
+        if (!f) continue;
+        w.kw[q] |= f;
+        w.tw[q] = todo & ~f;
+      }
+      __syncthreads();
+    }
+  }
+  if (tid == 0) {
+    w.off[0] = 0;
+    w.head[0] = n;
+    w.head[1] = (unsigned)level;
+  }
+}
+
+// A listed cell's window: flags (bit n: window cell n, row major, known
+// before the cell's front), origin relative to the cell, and whether an
+// unknown window cell holds a non-finite value (the reference multiplies
+// it by its zero flag, which makes the fit NaN).
+struct LsqWindow {
+  unsigned mask;
+  int dy, dx;  // [-3, 1]
+  bool nan_x, nan_y;
+};
+__device__ __forceinline__ unsigned lsq_pack(const LsqWindow& v, int m0, int m1) {
+  return v.mask | (unsigned)(v.dy + 3) << 9 | (unsigned)(v.dx + 3) << 12 | (v.nan_x ? 1u : 0u) << 15 |
+         (v.nan_y ? 1u : 0u) << 16 | (unsigned)m0 << 17 | (unsigned)m1 << 19;
+}
+__device__ __forceinline__ LsqWindow lsq_unpack(unsigned p, int& m0, int& m1) {
+  m0 = (int)(p >> 17) & 3;
+  m1 = (int)(p >> 19) & 1;
+  return LsqWindow{p & 511u, (int)(p >> 9 & 7u) - 3, (int)(p >> 12 & 7u) - 3, (p >> 15 & 1u) != 0u,
+                   (p >> 16 & 1u) != 0u};
+}
+
+// Window and factor of cell c = (j, i) of front `level` (a cell is known
+// before it when its level is lower).
+__device__ __forceinline__ LsqWindow lsq_window_of(const LsqWork& w, const double* __restrict__ ex,
+                                                   const double* __restrict__ ey,
+                                                   const double* __restrict__ g, int n0, int n1,
+                                                   int j, int i, int level, LsqFactor& f) {
+  short local_sum = 0, lx = 0, ly = 0;
+#pragma unroll
+  for (int jl = -1; jl <= 1; ++jl)
+#pragma unroll
+    for (int il = -1; il <= 1; ++il) {
+      const int jj = j + jl, ii = i + il;
+      const bool in = jj >= 0 && jj < n0 && ii >= 0 && ii < n1;
+      const short k = (in && w.lev[(int64_t)jj * n1 + ii] < level) ? short(1) : short(0);
+      local_sum += k;  // the cell itself is unknown
+      lx += k * short(il + 1);
+      ly += k * short(jl + 1);
+    }
+  LsqWindow v{0u, lsq_start_code(ly, local_sum), lsq_start_code(lx, local_sum), false, false};
+  double m[9];
+#pragma unroll
+  for (int n = 0; n < 9; ++n) {
+    const int jl = j + v.dy + n / 3, il = i + v.dx + n % 3;
+    const bool in = (jl >= 0 && jl < n0 && il >= 0 && il < n1);
+    const int64_t c = (int64_t)jl * n1 + il;
+    const bool known = in && w.lev[c] < level;
+    m[n] = known ? 1.0 : 0.0;
+    if (known) {
+      v.mask |= 1u << n;
+    } else if (in) {
+      v.nan_x = v.nan_x || !isfinite(ex[c]);
+      v.nan_y = v.nan_y || !isfinite(ey[c]);
+    }
+  }
+  f = lsq_window_factor(m, g, g, n0, n1, j + v.dy, i + v.dx);
+  return v;
+}
+
+// Windows of listed cells idx, idx + stride, ..., and the factors of the
+// first fcap (the solve pass factors the rest itself).
+__device__ __forceinline__ void lsq_factor_body(const LsqWork& w, const double* __restrict__ ex,
+                                                const double* __restrict__ ey,
+                                                const double* __restrict__ g, int n0, int n1,
+                                                int idx, int stride) {
+  const int n = (int)w.head[0];
+  const size_t cap = (size_t)w.fcap;
+  for (int k = idx; k < n; k += stride) {
+    const LsqEntry t = w.list[k];
+    const int j = t.cell / n1, i = t.cell - j * n1;
+    LsqFactor f;
+    const LsqWindow v = lsq_window_of(w, ex, ey, g, n0, n1, j, i, t.level, f);
+    w.win[k] = lsq_pack(v, f.m0, f.m1);
+    if (k >= w.fcap) continue;
+    w.fac[k] = f.c1;
+    w.fac[cap + k] = f.c2;
+    w.fac[2 * cap + k] = f.c3;
+    w.fac[3 * cap + k] = f.u00;
+    w.fac[4 * cap + k] = f.u01;
+    w.fac[5 * cap + k] = f.u02;
+    w.fac[6 * cap + k] = f.u11;
+    w.fac[7 * cap + k] = f.u12;
+    w.fac[8 * cap + k] = f.u22;
+  }
+}
+
+// Value-dependent part of one component's fit of cell (j, i): right-hand
+// side from the window's known cells (an unknown one adds +-0 to a sum that
+// began at +0), back substitution, value in place.
+__device__ __forceinline__ void lsq_fit_window(const LsqWindow& v, bool nan, const LsqFactor& f,
+                                               double* e, const double* __restrict__ g, int n0,
+                                               int n1, int j, int i) {
+  const int c = j * n1 + i, o = c + v.dy * n1 + v.dx;
+  double x[9], l1[3], l2[3];
+#pragma unroll
+  for (int n = 0; n < 9; ++n)
+    x[n] = e[(v.mask >> n & 1u) ? o + (n / 3) * n1 + n % 3 : c];
+#pragma unroll
+  for (int n = 0; n < 3; ++n) {  // clamped: a window cell off the grid is unknown
+    l1[n] = g[min(max(i + v.dx + n, 0), n1 - 1)];
+    l2[n] = g[min(max(j + v.dy + n, 0), n0 - 1)];
+  }
+  const double px = g[i], py = g[j];
+  double b0 = 0.0, b1 = 0.0, b2 = 0.0;
+#pragma unroll
+  for (int n = 0; n < 9; ++n) {
+    const bool known = (v.mask >> n & 1u) != 0u;
+    b0 = known ? b0 + x[n] : b0;
+    b1 = known ? b1 + l1[n % 3] * x[n] : b1;
+    b2 = known ? b2 + l2[n / 3] * x[n] : b2;
+  }
+  if (nan) b0 = b1 = b2 = __longlong_as_double(0x7ff8000000000000LL);
+  e[c] = lsq_eval(f, b0, b1, b2, px, py);
+}
+
+// A listed cell whose factor was not kept (out of line: its registers would
+// spill those of the common path).
+__device__ __attribute__((noinline)) void lsq_fit_unfactored(const LsqWindow& v, bool nan,
+                                                             double* e, const double* g, int n0,
+                                                             int n1, int j, int i) {
+  double m[9];
+#pragma unroll
+  for (int n = 0; n < 9; ++n) m[n] = (v.mask >> n & 1u) ? 1.0 : 0.0;
+  const LsqFactor f = lsq_window_factor(m, g, g, n0, n1, j + v.dy, i + v.dx);
+  lsq_fit_window(v, nan, f, e, g, n0, n1, j, i);
+}
+
+// A listed cell's window and factor as the factor pass left them (the
+// factor of the last kept one when the cell's own was not).
+struct LsqRecord {
+  int cell;
+  unsigned win;
+  LsqFactor f;
+};
+__device__ __forceinline__ LsqRecord lsq_record(const LsqWork& w, int k) {
+  const size_t cap = (size_t)w.fcap, q = (size_t)min(k, w.fcap - 1);
+  LsqRecord r;
+  r.cell = w.list[k].cell;
+  r.win = w.win[k];
+  r.f.c1 = w.fac[q];
+  r.f.c2 = w.fac[cap + q];
+  r.f.c3 = w.fac[2 * cap + q];
+  r.f.u00 = w.fac[3 * cap + q];
+  r.f.u01 = w.fac[4 * cap + q];
+  r.f.u02 = w.fac[5 * cap + q];
+  r.f.u11 = w.fac[6 * cap + q];
+  r.f.u12 = w.fac[7 * cap + q];
+  r.f.u22 = w.fac[8 * cap + q];
+  return r;
+}
+
+// One component's fits of one case (e: its values; second: the second
+// component), front by front, in place: a fit reads only cells known before
+// its front (the value it loads for another window cell is its own cell's,
+// and is not used) and writes its own cell.  A thread's first record of the
+// next front is loaded before this front's barrier, so that the front after
+// starts with its window's values.
+__device__ __forceinline__ void lsq_solve_body(const LsqWork& w, double* e, bool second,
+                                               const double* __restrict__ g, int n0, int n1) {
+  const int levels = (int)w.head[1], total = (int)w.head[0];
+  const int tid = threadIdx.x, nth = blockDim.x;
+  if (total == 0) return;
+  int begin = 0, end = w.off[1], next = levels > 1 ? w.off[2] : end;
+  LsqRecord r = lsq_record(w, min(tid, total - 1));
+  for (int level = 1; level <= levels; ++level) {
+    const LsqRecord r1 = lsq_record(w, min(end + tid, total - 1));
+    const int after = level + 2 <= levels ? w.off[level + 2] : next;
+    for (int k = begin + tid; k < end; k += nth) {
+      if (k != begin + tid) r = lsq_record(w, k);
+      const int j = r.cell / n1, i = r.cell - j * n1;
+      const LsqWindow v = lsq_unpack(r.win, r.f.m0, r.f.m1);
+      const bool nan = second ? v.nan_y : v.nan_x;
+      if (k < w.fcap)
+        lsq_fit_window(v, nan, r.f, e, g, n0, n1, j, i);
+      else
+        lsq_fit_unfactored(v, nan, e, g, n0, n1, j, i);
+    }
+    __syncthreads();
+    r = r1;
+    begin = end;
+    end = next;
+    next = after;
+  }
+}
+
+__global__ void __launch_bounds__(kLsqThreads) lsq_levels_kernel(LsqWork w, int nr, int nz,
+                                                                 const int* __restrict__ zone) {
+  lsq_levels_body(w, nr, nz, zone);
+}
+__global__ void __launch_bounds__(256) lsq_factor_kernel(LsqWork w, const double* __restrict__ ex,
+                                                         const double* __restrict__ ey,
+                                                         const double* __restrict__ g, int n0,
+                                                         int n1) {
+  lsq_factor_body(w, ex, ey, g, n0, n1, blockIdx.x * blockDim.x + threadIdx.x,
+                  gridDim.x * blockDim.x);
+}
+// 512 threads: a front has a few hundred cells, and two records in flight
+// need more than the 128 registers that 1024 threads would leave.
+constexpr int kLsqSolveThreads = 512;
+__global__ void __launch_bounds__(kLsqSolveThreads) lsq_solve_kernel(LsqWork w, double* ex,
+                                                                     double* ey,
+                                                                     const double* __restrict__ g,
+                                                                     int n0, int n1) {
+  lsq_solve_body(w, blockIdx.x ? ey : ex, blockIdx.x != 0, g, n0, n1);
+}
+
+// A band's cells, one per thread at a time (a 256-row case lists about
+// 5,000).
+constexpr int kLsqFactorBlocks = 64;
+
+hipError_t launch_lsq_fronts(const LsqWork& w, double* e1d, double* e2d, const double* z, int nr,
+                             int nz, const int* zone, hipStream_t s) {
+  lsq_levels_kernel<<<1, kLsqThreads, 0, s>>>(w, nr, nz, zone);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  lsq_factor_kernel<<<kLsqFactorBlocks, 256, 0, s>>>(w, e1d, e2d, z, 2 * nr, nz);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  lsq_solve_kernel<<<2, kLsqSolveThreads, 0, s>>>(w, e1d, e2d, z, 2 * nr, nz);
+  return hipGetLastError();
+}
+
+// Soft batches: the same passes, one workgroup (levels, solve) or
+// kLsqFactorBlocks workgroups (factor) per case.
+template <typename B>
+__global__ void __launch_bounds__(kLsqThreads) soft_batch_lsq_levels_kernel(
+    const SoftCaseT<B>* __restrict__ cs) {
+  const SoftCaseT<B>& C = cs[blockIdx.x];
+  lsq_levels_body(C.lw, C.nr, C.nz, C.zone);
+}
+template <typename B>
+__global__ void __launch_bounds__(256) soft_batch_lsq_factor_kernel(
+    const SoftCaseT<B>* __restrict__ cs) {
+  const SoftCaseT<B>& C = cs[blockIdx.y];
+  lsq_factor_body(C.lw, C.e1d, C.e2d, C.z, 2 * C.nr, C.nz, blockIdx.x * blockDim.x + threadIdx.x,
+                  gridDim.x * blockDim.x);
+}
+template <typename B>
+__global__ void __launch_bounds__(kLsqSolveThreads) soft_batch_lsq_solve_kernel(
+    const SoftCaseT<B>* __restrict__ cs) {
+  const SoftCaseT<B>& C = cs[blockIdx.y];
+  lsq_solve_body(C.lw, blockIdx.x ? C.e2d : C.e1d, blockIdx.x != 0, C.z, 2 * C.nr, C.nz);
+}
+
+template <typename B>
+hipError_t launch_soft_batch_lsq(const SoftCaseT<B>* cases, const SoftBatchDims& d,
+                                 hipStream_t s) {
+  soft_batch_lsq_levels_kernel<B><<<d.ncase, kLsqThreads, 0, s>>>(cases);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  soft_batch_lsq_factor_kernel<B><<<dim3(kLsqFactorBlocks, d.ncase), 256, 0, s>>>(cases);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  soft_batch_lsq_solve_kernel<B><<<dim3(2, d.ncase), kLsqSolveThreads, 0, s>>>(cases);
+  return hipGetLastError();
+}
+
+template hipError_t launch_soft_batch_lsq<double>(const SoftCaseT<double>*, const SoftBatchDims&,
+                                                  hipStream_t);
+template hipError_t launch_soft_batch_lsq<float>(const SoftCaseT<float>*, const SoftBatchDims&,
+                                                 hipStream_t);
 
 }  // namespace axs
 
@@ -532,7 +739,7 @@ axs_status axs_extrapolate_lsq_first_order_f64(int16_t* current_flag, const int1
   // Sweeps are issued in batches; a sweep whose predecessor found nothing
   // exits at once, so the host only reads the counters once per batch.
   constexpr int kBatch = 8;
-  LsqWork w{};
+  LsqSweepWork w{};
   AXS_HIP(hipMalloc(reinterpret_cast<void**>(&w.nx), sizeof(double) * n));
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&w.ny), sizeof(double) * n);
   if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&w.pend), n);

@@ -1,72 +1,48 @@
-// Least-squares extrapolation sweep shared by the drop-in entry point and
-// the soft-body stepper.
+// Least-squares extrapolation of the soft-body steps.
 #pragma once
 
 #include "axs_common.hpp"
 
 namespace axs {
 
-struct LsqWork {
-  double* nx;          // fitted eta_x of this sweep, (n0, n1)
-  double* ny;          // fitted eta_y of this sweep, (n0, n1)
-  int8_t* pend;        // 1 where a cell was fitted this sweep
-  unsigned* counters;  // cells fitted per sweep (one slot per sweep; the tail's count after them)
-  int* list;           // cells with current ^ target set (list form), (n0, n1) ints
-  unsigned* count;     // entries of list
-  int16_t* cur2;       // second flag and value buffers of the ping-pong sweeps
-  double* ex2;
-  double* ey2;
-  int* tail;           // the tail's four lists (unknown and just fitted, twice), list capacity each
-  int cap;             // list capacity (entries)
+struct LsqEntry {
+  int cell, level;
 };
 
-// One sweep (fit + commit).  Sweep `sweep` exits at once when
-// counters[sweep - 1] is zero, so many sweeps can be queued without a sync.
-hipError_t launch_lsq_sweep(int16_t* cur, const int16_t* tgt, double* ex, double* ey,
-                            const double* gx, const double* gy, int n0, int n1, LsqWork w,
-                            int sweep, hipStream_t s);
-// List form: launch_lsq_list collects the cells with current ^ target set
-// (*w.count must be zero; the caller clears it after the last sweep), then
-// each launch_lsq_sweep_list sweeps only those cells, with the same results
-// as launch_lsq_sweep on the whole grid.
-hipError_t launch_lsq_list(const int16_t* cur, const int16_t* tgt, int64_t n, LsqWork w,
-                           hipStream_t s);
-hipError_t launch_lsq_sweep_list(int16_t* cur, const int16_t* tgt, double* ex, double* ey,
-                                 const double* gx, const double* gy, int n0, int n1, LsqWork w,
-                                 int sweep, hipStream_t s);
-// One sweep over the listed cells in one launch: reads flags and values from
-// (cur_in, ex_in, ey_in), writes (cur_out, ex_out, ey_out) for every listed
-// cell (fitted, or copied through); cells off the list must already be equal
-// in both sets.  After the loop has ended (the previous sweep fitted
-// nothing) a sweep returns at once: the result is the set written by the
-// first sweep that fitted nothing, or by the last sweep
-// (lsq_result_is_second picks it).
-hipError_t launch_lsq_sweep_pingpong(const int16_t* cur_in, const double* ex_in,
-                                     const double* ey_in, int16_t* cur_out, double* ex_out,
-                                     double* ey_out, const int16_t* tgt, const double* gx,
-                                     const double* gy, int n0, int n1, LsqWork w, int sweep,
-                                     hipStream_t s);
-hipError_t launch_fill_u32(unsigned* p, int n, unsigned v, hipStream_t s);
-// After ping-pong sweeps 0..sweeps-1 over the first set (cur, ex, ey) and
-// the second (w.cur2, w.ex2, w.ey2): when the last of them still fitted
-// cells, one workgroup carries the reference's loop on over the listed cells
-// (block barriers between sweeps) until a sweep fits nothing, and leaves the
-// result in the set lsq_result_is_second names.  Its first sweep covers the
-// list; later ones only the cells still unknown and those fitted by the
-// sweep before (copied across, so each set ends up with every fit), kept in
-// w.tail.  w.counters[sweeps] receives the sweeps it ran (0 when the loop
-// had ended).  It ends within (list entries + 1) sweeps: every sweep but
-// the last fills a listed cell.
-hipError_t launch_lsq_sweep_tail(int16_t* cur, double* ex, double* ey, const int16_t* tgt,
-                                 const double* gx, const double* gy, int n0, int n1, LsqWork w,
-                                 int sweeps, hipStream_t s);
+// Buffers of one case's extrapolation over its doubled (2 nr, nz) grid.  The
+// pass before it (the mirror) writes every cell's flags and the values of
+// the target cells; the values are extrapolated in place.
+struct LsqWork {
+  // bit rows of wstride words, 32 cells a word: cells known before the
+  // extrapolation, and target cells (the known ones among them)
+  unsigned *kb, *tb;
+  unsigned *kw, *tw, *fw;  // fronts of a box that does not fit in LDS
+  int wstride;
+  int* lev;       // 0 known, else the front that fits the cell; kLsqNever: none has yet
+  LsqEntry* list; // cells to fit, front after front
+  int* off;       // list end of each front (off[0] = 0)
+  unsigned* head; // listed cells, fronts
+  unsigned* win;  // packed windows of the listed cells
+  double* fac;    // factors of the first fcap of them, nine arrays of fcap
+  int fcap;
+};
 
-// True when ping-pong sweeps 0..sweeps-1 (sweep q writing the second set when
-// q is even) left their result in the second buffer set.
-__device__ __forceinline__ bool lsq_result_is_second(const unsigned* counters, int sweeps) {
-  int last = 0;
-  while (last < sweeps - 1 && counters[last] != 0u) ++last;
-  return (last & 1) == 0;
-}
+constexpr int kLsqNever = 0x7fffffff;
+
+// Words per bit row: whole 256-column workgroups of the mirror pass.
+__host__ __device__ constexpr int lsq_words(int nz) { return (nz + 255) / 256 * 8; }
+// Most fronts of a doubled grid of n cells (both sizes even): a shortest
+// path between 8-neighbours holds at most two cells of a 2 x 2 block.
+__host__ __device__ constexpr int64_t lsq_max_fronts(int64_t n) { return n / 2; }
+// Factors kept per case: a sixteenth of the doubled grid's n (a band a few
+// cells wide is 2% of it at 256 rows).
+__host__ __device__ constexpr int lsq_factor_cap(int64_t n) { return int(n / 16 + 1); }
+
+// Extrapolates (e1d, e2d) of a case whose known cells are all targets: the
+// reference's loop (core/src/extrapolate_using_least_squares.hpp:142-446),
+// bit for bit, in three launches.  z: coordinates of both axes.  zone[1]:
+// the last physical row with a target cell, -1 if none.
+hipError_t launch_lsq_fronts(const LsqWork& w, double* e1d, double* e2d, const double* z, int nr,
+                             int nz, const int* zone, hipStream_t s);
 
 }  // namespace axs

@@ -16,17 +16,12 @@
 //   reinit            narrow-band signed distance, masked cells keep phi
 //                     (:159-162; axs_reinit.hip)
 //   lsq_mirror        chi = smooth Heaviside(phi) (:165-166); doubled-grid
-//                     phi, eta, flags; the sweep counters cleared
-//                     (extrapolate_eta_using_least_squares_unb.py:19-24,
+//                     eta and flags (extrapolate_eta_using_least_squares_unb.py:19-24,
 //                     extrapolate_using_least_squares.py:33-35)
-//   lsq_sweeps        least-squares extrapolation sweeps until a sweep
-//                     fits nothing, over a list of the cells to fill made
-//                     once per step; each sweep is one launch reading one
-//                     buffer set and writing the other, and returns at
-//                     once after the loop has ended; a loop longer than
-//                     the queued sweeps is finished by one workgroup
-//   lsq_back          eta = doubled eta's physical half (:29-30), from
-//                     the buffer set holding the result
+//   lsq_fronts        least-squares extrapolation, the reference's sweeps
+//                     until one fits nothing (axs_lsq.hip): the fronts of
+//                     cells, their factored fits, the fits front by front
+//   lsq_back          eta = doubled eta's physical half (:29-30)
 //   solid_sigma       stresses (solid_sigma.py:4-29), blended by chi as they
 //                     are stored (:197-199)
 //   div_tau           omega += dt curl(div sigma) (div_tau.py:4-34)
@@ -107,7 +102,11 @@ __device__ __forceinline__ void soft_dt_body(double* __restrict__ sc, double* __
 }
 
 __global__ void soft_dt_kernel(double* __restrict__ sc, double* __restrict__ slots,
-                               SoftConfig cfg) {
+                               int* __restrict__ zone, SoftConfig cfg) {
+  if (threadIdx.x == 0) {  // an empty target zone for the mirror to record
+    zone[0] = cfg.nr;
+    zone[1] = -1;
+  }
   if (cfg.streaming && threadIdx.x == 0 && sc[kSsFreqTimer] >= cfg.freq_limit)
     sc[kSsFreqTimer] = 0.0;  // :128-161 (the cycle's plot resets the timer)
   soft_dt_body(sc, slots, cfg.CFL, cfg.dx, cfg.eps, cfg.G, cfg.rho_f, cfg.nu);
@@ -191,16 +190,17 @@ __global__ void soft_pin_kernel(double* __restrict__ e1, double* __restrict__ e2
 // chi = smooth Heaviside(phi) (:165-166, written from the upper half of the
 // doubled rows), the doubled grid of
 // extrapolate_eta_using_least_squares_unb.py:19-24 and the flags of
-// extrapolate_using_least_squares.py:33-35 (lower bound 0); block (0, 0)
-// also clears the extrapolation sweeps' counters.  Returns whether the cell
-// lies in the extrapolation's target zone.
+// extrapolate_using_least_squares.py:33-35 (lower bound 0).  Sets whether
+// the cell is known and whether it lies in the extrapolation's target zone.
 template <typename O>
-__device__ __forceinline__ bool soft_lsq_mirror_at(
-    const double* __restrict__ phi, O* __restrict__ chi, double moll_zone,
-    const double* __restrict__ e1, const double* __restrict__ e2, double* __restrict__ e1d,
-    double* __restrict__ e2d, int16_t* __restrict__ cur, int16_t* __restrict__ tgt,
-    double* __restrict__ e1d2, double* __restrict__ e2d2, int16_t* __restrict__ cur2, int nr,
-    int nz, double extrap_zone, int I, int j) {
+__device__ __forceinline__ void soft_lsq_mirror_at(const double* __restrict__ phi,
+                                                   O* __restrict__ chi, double moll_zone,
+                                                   const double* __restrict__ e1,
+                                                   const double* __restrict__ e2,
+                                                   double* __restrict__ e1d,
+                                                   double* __restrict__ e2d, int* __restrict__ lev,
+                                                   int nr, int nz, double extrap_zone, int I,
+                                                   int j, bool& known, bool& target) {
   const bool upper = I >= nr;
   const int i = upper ? I - nr : nr - 1 - I;
   const int64_t c = (int64_t)i * nz + j;
@@ -210,97 +210,94 @@ __device__ __forceinline__ bool soft_lsq_mirror_at(
   const double in = (h > 0.5) ? 1.0 : 0.0;
   const double pd = -p;
   const int64_t d = (int64_t)I * nz + j;
-  const int16_t known = (pd < 0.0) ? 1 : 0;
-  const int16_t target = (pd < extrap_zone) ? 1 : 0;
-  cur[d] = known;
-  tgt[d] = target;
-  cur2[d] = known;
+  known = pd < 0.0;
+  target = pd < extrap_zone;
+  lev[d] = known ? 0 : kLsqNever;
   // Values only inside the target zone: a fit weights each value of its
   // window by the cell's known flag and sums from +0, so a cell outside the
   // zone (never known in this step) adds +-0 whatever finite value it holds
   // (the buffers start zeroed and only ever receive finite fits); the copy
   // back gives such cells in * eta (in = 0 there) itself.
-  if (!target) return false;
-  const double a = in * e1[c];
+  if (!target) return;
+  e1d[d] = in * e1[c];
   const double b = in * e2[c];
-  e1d[d] = a;
   e2d[d] = upper ? b : -b;
-  // the second buffers of the ping-pong sweeps (cells off the list never
-  // change, so both copies must hold them)
-  e1d2[d] = a;
-  e2d2[d] = upper ? b : -b;
-  return true;
 }
 
-__global__ void soft_lsq_mirror_kernel(const double* __restrict__ phi,
-                                       double* __restrict__ chi, double moll_zone,
-                                       const double* __restrict__ e1,
-                                       const double* __restrict__ e2, double* __restrict__ e1d,
-                                       double* __restrict__ e2d, int16_t* __restrict__ cur,
-                                       int16_t* __restrict__ tgt, double* __restrict__ e1d2,
-                                       double* __restrict__ e2d2, int16_t* __restrict__ cur2,
-                                       int nr, int nz, double extrap_zone,
-                                       unsigned* __restrict__ counters, int ncounters) {
-  if (blockIdx.x == 0 && blockIdx.y == 0)
-    for (int k = threadIdx.x; k < ncounters; k += blockDim.x) counters[k] = 0u;
+// The flags of a workgroup's 256-column segment of doubled row I as bits:
+// each wavefront holds two words' 64 columns.  Every thread calls it
+// (known = target = false beyond nz).
+__device__ __forceinline__ void soft_lsq_flag_bits(const LsqWork& w, int I, int j, bool known,
+                                                   bool target) {
+  const unsigned long long k = __ballot(known), t = __ballot(target);
+  const int lane = threadIdx.x & 63;
+  if ((lane & 31) == 0) {
+    const int64_t q = (int64_t)I * w.wstride + (j >> 5);
+    w.kb[q] = (unsigned)(k >> lane);
+    w.tb[q] = (unsigned)(t >> lane);
+  }
+}
+
+__global__ void __launch_bounds__(256) soft_lsq_mirror_kernel(
+    const double* __restrict__ phi, double* __restrict__ chi, double moll_zone,
+    const double* __restrict__ e1, const double* __restrict__ e2, double* __restrict__ e1d,
+    double* __restrict__ e2d, LsqWork w, int* __restrict__ zone, int nr, int nz,
+    double extrap_zone) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   const int I = blockIdx.y;  // doubled row, [0, 2 nr)
-  if (j >= nz) return;
-  soft_lsq_mirror_at(phi, chi, moll_zone, e1, e2, e1d, e2d, cur, tgt, e1d2, e2d2, cur2, nr, nz,
-                     extrap_zone, I, j);
+  bool known = false, target = false;
+  if (j < nz)
+    soft_lsq_mirror_at(phi, chi, moll_zone, e1, e2, e1d, e2d, w.lev, nr, nz, extrap_zone, I, j,
+                       known, target);
+  soft_lsq_flag_bits(w, I, j, known, target);
+  if (__syncthreads_or(target) && I >= nr && threadIdx.x == 0) {
+    atomicMin(zone, I - nr);
+    atomicMax(zone + 1, I - nr);
+  }
 }
 
-// Extrapolated eta back into the fields from whichever ping-pong buffer set
-// holds the sweeps' result.
-__global__ void soft_lsq_back_kernel(double* __restrict__ e1, double* __restrict__ e2,
-                                     const double* __restrict__ e1d,
-                                     const double* __restrict__ e2d,
-                                     const double* __restrict__ e1d2,
-                                     const double* __restrict__ e2d2,
-                                     const int16_t* __restrict__ tgt,
-                                     const unsigned* __restrict__ counters, int sweeps, int64_t n,
-                                     int64_t off) {
-  __shared__ int s_second;  // the same for every cell: once per workgroup
-  if (threadIdx.x == 0) s_second = lsq_result_is_second(counters, sweeps) ? 1 : 0;
-  __syncthreads();
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n) return;
-  if (!tgt[off + c]) {  // outside the target zone: in * eta with in = 0
+// Extrapolated eta back into the fields: the target zone's cells from the
+// doubled grid's physical half; outside it in * eta with in = 0.
+__device__ __forceinline__ void soft_lsq_back_at(double* __restrict__ e1, double* __restrict__ e2,
+                                                 const double* __restrict__ e1d,
+                                                 const double* __restrict__ e2d,
+                                                 const double* __restrict__ phi,
+                                                 double extrap_zone, int64_t n, int64_t c) {
+  if (!(-phi[c] < extrap_zone)) {
     e1[c] = 0.0 * e1[c];
     e2[c] = 0.0 * e2[c];
     return;
   }
-  const bool second = s_second != 0;
-  e1[c] = (second ? e1d2 : e1d)[off + c];
-  e2[c] = (second ? e2d2 : e2d)[off + c];
+  e1[c] = e1d[n + c];
+  e2[c] = e2d[n + c];
 }
 
+__global__ void soft_lsq_back_kernel(double* __restrict__ e1, double* __restrict__ e2,
+                                     const double* __restrict__ e1d,
+                                     const double* __restrict__ e2d,
+                                     const double* __restrict__ phi, double extrap_zone,
+                                     int64_t n) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < n) soft_lsq_back_at(e1, e2, e1d, e2d, phi, extrap_zone, n, c);
+}
+
+// queue > 0: steps whose loop takes `queue` sweeps or more are counted.
 __device__ __forceinline__ void soft_finalize_body(double* __restrict__ sc,
-                                                   const unsigned* __restrict__ counters,
-                                                   int sweeps, unsigned* __restrict__ list_count,
+                                                   const unsigned* __restrict__ head, int queue,
                                                    unsigned* __restrict__ need) {
-  *list_count = 0u;  // for the next step's list of cells to extrapolate
-  // sweeps that fitted cells: the queued ones, then the tail's (its last
-  // sweep fits nothing)
-  int used = 0;
-  while (used < sweeps && counters[used] != 0u) ++used;
-  if (used == sweeps && counters[sweeps] != 0u) {
-    used += (int)counters[sweeps] - 1;
-    sc[kSsLsqUnconverged] = sc[kSsLsqUnconverged] + 1.0;  // steps the tail finished
-  }
+  const unsigned used = head[1];  // sweeps that fitted cells
+  if (queue > 0 && used >= (unsigned)queue) sc[kSsLsqUnconverged] = sc[kSsLsqUnconverged] + 1.0;
   sc[kSsLsqSweeps] = double(used);
-  atomicMax(need, (unsigned)used + 1u);  // sweeps this loop took
+  if (need) atomicMax(need, used + 1u);  // sweeps the reference's loop takes
   sc[kSsT] = sc[kSsT] + sc[kSsDt];
   sc[kSsIt] = sc[kSsIt] + 1.0;
 }
 
-__global__ void soft_finalize_kernel(double* __restrict__ sc,
-                                     const unsigned* __restrict__ counters, int sweeps,
-                                     unsigned* __restrict__ list_count,
-                                     unsigned* __restrict__ need, int streaming) {
+__global__ void soft_finalize_kernel(double* __restrict__ sc, const unsigned* __restrict__ head,
+                                     int queue, int streaming) {
   if (threadIdx.x != 0) return;
   if (streaming) sc[kSsFreqTimer] = sc[kSsFreqTimer] + sc[kSsDt];
-  soft_finalize_body(sc, counters, sweeps, list_count, need);
+  soft_finalize_body(sc, head, queue, nullptr);
 }
 
 template <typename T>
@@ -332,7 +329,6 @@ struct SoftStepperT {
   B *w0 = nullptr, *w1 = nullptr, *tmp = nullptr, *spec = nullptr;
   double *e1n = nullptr, *e2n = nullptr, *slots = nullptr;
   double *e1d = nullptr, *e2d = nullptr;
-  int16_t *cur = nullptr, *tgt = nullptr;
   B *s11 = nullptr, *s12 = nullptr, *s22 = nullptr;
   B *g1z = nullptr, *g1r = nullptr, *g2z = nullptr, *g2r = nullptr;
   B *tz = nullptr, *tr = nullptr;
@@ -341,15 +337,7 @@ struct SoftStepperT {
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
   hipStream_t graph_stream = nullptr;
-  // queued-sweep growth: the most sweeps a step has taken (device), its
-  // pinned host copy and the event that says the copy has landed
-  static constexpr int kMaxQueued = 4096;
-  unsigned* need = nullptr;
-  unsigned* need_host = nullptr;
-  hipEvent_t need_ev = nullptr;
-  bool need_pending = false;
-  int since_request = 0;  // graph launches queued after the pending copy
-  int* zone = nullptr;    // batch cases: the target zone's rows (zone_row)
+  int* zone = nullptr;    // the target zone's rows, then the last step's (zone_row)
 
   template <typename P>
   hipError_t alloc(P** p, size_t bytes) {
@@ -394,11 +382,18 @@ struct SoftStepperT {
     if ((e = alloc(&rw.cnt, 3 * sizeof(unsigned))) != hipSuccess) return e;
     if ((e = alloc(&e1d, nd * D8)) != hipSuccess) return e;
     if ((e = alloc(&e2d, nd * D8)) != hipSuccess) return e;
-    if ((e = alloc(&cur, nd * sizeof(int16_t))) != hipSuccess) return e;
-    if ((e = alloc(&tgt, nd * sizeof(int16_t))) != hipSuccess) return e;
-    if ((e = alloc(&lw.counters, sizeof(unsigned) * (kMaxQueued + 1))) != hipSuccess) return e;
-    if ((e = alloc(&need, sizeof(unsigned))) != hipSuccess) return e;
-    if ((e = hipMemset(need, 0, sizeof(unsigned))) != hipSuccess) return e;
+    lw.wstride = lsq_words(cfg.nz);
+    lw.fcap = lsq_factor_cap((int64_t)nd);
+    const size_t wb = sizeof(unsigned) * 2 * (size_t)cfg.nr * lw.wstride;
+    for (unsigned** f : {&lw.kb, &lw.tb, &lw.kw, &lw.tw, &lw.fw})
+      if ((e = alloc(f, wb)) != hipSuccess) return e;
+    if ((e = alloc(&lw.lev, nd * sizeof(int))) != hipSuccess) return e;
+    if ((e = alloc(&lw.list, nd * sizeof(LsqEntry))) != hipSuccess) return e;
+    const size_t fronts = (size_t)lsq_max_fronts((int64_t)nd) + 1;
+    if ((e = alloc(&lw.off, fronts * sizeof(int))) != hipSuccess) return e;
+    if ((e = alloc(&lw.head, 2 * sizeof(unsigned))) != hipSuccess) return e;
+    if ((e = alloc(&lw.win, nd * sizeof(unsigned))) != hipSuccess) return e;
+    if ((e = alloc(&lw.fac, 9 * (size_t)lw.fcap * D8)) != hipSuccess) return e;
     // every row: the first step a case takes here visits the whole grid
     // (its flags and values are written nowhere else before it), also when
     // its state was loaded from another run
@@ -406,20 +401,6 @@ struct SoftStepperT {
     if ((e = alloc(&zone, sizeof(all_rows))) != hipSuccess) return e;
     if ((e = hipMemcpy(zone, all_rows, sizeof(all_rows), hipMemcpyHostToDevice)) != hipSuccess)
       return e;
-    if (cfg.lsq_grow) {
-      if ((e = hipHostMalloc(reinterpret_cast<void**>(&need_host), sizeof(unsigned),
-                             hipHostMallocDefault)) != hipSuccess)
-        return e;
-      if ((e = hipEventCreateWithFlags(&need_ev, hipEventDisableTiming)) != hipSuccess) return e;
-    }
-    if ((e = alloc(&lw.list, nd * sizeof(int))) != hipSuccess) return e;
-    if ((e = alloc(&lw.tail, 4 * nd * sizeof(int))) != hipSuccess) return e;
-    lw.cap = (int)nd;
-    if ((e = alloc(&lw.cur2, nd * sizeof(int16_t))) != hipSuccess) return e;
-    if ((e = alloc(&lw.ex2, nd * D8)) != hipSuccess) return e;
-    if ((e = alloc(&lw.ey2, nd * D8)) != hipSuccess) return e;
-    if ((e = alloc(&lw.count, sizeof(unsigned))) != hipSuccess) return e;
-    if ((e = hipMemset(lw.count, 0, sizeof(unsigned))) != hipSuccess) return e;
     if ((e = alloc(&slots, D8 * kSlotsPerCase)) != hipSuccess) return e;
     // scratch the reference allocates once and never fully rewrites
     // (gradient and tau scratch keep zeros where they are never written)
@@ -431,7 +412,7 @@ struct SoftStepperT {
     if ((e = hipGetLastError()) != hipSuccess) return e;
     // the doubled grid's values: cells outside a step's target zone keep
     // what they hold, which must be finite
-    for (double* f : {e1d, e2d, lw.ex2, lw.ey2}) {
+    for (double* f : {e1d, e2d}) {
       soft_zero_kernel<double><<<ceil_div((int64_t)nd, 256), 256>>>(f, (int64_t)nd, 1);
       if ((e = hipGetLastError()) != hipSuccess) return e;
     }
@@ -441,8 +422,6 @@ struct SoftStepperT {
 
   ~SoftStepperT() {
     drop_graphs();
-    if (need_ev) (void)hipEventDestroy(need_ev);
-    if (need_host) (void)hipHostFree(need_host);
     for (void* p : allocs) (void)hipFree(p);
     delete plan;
   }
@@ -472,7 +451,7 @@ struct SoftStepperT {
     const int mb = std::min<int64_t>(ceil_div(n, 256), 1024);
     soft_velocity_max_kernel<<<mb, 256, 0, s>>>(buf.u_z, buf.u_r, n, slots);
     AXS_TRY_LAUNCH();
-    soft_dt_kernel<<<1, 64, 0, s>>>(sc, slots, cfg);
+    soft_dt_kernel<<<1, 64, 0, s>>>(sc, slots, zone, cfg);
     AXS_TRY_LAUNCH();
     AXS_TRY_STEP(launch_eno3_refmap<double>(buf.eta1, buf.eta2, buf.u_z, buf.u_r, e1n, e2n, nr,
                                             nz, Scalar<double>{0.0, sc + kSsDtByDx}, s));
@@ -486,24 +465,12 @@ struct SoftStepperT {
                                                     Scalar<double>{0.0, sc + kSsDtByDx}, -1.0,
                                                     s));
     soft_lsq_mirror_kernel<<<dim3(ceil_div(nz, 256), 2 * nr), 256, 0, s>>>(
-        buf.phi, buf.char_func, cfg.moll_zone, buf.eta1, buf.eta2, e1d, e2d, cur, tgt, lw.ex2,
-        lw.ey2, lw.cur2, nr, nz, cfg.extrap_zone, lw.counters, cfg.lsq_sweeps + 1);
+        buf.phi, buf.char_func, cfg.moll_zone, buf.eta1, buf.eta2, e1d, e2d, lw, zone, nr, nz,
+        cfg.extrap_zone);
     AXS_TRY_LAUNCH();
-    AXS_TRY_STEP(launch_lsq_list(cur, tgt, 2 * n, lw, s));
-    // ping-pong sweeps (sweep q reads the first set when q is even); those
-    // after the loop has ended return at once
-    for (int q = 0; q < cfg.lsq_sweeps; ++q) {
-      const bool odd = q & 1;
-      AXS_TRY_STEP(launch_lsq_sweep_pingpong(odd ? lw.cur2 : cur, odd ? lw.ex2 : e1d,
-                                             odd ? lw.ey2 : e2d, odd ? cur : lw.cur2,
-                                             odd ? e1d : lw.ex2, odd ? e2d : lw.ey2, tgt, buf.z,
-                                             buf.z, 2 * nr, nz, lw, q, s));
-    }
-    // a loop longer than the queued sweeps ends in one workgroup
-    AXS_TRY_STEP(launch_lsq_sweep_tail(cur, e1d, e2d, tgt, buf.z, buf.z, 2 * nr, nz, lw,
-                                       cfg.lsq_sweeps, s));
-    soft_lsq_back_kernel<<<ceil_div(n, 256), 256, 0, s>>>(
-        buf.eta1, buf.eta2, e1d, e2d, lw.ex2, lw.ey2, tgt, lw.counters, cfg.lsq_sweeps, n, n);
+    AXS_TRY_STEP(launch_lsq_fronts(lw, e1d, e2d, buf.z, nr, nz, zone, s));
+    soft_lsq_back_kernel<<<ceil_div(n, 256), 256, 0, s>>>(buf.eta1, buf.eta2, e1d, e2d, buf.phi,
+                                                          cfg.extrap_zone, n);
     AXS_TRY_LAUNCH();
     // the TG driver (:186-213) adds the stress to the tapered vorticity and
     // then advects it; the streaming driver (:198-264) advects it first
@@ -528,7 +495,7 @@ struct SoftStepperT {
     AXS_TRY_STEP(launch_rk2<double, RRow<double>>(
         w1, tmp, buf.vorticity, RRow<double>{buf.r}, nr, nz, Scalar<double>{0.0, sc + kSsHalfNuDt},
         Scalar<double>{0.0, sc + kSsNuDt}, cfg.dx, s));
-    soft_finalize_kernel<<<1, 64, 0, s>>>(sc, lw.counters, cfg.lsq_sweeps, lw.count, need,
+    soft_finalize_kernel<<<1, 64, 0, s>>>(sc, lw.head, cfg.lsq_grow ? 0 : cfg.lsq_sweeps,
                                           cfg.streaming);
     AXS_TRY_LAUNCH();
 #undef AXS_TRY_STEP
@@ -572,36 +539,6 @@ struct SoftStepperT {
     return hipSuccess;
   }
 
-  // Queued-sweep growth (cfg.lsq_grow): a graph launch is followed by an
-  // asynchronous copy of the most sweeps a step has taken; once it has
-  // landed (polled; waited for only when 16 graph launches are queued behind
-  // it, so the device keeps ~128 steps of work) the queue grows to that + 4,
-  // rounded up to 4, and the graphs are dropped to be captured again.  Loops
-  // that outrun the queue meanwhile are finished by the extrapolation tail.
-  hipError_t poll_need() {
-    if (!need_pending) return hipSuccess;
-    hipError_t e = since_request >= 16 ? hipEventSynchronize(need_ev) : hipEventQuery(need_ev);
-    if (e == hipErrorNotReady) return hipSuccess;
-    if (e != hipSuccess) return e;
-    need_pending = false;
-    const int want = std::min(kMaxQueued, (int)((*need_host + 4u + 3u) / 4u * 4u));
-    if (want > cfg.lsq_sweeps) {
-      cfg.lsq_sweeps = want;
-      drop_graphs();
-    }
-    return hipSuccess;
-  }
-  hipError_t request_need(hipStream_t s) {
-    if (need_pending) return hipSuccess;
-    hipError_t e = hipMemcpyAsync(need_host, need, sizeof(unsigned), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipEventRecord(need_ev, s);
-    if (e == hipSuccess) {
-      need_pending = true;
-      since_request = 0;
-    }
-    return e;
-  }
-
   hipError_t run(int nsteps, bool use_graph, hipStream_t s) {
     if (!use_graph) {
       for (int q = 0; q < nsteps; ++q) {
@@ -614,13 +551,10 @@ struct SoftStepperT {
     hipError_t e = hipSuccess;
     int q = 0;
     while (q < nsteps) {
-      if (cfg.lsq_grow && (e = poll_need()) != hipSuccess) return e;
       if (!graph_exec && (e = capture(s)) != hipSuccess) return e;
       const bool chunk = q + kChunkSteps <= nsteps;
       if ((e = hipGraphLaunch(chunk ? chunk_exec : graph_exec, s)) != hipSuccess) return e;
       q += chunk ? kChunkSteps : 1;
-      ++since_request;
-      if (cfg.lsq_grow && (e = request_need(s)) != hipSuccess) return e;
     }
     return hipSuccess;
   }
@@ -654,20 +588,18 @@ __global__ void soft_batch_pin_kernel(const SoftCaseT<B>* __restrict__ cs,
 }
 
 template <typename B>
-__global__ void soft_batch_mirror_kernel(const SoftCaseT<B>* __restrict__ cs,
-                                         const uint32_t* __restrict__ blocks, int ncounters) {
+__global__ void __launch_bounds__(256) soft_batch_mirror_kernel(
+    const SoftCaseT<B>* __restrict__ cs, const uint32_t* __restrict__ blocks) {
   const SoftBlock b = soft_block(blocks);  // a row of the doubled grid
   const SoftCaseT<B>& C = cs[b.c];
-  if (b.i == 0 && b.j < 256)  // the case's first workgroup clears its sweep counters
-    for (int k = threadIdx.x; k < ncounters; k += blockDim.x) C.lw.counters[k] = 0u;
   // rows beyond the last zone keep their flags (0) and chi (0) from the
   // step that last visited them (the whole workgroup leaves together)
   if (!prev_zone_row(C, b.i >= C.nr ? b.i - C.nr : C.nr - 1 - b.i)) return;
-  bool target = false;
+  bool known = false, target = false;
   if (b.j < C.nz)
-    target = soft_lsq_mirror_at(C.phi, C.chi, C.moll_zone, C.eta1, C.eta2, C.e1d, C.e2d, C.cur,
-                                C.tgt, C.lw.ex2, C.lw.ey2, C.lw.cur2, C.nr, C.nz,
-                                C.extrap_zone, b.i, b.j);
+    soft_lsq_mirror_at(C.phi, C.chi, C.moll_zone, C.eta1, C.eta2, C.e1d, C.e2d, C.lw.lev, C.nr,
+                       C.nz, C.extrap_zone, b.i, b.j, known, target);
+  soft_lsq_flag_bits(C.lw, b.i, b.j, known, target);
   // the workgroup is one row segment: its row joins the zone if any cell
   // of the segment is a target (upper half: the physical rows)
   if (__syncthreads_or(target) && b.i >= C.nr && threadIdx.x == 0) {
@@ -678,40 +610,26 @@ __global__ void soft_batch_mirror_kernel(const SoftCaseT<B>* __restrict__ cs,
 
 template <typename B>
 __global__ void soft_batch_back_kernel(const SoftCaseT<B>* __restrict__ cs,
-                                       const uint32_t* __restrict__ blocks, int sweeps) {
-  __shared__ int s_second;
+                                       const uint32_t* __restrict__ blocks) {
   const SoftBlock b = soft_block(blocks);
   const SoftCaseT<B>& C = cs[b.c];
-  if (!zone_row(C, b.i)) return;  // the whole workgroup (one row)
-  if (threadIdx.x == 0) s_second = lsq_result_is_second(C.lw.counters, sweeps) ? 1 : 0;
-  __syncthreads();
-  if (b.j >= C.nz) return;
-  const int64_t n = (int64_t)C.nr * C.nz, c = (int64_t)b.i * C.nz + b.j;
-  if (!C.tgt[n + c]) {  // outside the target zone: in * eta with in = 0
-    C.eta1[c] = 0.0 * C.eta1[c];
-    C.eta2[c] = 0.0 * C.eta2[c];
-    return;
-  }
-  const bool second = s_second != 0;
-  C.eta1[c] = (second ? C.lw.ex2 : C.e1d)[n + c];
-  C.eta2[c] = (second ? C.lw.ey2 : C.e2d)[n + c];
+  if (b.j >= C.nz || !zone_row(C, b.i)) return;
+  soft_lsq_back_at(C.eta1, C.eta2, C.e1d, C.e2d, C.phi, C.extrap_zone, (int64_t)C.nr * C.nz,
+                   (int64_t)b.i * C.nz + b.j);
 }
 
 template <typename B>
-__global__ void soft_batch_finalize_kernel(const SoftCaseT<B>* __restrict__ cs, int sweeps) {
+__global__ void soft_batch_finalize_kernel(const SoftCaseT<B>* __restrict__ cs) {
   if (threadIdx.x != 0) return;
   const SoftCaseT<B>& C = cs[blockIdx.x];
-  soft_finalize_body(C.scalars, C.lw.counters, sweeps, C.lw.count, C.need);
+  soft_finalize_body(C.scalars, C.lw.head, 0, C.need);
 }
 
 // Many soft cases stepped together: each pass of the step is one launch over
 // all cases (SoftCaseT table on the device), in the single-case step's
 // order, so a case's results are the same bits alone and in any mix.  Cases
 // join and leave between runs; the step graphs are captured again after a
-// change.  The extrapolation queue (sweeps launched per step) is the
-// batch's, grown from the most sweeps any case has taken as in the single
-// stepper; the result never depends on it (a longer loop is finished by each
-// case's tail workgroup).
+// change.
 template <typename B>
 struct SoftBatchT {
   struct Entry {
@@ -724,12 +642,7 @@ struct SoftBatchT {
   SoftCaseT<B>* d_cases = nullptr;
   std::vector<SoftCaseT<B>> h_cases;
   SoftBatchDims dims{};
-  int sweeps = 12;
-  unsigned* need = nullptr;
-  unsigned* need_host = nullptr;
-  hipEvent_t need_ev = nullptr;
-  bool need_pending = false;
-  int since_request = 0;
+  unsigned* need = nullptr;  // most sweeps an extrapolation loop has taken (device)
   static constexpr int kChunkSteps = 8;
   hipGraph_t graph = nullptr, chunk_graph = nullptr;
   hipGraphExec_t graph_exec = nullptr, chunk_exec = nullptr;
@@ -748,12 +661,7 @@ struct SoftBatchT {
     if (e != hipSuccess) return e;
     if ((e = hipMalloc(reinterpret_cast<void**>(&need), sizeof(unsigned))) != hipSuccess) return e;
     if ((e = hipMemset(need, 0, sizeof(unsigned))) != hipSuccess) return e;
-    if ((e = hipMalloc(reinterpret_cast<void**>(&d_rcnt), 3 * sizeof(unsigned))) != hipSuccess)
-      return e;
-    if ((e = hipHostMalloc(reinterpret_cast<void**>(&need_host), sizeof(unsigned),
-                           hipHostMallocDefault)) != hipSuccess)
-      return e;
-    return hipEventCreateWithFlags(&need_ev, hipEventDisableTiming);
+    return hipMalloc(reinterpret_cast<void**>(&d_rcnt), 3 * sizeof(unsigned));
   }
 
   void drop_graphs() {
@@ -771,8 +679,6 @@ struct SoftBatchT {
     (void)hipDeviceSynchronize();
     drop_graphs();
     for (Entry& c : cases) delete c.st;
-    if (need_ev) (void)hipEventDestroy(need_ev);
-    if (need_host) (void)hipHostFree(need_host);
     if (need) (void)hipFree(need);
     if (d_cases) (void)hipFree(d_cases);
     if (d_blocks) (void)hipFree(d_blocks);
@@ -822,8 +728,6 @@ struct SoftBatchT {
     C.slots = S.slots;
     C.e1d = S.e1d;
     C.e2d = S.e2d;
-    C.cur = S.cur;
-    C.tgt = S.tgt;
     C.s11 = S.s11;
     C.s12 = S.s12;
     C.s22 = S.s22;
@@ -943,10 +847,7 @@ struct SoftBatchT {
     if ((int)cases.size() >= max_cases) return hipErrorInvalidValue;
     SoftStepperT<B>* st = new (std::nothrow) SoftStepperT<B>();
     if (!st) return hipErrorOutOfMemory;
-    SoftConfig cc = c;
-    cc.lsq_sweeps = kMaxQueued;  // counters sized for the largest queue
-    cc.lsq_grow = 0;
-    hipError_t e = st->init(cc, b, true);
+    hipError_t e = st->init(c, b, true);
     if (e != hipSuccess) {
       delete st;
       return e;
@@ -976,8 +877,6 @@ struct SoftBatchT {
     return hipErrorInvalidValue;
   }
 
-  static constexpr int kMaxQueued = SoftStepper::kMaxQueued;
-
   hipError_t enqueue_step(hipStream_t s) {
     const SoftCaseT<B>* T = d_cases;
     const SoftBatchDims& d = dims;
@@ -1002,17 +901,15 @@ struct SoftBatchT {
     soft_batch_pin_kernel<B><<<d.ncell_blocks, 256, 0, s>>>(T, d.cell_blocks);
     AXS_TRY_LAUNCH();
     AXS_TRY_STEP(launch_soft_batch_reinit(T, d, iters, s));
-    soft_batch_mirror_kernel<B><<<d.ndbl_blocks, 256, 0, s>>>(T, d.dbl_blocks, sweeps + 1);
+    soft_batch_mirror_kernel<B><<<d.ndbl_blocks, 256, 0, s>>>(T, d.dbl_blocks);
     AXS_TRY_LAUNCH();
-    AXS_TRY_STEP(launch_soft_batch_lsq_list(T, d, s));
-    for (int q = 0; q < sweeps; ++q) AXS_TRY_STEP(launch_soft_batch_lsq_sweep(T, d, q, s));
-    AXS_TRY_STEP(launch_soft_batch_lsq_tail(T, d, sweeps, s));
-    soft_batch_back_kernel<B><<<d.ncell_blocks, 256, 0, s>>>(T, d.cell_blocks, sweeps);
+    AXS_TRY_STEP(launch_soft_batch_lsq(T, d, s));
+    soft_batch_back_kernel<B><<<d.ncell_blocks, 256, 0, s>>>(T, d.cell_blocks);
     AXS_TRY_LAUNCH();
     AXS_TRY_STEP(launch_soft_batch_stress(T, d, s));
     AXS_TRY_STEP(launch_soft_batch_advect(T, d, s));
     AXS_TRY_STEP(launch_soft_batch_diffuse(T, d, s));
-    soft_batch_finalize_kernel<B><<<d.ncase, 64, 0, s>>>(T, sweeps);
+    soft_batch_finalize_kernel<B><<<d.ncase, 64, 0, s>>>(T);
     AXS_TRY_LAUNCH();
 #undef AXS_TRY_STEP
 #undef AXS_TRY_LAUNCH
@@ -1039,31 +936,6 @@ struct SoftBatchT {
     return hipSuccess;
   }
 
-  // Queue growth as in SoftStepper::poll_need.
-  hipError_t poll_need() {
-    if (!need_pending) return hipSuccess;
-    hipError_t e = since_request >= 16 ? hipEventSynchronize(need_ev) : hipEventQuery(need_ev);
-    if (e == hipErrorNotReady) return hipSuccess;
-    if (e != hipSuccess) return e;
-    need_pending = false;
-    const int want = std::min(kMaxQueued, (int)((*need_host + 4u + 3u) / 4u * 4u));
-    if (want > sweeps) {
-      sweeps = want;
-      drop_graphs();
-    }
-    return hipSuccess;
-  }
-  hipError_t request_need(hipStream_t s) {
-    if (need_pending) return hipSuccess;
-    hipError_t e = hipMemcpyAsync(need_host, need, sizeof(unsigned), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipEventRecord(need_ev, s);
-    if (e == hipSuccess) {
-      need_pending = true;
-      since_request = 0;
-    }
-    return e;
-  }
-
   hipError_t run(int nsteps, bool use_graph, hipStream_t s) {
     hipError_t e;
     if (table_dirty && (e = refresh()) != hipSuccess) return e;
@@ -1076,14 +948,11 @@ struct SoftBatchT {
     if (graph_stream != s) drop_graphs();
     int q = 0;
     while (q < nsteps) {
-      if ((e = poll_need()) != hipSuccess) return e;
       if (!graph_exec && (e = capture(s)) != hipSuccess) return e;
       const bool chunk = q + kChunkSteps <= nsteps;
       if ((e = hipGraphLaunch(chunk ? chunk_exec : graph_exec, s)) != hipSuccess) return e;
       ++(chunk ? chunk_launches : step_launches);
       q += chunk ? kChunkSteps : 1;
-      ++since_request;
-      if ((e = request_need(s)) != hipSuccess) return e;
     }
     return hipSuccess;
   }
@@ -1283,9 +1152,15 @@ axs_status axs_soft_batch_run(axs_soft_batch* bt, int nsteps, int use_graph, voi
 axs_status axs_soft_batch_info(const axs_soft_batch* bt, int* ncase, int* queued_sweeps,
                                int64_t* graph_launches, int64_t* captures) {
   AXS_CHECK_ARG(bt, "null batch");
+  if (queued_sweeps) {
+    unsigned need = 0u;
+    AXS_HIP(bt->with([&](const auto& b) {
+      return hipMemcpy(&need, b.need, sizeof(unsigned), hipMemcpyDeviceToHost);
+    }));
+    *queued_sweeps = std::max(12, (int)((need + 4u + 3u) / 4u * 4u));
+  }
   bt->with([&](const auto& b) {
     if (ncase) *ncase = (int)b.cases.size();
-    if (queued_sweeps) *queued_sweeps = b.sweeps;
     if (graph_launches) *graph_launches = b.chunk_launches + b.step_launches;
     if (captures) *captures = b.captures;
     return 0;

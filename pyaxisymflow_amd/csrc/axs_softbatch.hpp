@@ -53,7 +53,6 @@ struct SoftCaseT {
   // step scratch
   B *w0, *w1, *tmp, *spec;
   double *e1n, *e2n, *slots, *e1d, *e2d;
-  int16_t *cur, *tgt;
   B *s11, *s12, *s22, *g1z, *g1r, *g2z, *g2r, *tz, *tr;
   ReinitWork rw;
   int reinit_tile_base;  // the case's first entry in the batch's reinit tile table
@@ -111,7 +110,7 @@ __device__ __forceinline__ SoftBlock soft_block(const uint32_t* __restrict__ t) 
 }
 
 // Rows of a case that the passes after the mirror (copy back, stress,
-// stress divergence, extrapolation list) visit: the extrapolation's target
+// stress divergence) visit: the extrapolation's target
 // zone, recorded by the mirror pass of the same step, and kZoneMargin rows
 // either side; every row in the case's first step.  Beyond them the
 // reference map is zero (the copy back zeroes it outside the target zone,
@@ -160,14 +159,7 @@ template <typename B>
 hipError_t launch_soft_batch_reinit(const SoftCaseT<B>* cases, const SoftBatchDims& d,
                                     int iterations, hipStream_t s);
 template <typename B>
-hipError_t launch_soft_batch_lsq_list(const SoftCaseT<B>* cases, const SoftBatchDims& d,
-                                      hipStream_t s);
-template <typename B>
-hipError_t launch_soft_batch_lsq_sweep(const SoftCaseT<B>* cases, const SoftBatchDims& d,
-                                       int sweep, hipStream_t s);
-template <typename B>
-hipError_t launch_soft_batch_lsq_tail(const SoftCaseT<B>* cases, const SoftBatchDims& d,
-                                      int sweeps, hipStream_t s);
+hipError_t launch_soft_batch_lsq(const SoftCaseT<B>* cases, const SoftBatchDims& d, hipStream_t s);
 template <typename B>
 hipError_t launch_soft_batch_stress(const SoftCaseT<B>* cases, const SoftBatchDims& d,
                                     hipStream_t s);

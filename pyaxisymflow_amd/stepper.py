@@ -670,14 +670,11 @@ class SoftSphereStepper(_Checkpoint):
     1 / grid_size_z, nr = domain_AR * nz, moll_zone = 4 dx, extrap_zone =
     reinit_band = moll_zone + 4 dx, sphere of radius r_ball at (0.5, 0),
     vorticity C (kz^2 + kr^2) sin(kz z) sin(kr r) with kz = kr = 2 pi.
-    ``lsq_sweeps`` fixes the number of extrapolation sweeps queued per step
-    as separate launches; by default the queue starts at 12 and grows with
-    the most sweeps a step has needed (+ 4, rounded up to 4) as graph runs
-    learn it. The reference loops until a sweep fits nothing, which takes
-    8-21 sweeps for stiff solids and up to ~60 for the softest as they
-    deform; a loop longer than the queue is finished by one workgroup, so
-    the result is always the reference loop's. ``lsq_unconverged()`` counts
-    the steps the one-workgroup tail finished."""
+    The extrapolation runs the reference's sweeps until one fits nothing
+    (8-21 sweeps for stiff solids, up to ~60 for the softest as they
+    deform), all within the step's launches.  With ``lsq_sweeps`` given,
+    ``lsq_unconverged()`` counts the steps whose loop took that many sweeps
+    or more; the results do not depend on it."""
 
     _STATE = _SOFT_STATE
 
@@ -688,10 +685,6 @@ class SoftSphereStepper(_Checkpoint):
         self.use_graph = use_graph
         self.stream = torch.cuda.Stream(device=dev)
         _soft_case_state(self, grid_size_z, G, nu, rho_f, r_ball, domain_AR, C, kill_width)
-        # the reference's loop needs ~ band / dx sweeps at first and more as
-        # the solid deforms (15-21 for G >= 1 at nz = 512, ~60 after 1000
-        # steps at G = 0.1); every queued sweep costs a graph node (~5 us)
-        # even after the loop has ended, a tail sweep ~50 us
         if lsq_sweeps:
             self.cfg.lsq_sweeps, self.cfg.lsq_grow = int(lsq_sweeps), 0
         torch.cuda.synchronize(dev)
@@ -877,8 +870,9 @@ class SoftSphereBatch:
         self.stream.synchronize()
 
     def info(self):
-        """(cases, extrapolation sweeps queued per step, graph launches,
-        graph captures)."""
+        """(cases, an upper figure for the extrapolation sweeps of a step,
+        graph launches, graph captures).  The sweeps figure is the most any
+        step has taken + 4, rounded up to 4, and at least 12."""
         n, q = ctypes.c_int(), ctypes.c_int()
         g, c = ctypes.c_int64(), ctypes.c_int64()
         _lib.call("axs_soft_batch_info", self._h, ctypes.byref(n), ctypes.byref(q),
