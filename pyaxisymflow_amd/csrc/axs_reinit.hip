@@ -21,6 +21,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <utility>
 
 namespace axs {
 
@@ -34,9 +35,25 @@ int reinit_iterations(double narrow, double dx) {
 // sweeps per launch; a tile's sweeps read its cells and a halo of 2 S
 // (its read region).
 constexpr int kRtR = kReinitTileRows, kRtZ = kReinitTileCols;
-constexpr int kReinitSweepsPerLaunch = 2;
-constexpr int kReinitHalo = 2 * kReinitSweepsPerLaunch;
-static_assert(kReinitHalo <= kRtR && kReinitHalo <= kRtZ,
+// Launch shape by the number of tiles.  A grid whose tiles fit on the chip
+// at once (four 512-thread workgroups per CU) is bound by the latency of a
+// launch (list, flag, tile loads, one dependent update per sweep): more
+// sweeps per launch, and threads for a sweep's cells in one or two goes.
+// Beyond that the launches are bound by the work of their tiles, which the
+// halo multiplies.  Measured per reinit of 24 to 26 sweeps: one 256 x 128
+// case 135 us with 2 sweeps by 256 threads, 94 with 2 by 512, 79 with 3 or 4
+// by 512; twelve cases of 130 to 491 rows (10,000 tiles) 186 us with 2 by
+// 256 (before the reciprocals of eikonal_update; 160 with them), 148 with 3
+// by 256, 175 with 3 by 512, 156 with 4 by 256.
+struct ReinitFew {
+  static constexpr int S = 4, threads = 512;
+};
+struct ReinitMany {
+  static constexpr int S = 3, threads = 256;
+};
+constexpr int kReinitFewTiles = 1024;
+constexpr int kReinitMostSweeps = 4;
+static_assert(2 * kReinitMostSweeps <= kRtR && 2 * kReinitMostSweeps <= kRtZ,
               "a read region must lie in the 3 x 3 tiles around its tile");
 __host__ __device__ __forceinline__ int reinit_tile_cols(int nz) {
   return (nz + kRtZ - 1) / kRtZ;
@@ -107,17 +124,17 @@ __device__ __forceinline__ void reinit_init_at(const double* __restrict__ phi,
     fr = true;
   }
   dist[c] = dv;
-  frozen[c] = fr ? 1 : 0;
+  frozen[c] = uint8_t((fr ? 1 : 0) | (p < 0.0 ? 2 : 0));
   D[c] = fr ? dv : kBig;
   D1[c] = fr ? dv : kBig;
   ch0[c] = fr ? 1 : 0;
   ch1[c] = 0;
   if (fr) {  // the tiles whose read region holds the cell run the first launch
     const int ntc = reinit_tile_cols(nz), ntr = reinit_tile_count(nr, nz) / ntc;
-    const int r0 = max(0, floor_div(i - kReinitHalo, kRtR));
-    const int r1 = min(ntr - 1, floor_div(i + kReinitHalo, kRtR));
-    const int q0 = max(0, floor_div(j - kReinitHalo, kRtZ));
-    const int q1 = min(ntc - 1, floor_div(j + kReinitHalo, kRtZ));
+    const int r0 = max(0, floor_div(i - 2 * kReinitMostSweeps, kRtR));
+    const int r1 = min(ntr - 1, floor_div(i + 2 * kReinitMostSweeps, kRtR));
+    const int q0 = max(0, floor_div(j - 2 * kReinitMostSweeps, kRtZ));
+    const int q1 = min(ntc - 1, floor_div(j + 2 * kReinitMostSweeps, kRtZ));
     for (int r = r0; r <= r1; ++r)
       for (int q = q0; q <= q1; ++q) tiles[r * ntc + q] = 1u;
   }
@@ -140,43 +157,30 @@ __global__ void reinit_init_kernel(const double* __restrict__ phi, ReinitWork w,
 // sum(terms) = 1.  Where both axes enter and x is not above both axes'
 // upwind values, x comes from the axis with the smaller one alone (+ 2 dx/3
 // second order, + dx first order).
-// The iterate as the update reads it: kBig outside the domain (a neighbour
-// beyond the edge is not known).  From a global array, or from an LDS tile
-// of width w whose origin is global cell (i0, j0).
-struct GlobalIterate {
-  const double* __restrict__ D;
-  int nr, nz;
-  __device__ __forceinline__ double at(int i, int j) const {
-    return (i >= 0 && i < nr && j >= 0 && j < nz) ? D[(int64_t)i * nz + j] : kBig;
-  }
-};
-struct TileIterate {
-  const double* T;
-  int i0, j0, w, nr, nz;
-  __device__ __forceinline__ double at(int i, int j) const {
-    return (i >= 0 && i < nr && j >= 0 && j < nz) ? T[(i - i0) * w + (j - j0)] : kBig;
-  }
-};
-
-template <class IT>
-__device__ __forceinline__ double eikonal_update(const IT& D, int i, int j, double side,
-                                                 double dx) {
+// T: the cell's entry in an LDS tile of width w (kBig outside the domain: a
+// neighbour beyond the edge is not known); rcp[3 m + n] = RN(1 / (2 a)) for
+// the m-th and n-th term of the two axes (0 none, 1 first order, 2 second).
+// The quotients by 3 and 2 a take the reciprocal form (div_by: correctly
+// rounded, the values are distances and far from the range's ends).
+template <int W>
+__device__ __forceinline__ double eikonal_update(const double* __restrict__ T, double side,
+                                                 double dx, const double* __restrict__ rcp) {
   const double idx2 = 1.0 / (dx * dx);
   const double aa = 9.0 / 4.0;
   double a = 0.0, b = 0.0, c = 0.0;
   double tps[2], steps[2];
   bool used[2];
+  int term = 0;
 #pragma unroll
   for (int axis = 0; axis < 2; ++axis) {
+    const int st = axis == 0 ? W : 1;
     double v1 = kBig, v2 = kBig;
 #pragma unroll
     for (int s = -1; s <= 1; s += 2) {
-      const int i1 = axis == 0 ? i + s : i, j1 = axis == 0 ? j : j + s;
-      const int i2 = axis == 0 ? i + 2 * s : i, j2 = axis == 0 ? j : j + 2 * s;
       double n1 = kBig, n2 = kBig;
-      const double u1 = D.at(i1, j1);
+      const double u1 = T[s * st];
       if (u1 < kBig) n1 = side * u1;
-      const double u2 = D.at(i2, j2);
+      const double u2 = T[2 * s * st];
       if (u2 < kBig) n2 = side * u2;
       if (n1 < v1) {
         v2 = (n2 <= n1) ? n2 : kBig;
@@ -187,40 +191,22 @@ __device__ __forceinline__ double eikonal_update(const IT& D, int i, int j, doub
     const bool first = v1 < kBig && !second;
     const double w1 = (v1 < kBig) ? v1 : 0.0;
     const double w2 = second ? v2 : 0.0;
-    const double tp = second ? (4.0 * w1 - w2) / 3.0 : w1;
+    const double tp = second ? div_by(4.0 * w1 - w2, 3.0, 1.0 / 3.0) : w1;
     a = a + (second ? idx2 * aa : (first ? idx2 : 0.0));
     b = b - (second ? idx2 * 2.0 * aa * tp : (first ? idx2 * 2.0 * w1 : 0.0));
     c = c + (second ? idx2 * aa * tp * tp : (first ? idx2 * w1 * w1 : 0.0));
     used[axis] = second || first;
     tps[axis] = used[axis] ? tp : kBig;
     steps[axis] = second ? (2.0 / 3.0) * dx : dx;
+    term = 3 * term + (second ? 2 : (first ? 1 : 0));
   }
   if (!(a > 0.0)) return kBig;
   c = c - 1.0;
   const double det = b * b - 4.0 * a * c;
-  double x = (-b + sqrt(fmax(det, 0.0))) / (2.0 * a);
+  double x = div_by(-b + sqrt(fmax(det, 0.0)), 2.0 * a, rcp[term]);
   if (used[0] && used[1] && (det < 0.0 || x < tps[0] || x < tps[1]))
     x = (tps[0] <= tps[1]) ? tps[0] + steps[0] : tps[1] + steps[1];
   return x;
-}
-
-// One Jacobi sweep: every cell that is not frozen takes its update from the
-// previous iterate (values may move either way: the second-order update is
-// not monotone in its neighbours).
-__device__ __forceinline__ void reinit_sweep_at(const double* __restrict__ Din,
-                                                double* __restrict__ Dout,
-                                                const double* __restrict__ phi,
-                                                const uint8_t* __restrict__ frozen, int nr,
-                                                int nz, double dx, int i, int j) {
-  const int64_t c = (int64_t)i * nz + j;
-  const double dc = Din[c];
-  if (frozen[c]) {
-    Dout[c] = dc;
-    return;
-  }
-  const double side = (phi[c] < 0.0) ? -1.0 : 1.0;
-  const double m = eikonal_update(GlobalIterate{Din, nr, nz}, i, j, side, dx);
-  Dout[c] = (m >= kBig) ? dc : side * m;
 }
 
 // S Jacobi sweeps of one 8 x 32 tile in LDS (temporal blocking): the tile
@@ -234,15 +220,17 @@ template <int S>
 struct ReinitTile {
   static constexpr int H = 2 * S, RR = kRtR + 2 * H, RZ = kRtZ + 2 * H, NC = RR * RZ;
   double a[NC], b[NC];
+  double rcp[9];  // RN(1 / (2 a)) of eikonal_update
   uint8_t f[NC];
   uint8_t ca[NC], cb[NC];  // changed by the sweep before (ping-pong)
 };
 
 // The tiles (neighbour index (dr + 1) * 3 + dc + 1, itself = 4) whose read
 // region holds cell (a, b) of a tile.
+template <int H>
 __device__ __forceinline__ unsigned reinit_touch(int a, int b) {
-  const unsigned rows = 2u | (a < kReinitHalo ? 1u : 0u) | (a >= kRtR - kReinitHalo ? 4u : 0u);
-  const unsigned cols = 2u | (b < kReinitHalo ? 1u : 0u) | (b >= kRtZ - kReinitHalo ? 4u : 0u);
+  const unsigned rows = 2u | (a < H ? 1u : 0u) | (a >= kRtR - H ? 4u : 0u);
+  const unsigned cols = 2u | (b < H ? 1u : 0u) | (b >= kRtZ - H ? 4u : 0u);
   unsigned m = 0u;
 #pragma unroll
   for (int r = 0; r < 3; ++r)
@@ -260,13 +248,12 @@ __device__ __forceinline__ unsigned reinit_touch(int a, int b) {
 // `more`.
 template <int S>
 __device__ __forceinline__ void reinit_tile_step(
-    const double* __restrict__ Din, double* __restrict__ Dout, const double* __restrict__ phi,
+    const double* __restrict__ Din, double* __restrict__ Dout,
     const uint8_t* __restrict__ frozen, const uint8_t* __restrict__ ch_in,
     uint8_t* __restrict__ ch_out, unsigned* __restrict__ flags_k, unsigned* __restrict__ flags_n,
     unsigned* __restrict__ list_n, unsigned* __restrict__ cnt_n, unsigned base, bool more, int nr,
     int nz, double dx, int tr, int tc, int nsw, ReinitTile<S>& L) {
   using Tl = ReinitTile<S>;
-  static_assert(Tl::H == kReinitHalo, "read region");
   const int tid = threadIdx.x, nth = blockDim.x;
   const int ti0 = tr * kRtR, tj0 = tc * kRtZ;
   const int ntc = reinit_tile_cols(nz), ntr = reinit_tile_count(nr, nz) / ntc;
@@ -277,24 +264,13 @@ __device__ __forceinline__ void reinit_tile_step(
     flags_k[t] = 0u;
     s_touch = 0u;
   }
-  __syncthreads();
-  if (!(s_flag & 1u)) {  // ran last launch, quiet since: bring the other buffer up to date
-    for (int e = tid; e < kRtR * kRtZ; e += nth) {
-      const int i = ti0 + e / kRtZ, j = tj0 + e % kRtZ;
-      if (i >= nr || j >= nz) continue;
-      const int64_t c = (int64_t)i * nz + j;
-      Dout[c] = Din[c];
-      ch_out[c] = 0;
-    }
-    __syncthreads();  // the shared words are read before the next tile sets them
-    return;
-  }
+  // the read region, loaded while the flag is still on its way
   for (int e = tid; e < Tl::NC; e += nth) {
     const int i = ti0 - Tl::H + e / Tl::RZ, j = tj0 - Tl::H + e % Tl::RZ;
     if (i >= 0 && i < nr && j >= 0 && j < nz) {
       const int64_t c = (int64_t)i * nz + j;
       L.a[e] = Din[c];
-      L.f[e] = uint8_t((frozen[c] ? 1 : 0) | (phi[c] < 0.0 ? 2 : 0));
+      L.f[e] = frozen[c];
       L.ca[e] = ch_in[c];
     } else {
       L.a[e] = kBig;
@@ -302,27 +278,47 @@ __device__ __forceinline__ void reinit_tile_step(
       L.ca[e] = 0;
     }
   }
+  if (tid >= 64 && tid < 73) {
+    const int m = (tid - 64) / 3, n = (tid - 64) % 3;
+    const double idx2 = 1.0 / (dx * dx), term[3] = {0.0, idx2, idx2 * (9.0 / 4.0)};
+    double a = 0.0;
+    a = a + term[m];
+    a = a + term[n];
+    L.rcp[tid - 64] = 1.0 / (2.0 * a);
+  }
   __syncthreads();
+  if (!(s_flag & 1u)) {  // ran last launch, quiet since: bring the other buffer up to date
+    for (int e = tid; e < kRtR * kRtZ; e += nth) {
+      const int a = e / kRtZ, b = e % kRtZ, i = ti0 + a, j = tj0 + b;
+      if (i >= nr || j >= nz) continue;
+      const int64_t c = (int64_t)i * nz + j;
+      Dout[c] = L.a[(a + Tl::H) * Tl::RZ + (b + Tl::H)];
+      ch_out[c] = 0;
+    }
+    __syncthreads();  // the shared words are read before the next tile sets them
+    return;
+  }
   double* A = L.a;
   double* B = L.b;
   uint8_t* CA = L.ca;
   uint8_t* CB = L.cb;
-  for (int s = 0; s < nsw; ++s) {
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    if (s >= nsw) break;
+    constexpr int RZ = Tl::RZ;
     const int h = Tl::H - 2 * (s + 1);  // halo of the cells this sweep updates
     const int w = kRtZ + 2 * h, n = (kRtR + 2 * h) * w;
-    const TileIterate it{A, ti0 - Tl::H, tj0 - Tl::H, Tl::RZ, nr, nz};
     for (int e = tid; e < n; e += nth) {
       const int a = e / w - h, b = e % w - h;  // tile-relative
-      const int li = (a + Tl::H) * Tl::RZ + (b + Tl::H);
+      const int li = (a + Tl::H) * RZ + (b + Tl::H);
       const uint8_t fl = L.f[li];
       const double dc = A[li];
       double v = dc;
-      const int RZ = Tl::RZ;
       const bool inputs_changed = CA[li - 2 * RZ] | CA[li - RZ] | CA[li + RZ] | CA[li + 2 * RZ] |
                                   CA[li - 2] | CA[li - 1] | CA[li + 1] | CA[li + 2];
       if (!(fl & 5) && inputs_changed) {
         const double side = (fl & 2) ? -1.0 : 1.0;
-        const double m = eikonal_update(it, ti0 + a, tj0 + b, side, dx);
+        const double m = eikonal_update<RZ>(A + li, side, dx, L.rcp);
         v = (m >= kBig) ? dc : side * m;
       }
       B[li] = v;
@@ -344,7 +340,7 @@ __device__ __forceinline__ void reinit_tile_step(
       const int li = (a + Tl::H) * Tl::RZ + (b + Tl::H);
       Dout[(int64_t)i * nz + j] = A[li];
       ch_out[(int64_t)i * nz + j] = CA[li];
-      if (CA[li]) touch |= reinit_touch(a, b);
+      if (CA[li]) touch |= reinit_touch<Tl::H>(a, b);
     }
   }
   if (touch) atomicOr(&s_touch, touch);
@@ -369,12 +365,13 @@ __global__ void reinit_first_list_kernel(const unsigned* __restrict__ flags, int
 
 // Launch k over its list: every workgroup takes entries blockIdx.x,
 // blockIdx.x + gridDim.x, ...
-template <int S>
-__global__ void __launch_bounds__(256) reinit_list_kernel(
-    const double* __restrict__ Din, double* __restrict__ Dout, const double* __restrict__ phi,
+template <class Shape>
+__global__ void __launch_bounds__(Shape::threads) reinit_list_kernel(
+    const double* __restrict__ Din, double* __restrict__ Dout,
     const uint8_t* __restrict__ frozen, const uint8_t* __restrict__ ch_in,
     uint8_t* __restrict__ ch_out, unsigned* __restrict__ flags, unsigned* __restrict__ list,
     unsigned* __restrict__ cnt, int nr, int nz, double dx, int k, int nsw, int more) {
+  constexpr int S = Shape::S;
   __shared__ ReinitTile<S> L;
   const int nt = reinit_tile_count(nr, nz), ntc = reinit_tile_cols(nz);
   const int p = k & 1;
@@ -382,7 +379,7 @@ __global__ void __launch_bounds__(256) reinit_list_kernel(
   const int n = (int)cnt[k % 3];
   for (int idx = blockIdx.x; idx < n; idx += gridDim.x) {
     const int t = (int)list[(size_t)p * nt + idx];
-    reinit_tile_step<S>(Din, Dout, phi, frozen, ch_in, ch_out, flags + (size_t)p * nt,
+    reinit_tile_step<S>(Din, Dout, frozen, ch_in, ch_out, flags + (size_t)p * nt,
                         flags + (size_t)(p ^ 1) * nt, list + (size_t)(p ^ 1) * nt,
                         cnt + (k + 1) % 3, 0u, more != 0, nr, nz, dx, t / ntc, t % ntc, nsw, L);
   }
@@ -404,7 +401,7 @@ __device__ __forceinline__ void reinit_final_at(const double* __restrict__ phi,
     tiles[(size_t)nt + t] = 0u;
   }
   const int64_t c = (int64_t)i * nz + j;
-  const double d = frozen[c] ? dist[c] : D[c];
+  const double d = (frozen[c] & 1) ? dist[c] : D[c];
   const bool m = !(fabs(d) <= narrow);
   out[c] = m ? phi[c] : d;
   if (masked) masked[c] = m ? 1 : 0;
@@ -453,11 +450,11 @@ __global__ void soft_batch_reinit_first_list_kernel(const SoftCaseT<B>* __restri
   list_append(take, idx, reinterpret_cast<int*>(list), cnt);
 }
 
-template <typename B>
-__global__ void __launch_bounds__(256) soft_batch_reinit_list_kernel(
+template <typename B, class Shape>
+__global__ void __launch_bounds__(Shape::threads) soft_batch_reinit_list_kernel(
     const SoftCaseT<B>* __restrict__ cs, const uint32_t* __restrict__ tiles, int ntab,
     unsigned* __restrict__ list, unsigned* __restrict__ cnt, int k) {
-  constexpr int S = kReinitSweepsPerLaunch;
+  constexpr int S = Shape::S;
   __shared__ ReinitTile<S> L;
   const int p = k & 1;
   if (blockIdx.x == 0 && threadIdx.x == 0) cnt[(k + 2) % 3] = 0u;
@@ -471,7 +468,7 @@ __global__ void __launch_bounds__(256) soft_batch_reinit_list_kernel(
     const int tr = int((v >> 10) & 8191u), tc = int(v >> 23);
     const int nt = reinit_tile_count(C.nr, C.nz);
     const bool odd = p;
-    reinit_tile_step<S>(odd ? C.rw.d1 : C.rw.d0, odd ? C.rw.d0 : C.rw.d1, C.phi, C.rw.frozen,
+    reinit_tile_step<S>(odd ? C.rw.d1 : C.rw.d0, odd ? C.rw.d0 : C.rw.d1, C.rw.frozen,
                         odd ? C.rw.ch1 : C.rw.ch0, odd ? C.rw.ch0 : C.rw.ch1,
                         C.rw.tiles + (size_t)p * nt, C.rw.tiles + (size_t)(p ^ 1) * nt,
                         list + (size_t)(p ^ 1) * ntab, cnt + (k + 1) % 3,
@@ -482,11 +479,10 @@ __global__ void __launch_bounds__(256) soft_batch_reinit_list_kernel(
 
 template <typename B>
 __global__ void soft_batch_reinit_final_kernel(const SoftCaseT<B>* __restrict__ cs,
-                                               const uint32_t* __restrict__ blocks) {
+                                               const uint32_t* __restrict__ blocks, int S) {
   const SoftBlock b = soft_block(blocks);
   const SoftCaseT<B>& C = cs[b.c];
   if (b.j >= C.nz) return;
-  constexpr int S = kReinitSweepsPerLaunch;
   const int launches = (C.reinit_iterations + S - 1) / S;
   const double* D = (launches & 1) ? C.rw.d1 : C.rw.d0;
   reinit_final_at(C.phi, D, C.rw.dist, C.rw.frozen, C.rw.tiles, C.phi, nullptr, C.nr, C.nz, b.i,
@@ -512,13 +508,18 @@ hipError_t launch_soft_batch_reinit(const SoftCaseT<B>* cases, const SoftBatchDi
       cases, d.reinit_tiles, d.nreinit_tiles, d.reinit_list, d.reinit_cnt);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   const int grid = reinit_list_grid(d.nreinit_tiles);
-  for (int k = 0; k * kReinitSweepsPerLaunch < iterations; ++k) {
-    soft_batch_reinit_list_kernel<B><<<grid, 256, 0, s>>>(cases, d.reinit_tiles, d.nreinit_tiles,
-                                                       d.reinit_list, d.reinit_cnt, k);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
-  soft_batch_reinit_final_kernel<B><<<g, 256, 0, s>>>(cases, d.cell_blocks);
-  return hipGetLastError();
+  const auto sweeps = [&](auto shape) {
+    using Shape = decltype(shape);
+    for (int k = 0; k * Shape::S < iterations; ++k) {
+      soft_batch_reinit_list_kernel<B, Shape><<<grid, Shape::threads, 0, s>>>(
+          cases, d.reinit_tiles, d.nreinit_tiles, d.reinit_list, d.reinit_cnt, k);
+      const hipError_t le = hipGetLastError();
+      if (le != hipSuccess) return le;
+    }
+    soft_batch_reinit_final_kernel<B><<<g, 256, 0, s>>>(cases, d.cell_blocks, Shape::S);
+    return hipGetLastError();
+  };
+  return d.nreinit_tiles <= kReinitFewTiles ? sweeps(ReinitFew{}) : sweeps(ReinitMany{});
 }
 
 template hipError_t launch_soft_batch_reinit<double>(const SoftCaseT<double>*,
@@ -538,22 +539,25 @@ hipError_t launch_reinit(const double* phi, double* out, uint8_t* masked, int nr
   if ((e = hipGetLastError()) != hipSuccess) return e;
   double* a = w.d0;
   double* b = w.d1;
-  constexpr int S = kReinitSweepsPerLaunch;
   uint8_t* ca = w.ch0;
   uint8_t* cb = w.ch1;
   const int lg = reinit_list_grid(nt);
-  for (int q = 0, k = 0; q < iterations; q += S, ++k) {
-    reinit_list_kernel<S><<<lg, 256, 0, s>>>(a, b, phi, w.frozen, ca, cb, w.tiles, w.list, w.cnt,
-                                             nr, nz, dx, k, std::min(S, iterations - q),
-                                             q + S < iterations ? 1 : 0);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    double* t = a;
-    a = b;
-    b = t;
-    uint8_t* tc = ca;
-    ca = cb;
-    cb = tc;
-  }
+  const auto sweeps = [&](auto shape) {
+    using Shape = decltype(shape);
+    constexpr int S = Shape::S;
+    for (int q = 0, k = 0; q < iterations; q += S, ++k) {
+      reinit_list_kernel<Shape><<<lg, Shape::threads, 0, s>>>(
+          a, b, w.frozen, ca, cb, w.tiles, w.list, w.cnt, nr, nz, dx, k,
+          std::min(S, iterations - q), q + S < iterations ? 1 : 0);
+      const hipError_t le = hipGetLastError();
+      if (le != hipSuccess) return le;
+      std::swap(a, b);
+      std::swap(ca, cb);
+    }
+    return hipSuccess;
+  };
+  e = nt <= kReinitFewTiles ? sweeps(ReinitFew{}) : sweeps(ReinitMany{});
+  if (e != hipSuccess) return e;
   reinit_final_kernel<<<grid, 256, 0, s>>>(phi, a, w, out, masked, nr, nz, narrow);
   return hipGetLastError();
 }

@@ -11,7 +11,7 @@ struct ReinitWork {
   double* d0;       // distance iterate (ping)
   double* d1;       // distance iterate (pong)
   double* dist;     // interface distances of the frozen cells
-  uint8_t* frozen;  // 1 on interface cells
+  uint8_t* frozen;  // bit 0: interface cell, bit 1: negative side
   uint8_t* ch0;     // 1 where the last sweep changed the cell (ping)
   uint8_t* ch1;     // (pong)
   // sweep work lists over the 8 x 32 tiles (T = reinit_tile_total):
