@@ -2,13 +2,12 @@
 // transforms for grids whose nz the half-length register and Stockham
 // transforms do not cover (odd nz, or nz / 2 with a prime factor above 5).
 //
-// N that factors into 2, 3 and 5: one Stockham FFT of length N (fft_lds).
+// N that factors into primes up to 13: one Stockham FFT of length N (fft_lds).
 // Otherwise Bluestein's chirp-z form (L. Bluestein, "A linear filtering
 // approach to the computation of discrete Fourier transform", IEEE Trans.
 // Audio Electroacoust. 18(4), 1970): with w_n = e^{-i pi n^2 / N},
 //   X_k = sum_n v_n e^{-2 pi i n k / N} = w_k sum_n (v_n w_n) conj(w_{k-n}),
-// a circular convolution of length L >= 2N - 1 (the smallest 2,3,5-smooth
-// such L) computed by two length-L FFTs and a pointwise product with
+// a circular convolution of 2,3,5-smooth length L >= 2N - 1, computed by two length-L FFTs and a pointwise product with
 // bhat = FFT_L(b) / L, b_m = conj(w_m) for |m| < N (m taken mod L), which
 // the plan computes once on the device.  The chirp angle is reduced as
 // pi (n^2 mod 2N) / N on the host so that it stays exact for large n.  The
@@ -38,7 +37,8 @@ struct AnyDftArgs {
 // Host owner of one length's device tables.
 struct AnyDft {
   AnyDftArgs args{};
-  // the length-L FFT's launch shape: nth threads, PER butterflies each
+  // the length-L FFT's launch shape: nth threads, PER of fft_lds (plus
+  // kFftWide)
   int nth = 64, per = 1;
   std::vector<void*> owned;  // device tables
   hipError_t init(int N);
@@ -47,13 +47,32 @@ struct AnyDft {
   ~AnyDft();
 };
 
-// Butterflies of the plan's widest Stockham stage: L / (its smallest radix).
-// A workgroup of nth threads with PER butterflies each covers the length-L
-// FFT only if PER * nth reaches this.
-inline int widest_stage(const AnyDftArgs& a) {
-  int rmin = a.L > 1 ? a.L : 2;
-  for (int s = 0; s < a.fp.nstages; ++s) rmin = a.fp.radix[s] < rmin ? a.fp.radix[s] : rmin;
-  return a.L / rmin;
+// Radices 7, 8, 11 and 13 are kept out of the kernels of plans without them:
+// with them a row's kernel takes 112-128 registers instead of 48-74 at
+// PER <= 2, which halves the waves in flight (the implicit step at 1024 x 512,
+// chirp-z rows of 1025: 92 us with them, 70 without).
+constexpr int kFftWide = 8;
+inline bool fft_wide(const AnyDftArgs& a) {
+  for (int s = 0; s < a.fp.nstages; ++s)
+    if (a.fp.radix[s] > 5) return true;
+  return false;
+}
+// The fewest threads (a multiple of 64) that cover every stage of the
+// length-L FFT with PER = per, and the least PER with which nth threads do
+// (0: none).
+inline int fft_threads(const AnyDftArgs& a, int per, bool wide) {
+  int nth = 64;
+  for (int s = 0; s < a.fp.nstages; ++s) {
+    const int R = a.fp.radix[s], share = fft_share(R, per, wide);
+    const int need = (a.L / R + share - 1) / share;
+    nth = nth > need ? nth : (need + 63) / 64 * 64;
+  }
+  return nth;
+}
+inline int fft_per(const AnyDftArgs& a, int nth, bool wide) {
+  for (int per : {1, 2, 4})
+    if (nth >= fft_threads(a, per, wide)) return per;
+  return 0;
 }
 
 // Largest L one workgroup can hold in LDS (FP64: 8192 x 16 B = 128 KiB of
@@ -74,9 +93,9 @@ template <typename T, int PER>
 __device__ __forceinline__ void any_fft(Cplx<T>* work, const AnyDftArgs& a, int sgn, int tid,
                                         int nth) {
   if (a.stage)
-    fft_lds<T, PER>(work, a.fp, static_cast<const Cplx<T>*>(work + a.L), sgn, tid, nth);
+    fft_lds<T, PER & 7, (PER & kFftWide) != 0>(work, a.fp, static_cast<const Cplx<T>*>(work + a.L), sgn, tid, nth);
   else
-    fft_lds<T, PER>(work, a.fp, a.tw, sgn, tid, nth);
+    fft_lds<T, PER & 7, (PER & kFftWide) != 0>(work, a.fp, a.tw, sgn, tid, nth);
 }
 
 // In-place DFT of work[0..N) (exponent sign sgn), result in work[0..N),

@@ -2,7 +2,7 @@
 // Stokes and potential plans, the real DFT pair of the periodic-z plans, and
 // the DST-I of the implicit diffusion plan, each one row per workgroup with
 // the row's DFT in LDS (axs_anydft.hpp: Stockham when the length factors
-// into 2, 3 and 5, Bluestein's chirp-z form otherwise).  The grids of the
+// into primes up to 13, Bluestein's chirp-z form otherwise).  The grids of the
 // drivers (nz = 256 .. 4096, nz / 2 a power of two) keep the faster
 // half-length transforms of axs_stokes.hip; these cover every other nz the
 // reference's dense eig route accepts (kernels/FastDiagonalisationStokesSolver.py:41-128,
@@ -39,29 +39,47 @@ namespace axs {
 
 // ------------------------------------------------------------------ plan
 
-static bool radices_of(int M, FftPlanArgs* p) {
+// Radices of an M-point FFT: fours, a two, threes and fives; for M with a
+// factor 7, 11 or 13 (primes = 13 allows them) the power of two in the fewest
+// stages (two fours, not an eight and a two).
+static bool radices_of(int M, int primes, FftPlanArgs* p) {
   p->M = M;
   p->nstages = 0;
   int m = M;
-  for (int r : {4, 2, 3, 5}) {
-    while (m % r == 0) {
-      if (p->nstages >= kMaxFftStages) return false;
+  const auto stages = [&](int r, int most) {
+    for (int i = 0; i < most && m % r == 0 && p->nstages < kMaxFftStages; ++i) {
       p->radix[p->nstages++] = r;
       m /= r;
     }
+  };
+  if (primes > 5 && (M % 7 == 0 || M % 11 == 0 || M % 13 == 0)) {
+    const int e2 = __builtin_ctz(M), rest = e2 % 3;
+    stages(4, rest == 2 ? 1 : (rest == 1 && e2 > 1 ? 2 : 0));
+    stages(8, kMaxFftStages);
   }
+  for (int r : {4, 2, 3, 5, 7, 11, 13})
+    if (r <= primes) stages(r, kMaxFftStages);
   return m == 1;
 }
 
+// The chirp-z length is the smallest smooth one without a lone radix 2 (that
+// stage has the most butterflies and does the least), unless that is more
+// than 1 / 16 longer than the smallest of all: 4500 points instead of 4320 for
+// N = 2049, 284 -> 202 us per implicit step at 2048 x 1024; 1125 instead of
+// 1080 for 513, 33 -> 31 us at 512 x 256.  Factors 7, 11 and 13 are radices of
+// their own where the chirp-z form would do too (rows of 770, 385 = 5 x 7 x 11
+// points instead of two FFTs of 800: 68.6 -> 62.3 us per step of 770 x 386;
+// 113 -> 72 us at 1001 x 500); the longest rows stay those it holds.
 int any_dft_length(int N, bool* bluestein) {
   FftPlanArgs p;
-  if (radices_of(N, &p)) {
-    if (bluestein) *bluestein = false;
-    return N;
-  }
-  if (bluestein) *bluestein = true;
+  if (bluestein) *bluestein = false;
+  if (radices_of(N, 5, &p)) return N;
   int L = 2 * N - 1;
-  while (!radices_of(L, &p)) ++L;
+  while (!radices_of(L, 5, &p)) ++L;
+  if (L <= kAnyMaxL && radices_of(N, 13, &p)) return N;
+  if (bluestein) *bluestein = true;
+  for (int l = L; l <= std::min(L + L / 16, kAnyMaxL); ++l)
+    if (radices_of(l, 5, &p) && __builtin_ctz(l) % 2 == 0) return l;
   return L;
 }
 
@@ -103,20 +121,33 @@ hipError_t AnyDft::init(int N) {
   // staged only while the doubled footprint still lets two workgroups share
   // a CU (longer rows lose more to occupancy than the LDS twiddles save)
   args.stage = 2 * sizeof(Cplx<double>) * (size_t)L <= 65536 ? 1 : 0;
-  radices_of(L, &args.fp);
-  nth = std::min(1024, std::max(64, ((L / 2 + 63) / 64) * 64));
-  if (nth == 1024) {
-    // long rows: the threads of the rows the LDS holds on one CU fill it
-    // (2048 threads per CU); 1024 per row would leave room for two rows
-    // where the LDS holds four (L = 2160, the 1024-point DST-I's chirp-z:
-    // 90 -> 77 us per implicit step at 1024 x 512)
+  radices_of(L, 13, &args.fp);
+  const bool wide = fft_wide(args);
+  nth = std::max(64, (L / (wide ? 4 : 2) + 63) / 64 * 64);
+  if (nth >= 1024) {
+    // long rows: the butterflies per thread that keep the most rows in flight
+    // on a CU (its 160 KiB of LDS; the threads that the registers of PER = 1,
+    // 2, 4 and of the wide radices allow), the fewest where that is equal
+    // (1351 x 680, FFTs of 2880 points: 264 -> 188 us per step with 512
+    // threads, three rows on a CU, instead of 640; stokes 1501 x 700:
+    // 182 -> 116 us)
     const size_t lds = sizeof(Cplx<double>) * (size_t)L * (args.stage ? 2 : 1);
-    const int rows = std::max(1, (int)((size_t)160 * 1024 / lds));
-    nth = std::max(64, std::min(1024, (2048 / rows) / 64 * 64));
+    const int in_lds = (int)((size_t)160 * 1024 / lds);
+    int most = 0;
+    for (int p : {1, 2, 4}) {
+      const int t = fft_threads(args, p, wide);
+      const int threads = wide || p == 4 ? 1024 : p == 2 ? 1536 : 2048;
+      const int rows = std::min(in_lds, threads / t);
+      if (t <= 1024 && rows > most) {
+        most = rows;
+        nth = std::min(1024, threads / rows / 64 * 64);
+      }
+    }
+    if (!most) return hipErrorInvalidValue;
   }
-  per = (L / 2 + nth - 1) / nth;
-  if (per > 4) return hipErrorInvalidValue;
-  per = per <= 1 ? 1 : (per <= 2 ? 2 : 4);
+  nth = std::max(nth, fft_threads(args, 4, wide));
+  per = fft_per(args, nth, wide);
+  if (wide) per |= kFftWide;
   std::vector<Cplx<double>> tw(L);
   for (int t = 0; t < L; ++t) {
     const double ang = -2.0 * M_PI * (double)t / (double)L;
@@ -147,6 +178,7 @@ hipError_t AnyDft::init(int N) {
   if ((e = upload_table(&d_bhat, b)) != hipSuccess) return e;
   owned.push_back(d_bhat);
   const size_t shm = lds_bytes<double>();
+  // chirp-z lengths hold radices up to 5 only
   if (per == 1)
     any_bhat_kernel<1><<<1, nth, shm, 0>>>(d_bhat, args);
   else if (per == 2)
@@ -439,41 +471,22 @@ static void allow_large_lds() {
       (void)hipGetLastError();
       return;
     }
-    const void* ks[] = {
-        (const void*)any_bhat_kernel<1>, (const void*)any_bhat_kernel<2>,
-        (const void*)any_bhat_kernel<4>,
-        (const void*)any_dct2_rows_kernel<double, 1, false>,
-        (const void*)any_dct2_rows_kernel<double, 2, false>,
-        (const void*)any_dct2_rows_kernel<double, 4, false>,
-        (const void*)any_dct2_rows_kernel<double, 1, true>,
-        (const void*)any_dct2_rows_kernel<double, 2, true>,
-        (const void*)any_dct2_rows_kernel<double, 4, true>,
-        (const void*)any_dct2_rows_kernel<float, 1, false>,
-        (const void*)any_dct2_rows_kernel<float, 2, false>,
-        (const void*)any_dct2_rows_kernel<float, 4, false>,
-        (const void*)any_dct2_rows_kernel<float, 1, true>,
-        (const void*)any_dct2_rows_kernel<float, 2, true>,
-        (const void*)any_dct2_rows_kernel<float, 4, true>,
-        (const void*)any_dct3_rows_kernel<double, 1>, (const void*)any_dct3_rows_kernel<double, 2>,
-        (const void*)any_dct3_rows_kernel<double, 4>, (const void*)any_dct3_rows_kernel<float, 1>,
-        (const void*)any_dct3_rows_kernel<float, 2>, (const void*)any_dct3_rows_kernel<float, 4>,
-        (const void*)any_rfft_rows_kernel<1>, (const void*)any_rfft_rows_kernel<2>,
-        (const void*)any_rfft_rows_kernel<4>, (const void*)any_irfft_rows_kernel<1>,
-        (const void*)any_irfft_rows_kernel<2>, (const void*)any_irfft_rows_kernel<4>,
-        (const void*)any_dst1_rows_kernel<1>, (const void*)any_dst1_rows_kernel<2>,
-        (const void*)any_dst1_rows_kernel<4>,
-        (const void*)soft_batch_dct2_kernel<double, 1>,
-        (const void*)soft_batch_dct2_kernel<double, 2>,
-        (const void*)soft_batch_dct2_kernel<double, 4>,
-        (const void*)soft_batch_dct3_kernel<double, 1>,
-        (const void*)soft_batch_dct3_kernel<double, 2>,
-        (const void*)soft_batch_dct3_kernel<double, 4>,
-        (const void*)soft_batch_dct2_kernel<float, 1>,
-        (const void*)soft_batch_dct2_kernel<float, 2>,
-        (const void*)soft_batch_dct2_kernel<float, 4>,
-        (const void*)soft_batch_dct3_kernel<float, 1>,
-        (const void*)soft_batch_dct3_kernel<float, 2>,
-        (const void*)soft_batch_dct3_kernel<float, 4>};
+#define AXS_ANY_KERNELS(P)                                                                       \
+  (const void*)any_dct2_rows_kernel<double, P, false>,                                           \
+      (const void*)any_dct2_rows_kernel<double, P, true>,                                        \
+      (const void*)any_dct2_rows_kernel<float, P, false>,                                        \
+      (const void*)any_dct2_rows_kernel<float, P, true>,                                         \
+      (const void*)any_dct3_rows_kernel<double, P>, (const void*)any_dct3_rows_kernel<float, P>, \
+      (const void*)any_rfft_rows_kernel<P>, (const void*)any_irfft_rows_kernel<P>,               \
+      (const void*)any_dst1_rows_kernel<P>, (const void*)soft_batch_dct2_kernel<double, P>,      \
+      (const void*)soft_batch_dct3_kernel<double, P>,                                            \
+      (const void*)soft_batch_dct2_kernel<float, P>, (const void*)soft_batch_dct3_kernel<float, P>
+    const void* ks[] = {(const void*)any_bhat_kernel<1>,  (const void*)any_bhat_kernel<2>,
+                        (const void*)any_bhat_kernel<4>,  AXS_ANY_KERNELS(1),
+                        AXS_ANY_KERNELS(2),               AXS_ANY_KERNELS(4),
+                        AXS_ANY_KERNELS(1 | kFftWide),    AXS_ANY_KERNELS(2 | kFftWide),
+                        AXS_ANY_KERNELS(4 | kFftWide)};
+#undef AXS_ANY_KERNELS
     int limit = optin;
     for (const void* k : ks) {
       hipFuncAttributes fa{};
@@ -493,18 +506,24 @@ static void allow_large_lds() {
 
 // ------------------------------------------------------------------ launchers
 
-#define AXS_ANY_PER(PERV, CALL) \
-  do {                       \
-    if ((PERV) == 1) {       \
-      constexpr int P = 1;   \
-      CALL;                  \
-    } else if ((PERV) == 2) { \
-      constexpr int P = 2;   \
-      CALL;                  \
-    } else {                 \
-      constexpr int P = 4;   \
-      CALL;                  \
-    }                        \
+#define AXS_ANY_P(V, CALL) \
+  case V: {                \
+    constexpr int P = V;   \
+    CALL;                  \
+    break;                 \
+  }
+#define AXS_ANY_PER(PERV, CALL)      \
+  do {                               \
+    switch (PERV) {                  \
+      AXS_ANY_P(1, CALL)             \
+      AXS_ANY_P(2, CALL)             \
+      AXS_ANY_P(4, CALL)             \
+      AXS_ANY_P((1 | kFftWide), CALL) \
+      AXS_ANY_P((2 | kFftWide), CALL) \
+      AXS_ANY_P((4 | kFftWide), CALL) \
+      default:                       \
+        return hipErrorInvalidValue; \
+    }                                \
   } while (0)
 
 template <typename T>
@@ -584,6 +603,7 @@ template hipError_t launch_soft_batch_dct3<float>(const SoftCaseT<float>*, const
                                                   hipStream_t);
 
 #undef AXS_ANY_PER
+#undef AXS_ANY_P
 
 template hipError_t launch_any_dct2_rows<double>(const StokesPlan&, const double*, double*,
                                                  double*, const double*, const double*,

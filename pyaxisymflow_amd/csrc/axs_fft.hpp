@@ -1,4 +1,5 @@
-// In-LDS complex FFT (Stockham auto-sort, radices 4/2/3/5) and the real
+// In-LDS complex FFT (Stockham auto-sort; radices 4/2/3/5, and 8/7/11/13 for
+// the lengths of axs_anydft.hpp) and the real
 // DCT-II / DCT-III row transforms built on it.
 //
 // DCT-II of a real row x[0..N) (N even), X_k = sum_n x_n cos(pi k (2n+1) / (2N)):
@@ -11,6 +12,8 @@
 #pragma once
 
 #include "axs_common.hpp"
+
+#include <type_traits>
 
 namespace axs {
 
@@ -38,6 +41,66 @@ __device__ __forceinline__ Cplx<T> csub(Cplx<T> a, Cplx<T> b) { return {a.x - b.
 template <typename T>
 __device__ __forceinline__ Cplx<T> cconj(Cplx<T> a) { return {a.x, -a.y}; }
 
+// cos and sin of 2 pi k / P, k = 1 .. (P - 1) / 2
+template <int P>
+struct PrimeTurns;
+template <>
+struct PrimeTurns<7> {
+  static constexpr double c[3] = {0.62348980185873353053, -0.22252093395631440429,
+                                  -0.90096886790241912624};
+  static constexpr double s[3] = {0.78183148246802980871, 0.97492791218182360702,
+                                  0.43388373911755812048};
+};
+template <>
+struct PrimeTurns<11> {
+  static constexpr double c[5] = {0.84125353283118116886, 0.41541501300188642553,
+                                  -0.14231483827328514044, -0.65486073394528506406,
+                                  -0.95949297361449738989};
+  static constexpr double s[5] = {0.54064081745559758211, 0.90963199535451837141,
+                                  0.98982144188093273238, 0.75574957435425828377,
+                                  0.28173255684142969771};
+};
+template <>
+struct PrimeTurns<13> {
+  static constexpr double c[6] = {0.88545602565320989590, 0.56806474673115580251,
+                                  0.12053668025532305335, -0.35460488704253562597,
+                                  -0.74851074817110109863, -0.97094181742605202716};
+  static constexpr double s[6] = {0.46472317204376854566, 0.82298386589365639458,
+                                  0.99270887409805399280, 0.93501624268541482344,
+                                  0.66312265824079520238, 0.23931566428755776715};
+};
+
+// DFT of P points, P an odd prime, from the sums and differences of the
+// pairs a_j, a_{P-j}.
+template <typename T, int P>
+__device__ __forceinline__ void dft_prime(Cplx<T>* a, int sgn) {
+  constexpr int H = (P - 1) / 2;
+  Cplx<T> s[H], d[H];
+  Cplx<T> x0 = a[0];
+#pragma unroll
+  for (int j = 0; j < H; ++j) {
+    s[j] = cadd(a[j + 1], a[P - 1 - j]);
+    const Cplx<T> t = csub(a[j + 1], a[P - 1 - j]);
+    d[j] = {T(sgn) * t.x, T(sgn) * t.y};
+    x0 = cadd(x0, s[j]);
+  }
+#pragma unroll
+  for (int k = 1; k <= H; ++k) {
+    Cplx<T> m = a[0], n = {T(0), T(0)};
+#pragma unroll
+    for (int j = 1; j <= H; ++j) {
+      const int t = j * k % P, u = t <= H ? t : P - t;
+      const T c = T(PrimeTurns<P>::c[u - 1]);
+      const T w = t <= H ? T(PrimeTurns<P>::s[u - 1]) : T(-PrimeTurns<P>::s[u - 1]);
+      m = {m.x + c * s[j - 1].x, m.y + c * s[j - 1].y};
+      n = {n.x + w * d[j - 1].x, n.y + w * d[j - 1].y};
+    }
+    a[k] = {m.x - n.y, m.y + n.x};
+    a[P - k] = {m.x + n.y, m.y - n.x};
+  }
+  a[0] = x0;
+}
+
 // In-place DFT of size R on a[0..R), exponent sign `sgn` (-1 forward).
 template <typename T, int R>
 __device__ __forceinline__ void dft_small(Cplx<T>* a, int sgn) {
@@ -62,6 +125,22 @@ __device__ __forceinline__ void dft_small(Cplx<T>* a, int sgn) {
     a[0] = cadd(a[0], t);
     a[1] = cadd(m, jd);
     a[2] = csub(m, jd);
+  } else if constexpr (R == 8) {  // DFT-4s of the even and odd samples
+    constexpr double h = 0.70710678118654752440;
+    Cplx<T> e[4] = {a[0], a[2], a[4], a[6]}, o[4] = {a[1], a[3], a[5], a[7]};
+    dft_small<T, 4>(e, sgn);
+    dft_small<T, 4>(o, sgn);
+    const T g = T(sgn);
+    o[1] = {T(h) * (o[1].x - g * o[1].y), T(h) * (o[1].y + g * o[1].x)};
+    o[2] = {-g * o[2].y, g * o[2].x};
+    o[3] = {-T(h) * (o[3].x + g * o[3].y), T(h) * (g * o[3].x - o[3].y)};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      a[k] = cadd(e[k], o[k]);
+      a[k + 4] = csub(e[k], o[k]);
+    }
+  } else if constexpr (R == 7 || R == 11 || R == 13) {
+    dft_prime<T, R>(a, sgn);
   } else {  // R == 5: direct
     const T c1 = T(0.30901699437494742410), c2 = T(-0.80901699437494742410);
     const T s1 = T(0.95105651629515357212) * T(sgn), s2 = T(0.58778525229247312917) * T(sgn);
@@ -169,16 +248,38 @@ __device__ __forceinline__ void stockham_stage(Cplx<T>* buf, int M, int Ns, cons
   __syncthreads();
 }
 
+// Butterflies of radix R a thread takes in a stage of fft_lds: PER, or, WIDE,
+// as many as make about 2 PER points.
+__host__ __device__ constexpr int fft_share(int R, int PER, bool WIDE) {
+  return WIDE ? (2 * PER + R - 1) / R : PER;
+}
+
 // Full FFT of length p.M in LDS by nth threads (this one: tid), twiddles tw
-// as for stockham_stage.  Requires p.M / min(radix) <= PER * nth.  Every
-// thread of the block must call it (stages end in block barriers).
-template <typename T, int PER, typename W>
+// as for stockham_stage.  Requires p.M / R <= fft_share(R) * nth for every
+// radix; only WIDE plans hold radices 7, 8, 11 and 13.  Every thread of the
+// block must call it (stages end in block barriers).
+template <typename T, int PER, bool WIDE = false, typename W>
 __device__ void fft_lds(Cplx<T>* buf, const FftPlanArgs& p, const W* tw, int sgn, int tid,
                         int nth) {
   int Ns = 1;
   for (int s = 0; s < p.nstages; ++s) {
     const int R = p.radix[s];
-    if (R == 4)
+    if constexpr (WIDE) {
+      auto stage = [&](auto r) {
+        constexpr int RR = decltype(r)::value;
+        stockham_stage<T, RR, fft_share(RR, PER, true), W>(buf, p.M, Ns, tw, sgn, tid, nth);
+      };
+      switch (R) {
+        case 2: stage(std::integral_constant<int, 2>()); break;
+        case 3: stage(std::integral_constant<int, 3>()); break;
+        case 4: stage(std::integral_constant<int, 4>()); break;
+        case 5: stage(std::integral_constant<int, 5>()); break;
+        case 7: stage(std::integral_constant<int, 7>()); break;
+        case 8: stage(std::integral_constant<int, 8>()); break;
+        case 11: stage(std::integral_constant<int, 11>()); break;
+        default: stage(std::integral_constant<int, 13>()); break;
+      }
+    } else if (R == 4)
       stockham_stage<T, 4, PER, W>(buf, p.M, Ns, tw, sgn, tid, nth);
     else if (R == 2)
       stockham_stage<T, 2, PER, W>(buf, p.M, Ns, tw, sgn, tid, nth);

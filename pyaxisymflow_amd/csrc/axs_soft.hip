@@ -762,6 +762,19 @@ struct SoftBatchT {
   hipError_t refresh() {
     h_cases.clear();
     dims = SoftBatchDims{};
+    // the row workgroup of every case: the threads its FFT needs with the
+    // most butterflies each; one case with the wide radices brings them in
+    // for all
+    bool wide = false;
+    for (const Entry& c : cases) wide |= fft_wide(c.st->plan->any->args);
+    for (const Entry& c : cases)
+      dims.any_nth = std::max(dims.any_nth, fft_threads(c.st->plan->any->args, 4, wide));
+    for (const Entry& c : cases) {
+      const int per = fft_per(c.st->plan->any->args, dims.any_nth, wide);
+      if (!per || dims.any_nth > 1024) return hipErrorInvalidValue;
+      dims.any_per = std::max(dims.any_per, per);
+    }
+    if (wide) dims.any_per |= kFftWide;
     for (const Entry& c : cases) {
       const SoftStepperT<B>& S = *c.st;
       h_cases.push_back(describe(S, need));
@@ -769,20 +782,9 @@ struct SoftBatchT {
       dims.max_nr = std::max(dims.max_nr, P.nr);
       dims.max_nz = std::max(dims.max_nz, P.nz);
       dims.max_chunks = std::max(dims.max_chunks, (int)ceil_div(P.nz, P.tri_K));
-      // a Stockham stage gives every butterfly its own lane slot in one
-      // pass (at most 4 per thread, no loop): the widest stage, L / (the
-      // smallest radix) butterflies, sets the row workgroup, ~4 per thread
-      const int wide = widest_stage(P.any->args);
-      dims.any_nth =
-          std::max(dims.any_nth, std::min(1024, (int)(ceil_div(ceil_div(wide, 4), 64) * 64)));
       dims.any_lds = std::max(dims.any_lds, P.any->lds_bytes<B>());
       dims.tri_lds =
           std::max(dims.tri_lds, tri_lds_bytes(P.nr, kSoftBatchTriL, P.tri_K, P.tri_P, false));
-    }
-    for (const Entry& c : cases) {
-      const int per = (int)ceil_div(widest_stage(c.st->plan->any->args), dims.any_nth);
-      if (per > 4) return hipErrorInvalidValue;  // a stage would leave butterflies out
-      dims.any_per = std::max(dims.any_per, per <= 1 ? 1 : (per <= 2 ? 2 : 4));
     }
     dims.ncase = (int)cases.size();
     // block tables: every 256-cell row segment of every case, over its grid
