@@ -41,7 +41,8 @@ struct AnyDft {
   // kFftWide)
   int nth = 64, per = 1;
   std::vector<void*> owned;  // device tables
-  hipError_t init(int N);
+  // primes: 13, or 5 for a batch's rows (any_dft_length)
+  hipError_t init(int N, int primes = 13);
   template <typename T>
   size_t lds_bytes() const { return sizeof(Cplx<T>) * (size_t)args.L * (args.stage ? 2 : 1); }
   ~AnyDft();
@@ -78,8 +79,9 @@ inline int fft_per(const AnyDftArgs& a, int nth, bool wide) {
 // Largest L one workgroup can hold in LDS (FP64: 8192 x 16 B = 128 KiB of
 // the CU's 160 KiB); every length N with L <= kAnyMaxL is supported.
 constexpr int kAnyMaxL = 8192;
-// FFT length the chirp-z form needs for N (N itself when N is 2,3,5-smooth).
-int any_dft_length(int N, bool* bluestein);
+// FFT length of an N-point DFT: N itself when its prime factors are at most
+// `primes`, else what the chirp-z form takes.
+int any_dft_length(int N, bool* bluestein, int primes = 13);
 
 // Copies the FFT twiddles into LDS after the work entries when the plan
 // stages them; call before the barrier that precedes any_dft.

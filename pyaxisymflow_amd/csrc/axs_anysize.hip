@@ -69,15 +69,20 @@ static bool radices_of(int M, int primes, FftPlanArgs* p) {
 // 1080 for 513, 33 -> 31 us at 512 x 256.  Factors 7, 11 and 13 are radices of
 // their own where the chirp-z form would do too (rows of 770, 385 = 5 x 7 x 11
 // points instead of two FFTs of 800: 68.6 -> 62.3 us per step of 770 x 386;
-// 113 -> 72 us at 1001 x 500); the longest rows stay those it holds.
-int any_dft_length(int N, bool* bluestein) {
+// 113 -> 72 us at 1001 x 500); the longest rows stay those it holds.  A
+// batch's rows of many lengths run in one kernel, which the wide radices of
+// one would slow for all, so they keep to primes = 5 and the smallest
+// chirp-z length (twelve FP32 cases: 110 us of rows per step with the wide
+// radices, 119 without, inside the noise of the 960 us step).
+int any_dft_length(int N, bool* bluestein, int primes) {
   FftPlanArgs p;
   if (bluestein) *bluestein = false;
   if (radices_of(N, 5, &p)) return N;
   int L = 2 * N - 1;
   while (!radices_of(L, 5, &p)) ++L;
-  if (L <= kAnyMaxL && radices_of(N, 13, &p)) return N;
+  if (L <= kAnyMaxL && radices_of(N, primes, &p)) return N;
   if (bluestein) *bluestein = true;
+  if (primes == 5) return L;
   for (int l = L; l <= std::min(L + L / 16, kAnyMaxL); ++l)
     if (radices_of(l, 5, &p) && __builtin_ctz(l) % 2 == 0) return l;
   return L;
@@ -109,10 +114,10 @@ static void allow_large_lds();
 // bytes of dynamic LDS every any-kernel may take (raised by allow_large_lds)
 static int g_any_lds_limit = 65536;
 
-hipError_t AnyDft::init(int N) {
+hipError_t AnyDft::init(int N, int primes) {
   allow_large_lds();
   bool blue = false;
-  const int L = any_dft_length(N, &blue);
+  const int L = any_dft_length(N, &blue, primes);
   if (L > kAnyMaxL || sizeof(Cplx<double>) * (size_t)L > (size_t)g_any_lds_limit)
     return hipErrorInvalidValue;
   args.N = N;
@@ -121,7 +126,7 @@ hipError_t AnyDft::init(int N) {
   // staged only while the doubled footprint still lets two workgroups share
   // a CU (longer rows lose more to occupancy than the LDS twiddles save)
   args.stage = 2 * sizeof(Cplx<double>) * (size_t)L <= 65536 ? 1 : 0;
-  radices_of(L, 13, &args.fp);
+  radices_of(L, primes, &args.fp);
   const bool wide = fft_wide(args);
   nth = std::max(64, (L / (wide ? 4 : 2) + 63) / 64 * 64);
   if (nth >= 1024) {
@@ -478,15 +483,18 @@ static void allow_large_lds() {
       (const void*)any_dct2_rows_kernel<float, P, true>,                                         \
       (const void*)any_dct3_rows_kernel<double, P>, (const void*)any_dct3_rows_kernel<float, P>, \
       (const void*)any_rfft_rows_kernel<P>, (const void*)any_irfft_rows_kernel<P>,               \
-      (const void*)any_dst1_rows_kernel<P>, (const void*)soft_batch_dct2_kernel<double, P>,      \
-      (const void*)soft_batch_dct3_kernel<double, P>,                                            \
+      (const void*)any_dst1_rows_kernel<P>
+#define AXS_ANY_BATCH_KERNELS(P)                                                                    \
+  (const void*)soft_batch_dct2_kernel<double, P>, (const void*)soft_batch_dct3_kernel<double, P>, \
       (const void*)soft_batch_dct2_kernel<float, P>, (const void*)soft_batch_dct3_kernel<float, P>
     const void* ks[] = {(const void*)any_bhat_kernel<1>,  (const void*)any_bhat_kernel<2>,
                         (const void*)any_bhat_kernel<4>,  AXS_ANY_KERNELS(1),
                         AXS_ANY_KERNELS(2),               AXS_ANY_KERNELS(4),
                         AXS_ANY_KERNELS(1 | kFftWide),    AXS_ANY_KERNELS(2 | kFftWide),
-                        AXS_ANY_KERNELS(4 | kFftWide)};
+                        AXS_ANY_KERNELS(4 | kFftWide),    AXS_ANY_BATCH_KERNELS(1),
+                        AXS_ANY_BATCH_KERNELS(2),         AXS_ANY_BATCH_KERNELS(4)};
 #undef AXS_ANY_KERNELS
+#undef AXS_ANY_BATCH_KERNELS
     int limit = optin;
     for (const void* k : ks) {
       hipFuncAttributes fa{};
@@ -512,6 +520,16 @@ static void allow_large_lds() {
     CALL;                  \
     break;                 \
   }
+#define AXS_ANY_BATCH_PER(PERV, CALL) \
+  do {                                \
+    switch (PERV) {                   \
+      AXS_ANY_P(1, CALL)              \
+      AXS_ANY_P(2, CALL)              \
+      AXS_ANY_P(4, CALL)              \
+      default:                        \
+        return hipErrorInvalidValue;  \
+    }                                 \
+  } while (0)
 #define AXS_ANY_PER(PERV, CALL)      \
   do {                               \
     switch (PERV) {                  \
@@ -579,8 +597,8 @@ template <typename B>
 hipError_t launch_soft_batch_dct2(const SoftCaseT<B>* cases, const SoftBatchDims& d,
                                   hipStream_t s) {
   const dim3 grid(d.max_nr, d.ncase);
-  AXS_ANY_PER(d.any_per,
-              (soft_batch_dct2_kernel<B, P><<<grid, d.any_nth, d.any_lds, s>>>(cases)));
+  AXS_ANY_BATCH_PER(d.any_per,
+                              (soft_batch_dct2_kernel<B, P><<<grid, d.any_nth, d.any_lds, s>>>(cases)));
   return hipGetLastError();
 }
 
@@ -588,8 +606,8 @@ template <typename B>
 hipError_t launch_soft_batch_dct3(const SoftCaseT<B>* cases, const SoftBatchDims& d,
                                   hipStream_t s) {
   const dim3 grid(d.max_nr, d.ncase);
-  AXS_ANY_PER(d.any_per,
-              (soft_batch_dct3_kernel<B, P><<<grid, d.any_nth, d.any_lds, s>>>(cases)));
+  AXS_ANY_BATCH_PER(d.any_per,
+                              (soft_batch_dct3_kernel<B, P><<<grid, d.any_nth, d.any_lds, s>>>(cases)));
   return hipGetLastError();
 }
 
@@ -603,6 +621,7 @@ template hipError_t launch_soft_batch_dct3<float>(const SoftCaseT<float>*, const
                                                   hipStream_t);
 
 #undef AXS_ANY_PER
+#undef AXS_ANY_BATCH_PER
 #undef AXS_ANY_P
 
 template hipError_t launch_any_dct2_rows<double>(const StokesPlan&, const double*, double*,

@@ -763,18 +763,14 @@ struct SoftBatchT {
     h_cases.clear();
     dims = SoftBatchDims{};
     // the row workgroup of every case: the threads its FFT needs with the
-    // most butterflies each; one case with the wide radices brings them in
-    // for all
-    bool wide = false;
-    for (const Entry& c : cases) wide |= fft_wide(c.st->plan->any->args);
+    // most butterflies each
     for (const Entry& c : cases)
-      dims.any_nth = std::max(dims.any_nth, fft_threads(c.st->plan->any->args, 4, wide));
+      dims.any_nth = std::max(dims.any_nth, fft_threads(c.st->plan->any->args, 4, false));
     for (const Entry& c : cases) {
-      const int per = fft_per(c.st->plan->any->args, dims.any_nth, wide);
+      const int per = fft_per(c.st->plan->any->args, dims.any_nth, false);
       if (!per || dims.any_nth > 1024) return hipErrorInvalidValue;
       dims.any_per = std::max(dims.any_per, per);
     }
-    if (wide) dims.any_per |= kFftWide;
     for (const Entry& c : cases) {
       const SoftStepperT<B>& S = *c.st;
       h_cases.push_back(describe(S, need));

@@ -346,7 +346,7 @@ hipError_t StokesPlan::init_transforms(int nr_, int nz_, double dx_) {
     any_half = bc == 0 && nz % 2 == 0;
     any = new (std::nothrow) AnyDft();
     if (!any) return hipErrorOutOfMemory;
-    if ((e = any->init(any_half ? nz / 2 : nz)) != hipSuccess) return e;
+    if ((e = any->init(any_half ? nz / 2 : nz, force_general ? 5 : 13)) != hipSuccess) return e;
   }
   if (general && !any_half) {
     std::vector<Cplx<double>> h_ge2(nz);

@@ -7,8 +7,8 @@ radix 2.
 Bars (FP64): relative L2 against the exact discrete solutions 1e-12, as for
 the other lengths: a DFT of N <= 8192 points adds at most about
 eps log2(N) = 3e-15 to each of the two row passes, the radial solves are the
-same.  A batch that mixes lengths runs its rows with one case's
-radices and another's threads: the bits of a case stay those it has alone."""
+same.  A batch that mixes lengths runs its rows with the threads of
+the longest: the bits of a case stay those it has alone."""
 import numpy as np
 import pytest
 
@@ -71,8 +71,8 @@ def test_sine_rows(nz):
 
 @pytest.mark.parametrize("precision", ["f64", "f32"])
 def test_batch_rows_keep_a_case_s_bits(precision):
-    """Rows of 64 points (radices up to 5) alone, then beside rows of 182 and
-    of 154 points (radices 7, 11 and 13); and the 154-point case alone."""
+    """Rows of 64 points alone, then beside rows of 182 and of 154 points
+    (chirp-z in a batch); and the 154-point case alone."""
     from pyaxisymflow_amd.stepper import SoftSphereBatch
 
     def bits(c):
