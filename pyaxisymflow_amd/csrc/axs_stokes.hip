@@ -1051,7 +1051,10 @@ __device__ __forceinline__ double recip_nr(double m) {
 // memory (every mode reads the same rows, so they stay in L1/L2) instead of
 // being staged in LDS, which leaves the LDS to the scans and allows more
 // modes per workgroup on tall grids.
-template <typename T, int L, bool FULL, bool CG>
+// PIN: mode 0's last equation is x_{nr-1} = 0 instead (its matrix is singular
+// without): the reciprocal pivot of that row is set to 0, which makes its
+// value and everything carried through it 0.
+template <typename T, int L, bool FULL, bool CG, bool PIN = false>
 __device__ __forceinline__ void tridiag_columns_body(
     T* __restrict__ d, const double* __restrict__ a, const double* __restrict__ b,
     const double* __restrict__ c, const double* __restrict__ lam,
@@ -1111,7 +1114,8 @@ __device__ __forceinline__ void tridiag_columns_body(
     if (FULL || (active && i < nr)) {
       const double ai = ca(i);
       const double m = (cb(i) + lk) - ai * cp;
-      const double inv = recip_nr(m);
+      double inv = recip_nr(m);
+      if constexpr (PIN) inv = (k == 0 && i == nr - 1) ? 0.0 : inv;
       im[l] = inv;
       cp = cc(i) * inv;
       y = (x[l] - ai * y) * inv;
@@ -1212,7 +1216,7 @@ __device__ __forceinline__ void tridiag_columns_body(
     }
   }
 }
-template <typename T, int L, bool FULL, bool CG>
+template <typename T, int L, bool FULL, bool CG, bool PIN>
 __global__ void __launch_bounds__(1024) tridiag_columns_kernel(
     T* __restrict__ d, const double* __restrict__ a, const double* __restrict__ b,
     const double* __restrict__ c, const double* __restrict__ lam,
@@ -1222,8 +1226,8 @@ __global__ void __launch_bounds__(1024) tridiag_columns_kernel(
   const int nb = gridDim.x;
   int chunk = blockIdx.x;
   if (nb % 8 == 0) chunk = (blockIdx.x % 8) * (nb / 8) + blockIdx.x / 8;
-  tridiag_columns_body<T, L, FULL, CG>(d + (int64_t)blockIdx.y * nr * nz, a, b, c, lam, cseg, nr,
-                                       nz, K, P, chunk);
+  tridiag_columns_body<T, L, FULL, CG, PIN>(d + (int64_t)blockIdx.y * nr * nz, a, b, c, lam, cseg,
+                                            nr, nz, K, P, chunk);
 }
 
 // ------------------------------------------------------------ uneven batches
@@ -1476,24 +1480,6 @@ hipError_t launch_rfft_rows(const StokesPlan& pl, const double* src, double* dst
   return hipGetLastError();
 }
 
-// One tridiagonal system of nr rows held contiguously in d (segments of 16
-// rows, one thread each, coefficients read from global memory).
-__global__ void __launch_bounds__(256) tridiag_one_kernel(
-    double* __restrict__ d, const double* __restrict__ a, const double* __restrict__ b,
-    const double* __restrict__ c, const double* __restrict__ lam,
-    const double* __restrict__ cseg, int nr, int P) {
-  tridiag_columns_body<double, 16, false, true>(d, a, b, c, lam, cseg, nr, 1, 1, P, 0);
-}
-
-hipError_t launch_tridiag_one(double* d, const double* a, const double* b, const double* c,
-                              const double* lam, const double* cseg, int nr, hipStream_t s) {
-  const int P = (nr + 15) / 16;
-  if (P > 256) return hipErrorInvalidValue;
-  tridiag_one_kernel<<<1, P, tri_lds_bytes(nr, 16, 1, P, true), s>>>(d, a, b, c, lam, cseg, nr,
-                                                                      P);
-  return hipGetLastError();
-}
-
 template <typename T>
 hipError_t launch_tridiag(const StokesPlan& pl, T* d, hipStream_t s, int batch) {
   const int K = pl.tri_K, P = pl.tri_P;
@@ -1501,9 +1487,21 @@ hipError_t launch_tridiag(const StokesPlan& pl, T* d, hipStream_t s, int batch) 
   const bool full = (pl.nr % pl.tri_L == 0) && (pl.nz % K == 0);
   const bool cg = pl.tri_G;
   const size_t shm = tri_lds_bytes(pl.nr, pl.tri_L, K, P, cg);
-#define AXS_TRI_ONE(LL, F, G)                                                                    \
-  tridiag_columns_kernel<T, LL, F, G><<<blocks, K * P, shm, s>>>(d, pl.a, pl.b, pl.c, pl.lam,    \
-                                                                 pl.cseg, pl.nr, pl.nz, K, P)
+#define AXS_TRI_PIN(LL, F, G, PIN)                                                              \
+  tridiag_columns_kernel<T, LL, F, G, PIN><<<blocks, K * P, shm, s>>>(d, pl.a, pl.b, pl.c,      \
+                                                                      pl.lam, pl.cseg, pl.nr,   \
+                                                                      pl.nz, K, P)
+#define AXS_TRI_ONE(LL, F, G)                                                                   \
+  do {                                                                                          \
+    if constexpr (std::is_same_v<T, double>) {                                                  \
+      if (pl.pin_mode0)                                                                         \
+        AXS_TRI_PIN(LL, F, G, true);                                                            \
+      else                                                                                      \
+        AXS_TRI_PIN(LL, F, G, false);                                                           \
+    } else {                                                                                    \
+      AXS_TRI_PIN(LL, F, G, false);                                                             \
+    }                                                                                           \
+  } while (0)
 #define AXS_TRI(LL)                                                                              \
   do {                                                                                           \
     if (full && cg)                                                                              \
@@ -1531,6 +1529,7 @@ hipError_t launch_tridiag(const StokesPlan& pl, T* d, hipStream_t s, int batch) 
     default:
       return hipErrorInvalidValue;
   }
+#undef AXS_TRI_PIN
 #undef AXS_TRI_ONE
 #undef AXS_TRI
   return hipGetLastError();

@@ -50,6 +50,9 @@ struct StokesPlan {
   // true: the any-length row transforms for every nz (the form a soft batch
   // launches over cases of different lengths)
   bool force_general = false;
+  // mode 0 of the column pass with x_{nr-1} = 0 as its last equation (the
+  // potential's gauge; FP64 fields only)
+  bool pin_mode0 = false;
   // separates the cached column-pass searches of plans whose matrices
   // differ on the same grid (0: Stokes, 1: implicit diffusion)
   int tune_key = 0;
@@ -113,10 +116,6 @@ std::vector<double> pivot_table(const std::vector<double>& a, const std::vector<
 // rfft_rows_kernel), or their inverse.
 hipError_t launch_rfft_rows(const StokesPlan& pl, const double* src, double* dst,
                             const double* rscale, int rows, hipStream_t s, bool inverse);
-// One tridiagonal system a_i x_{i-1} + (b_i + lam[0]) x_i + c_i x_{i+1} = d_i
-// of nr <= 4096 contiguous rows, in place; cseg = pivot_table(..., nz = 1, L = 16).
-hipError_t launch_tridiag_one(double* d, const double* a, const double* b, const double* c,
-                              const double* lam, const double* cseg, int nr, hipStream_t s);
 // Row passes of a general plan (any nz; see StokesPlan::general).
 template <typename T>
 hipError_t launch_any_dct2_rows(const StokesPlan& pl, const T* src, T* tapered, T* dst,
