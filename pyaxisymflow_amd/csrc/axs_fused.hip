@@ -33,6 +33,7 @@
 // bit for bit: same comparison, same products, same sums).
 #include "axs_fused.hpp"
 
+#include <type_traits>
 #include <algorithm>
 
 namespace axs {
@@ -271,13 +272,31 @@ constexpr int kR5Z = kFZ + 10, kR5R = kFR + 10;
 constexpr int kR4Z = kFZ + 8, kR4R = kFR + 8;
 constexpr int kR2Z = kFZ + 4, kR2R = kFR + 4;
 constexpr int kR1Z = kFZ + 2, kR1R = kFR + 2;
-// Thread strips: penalisation 4 x 64 (kVS owned R4 rows + one R5 row above
-// and below), ENO3 rows kEH, stage 1 rows kSH, stage 2 rows kOH.
-constexpr int kVS = 6, kEH = 5, kSH = 6, kOH = 4;
-static_assert(kR5Z == 64 && 4 * kVS == kR4R, "penalisation strips cover R4 rows x R5 columns");
-static_assert(kR2R % kEH == 0 && kR1R % kSH == 0 && kFR % kOH == 0, "strip heights");
-static_assert((kR2R / kEH) * kR2Z <= 256 && (kR1R / kSH) * kR1Z <= 256 && (kFR / kOH) * kFZ <= 256,
-              "one strip per thread");
+// Thread strips of a workgroup of NT: penalisation NT / 64 x 64 (VS owned R4
+// rows + one R5 row above and below), ENO3 rows EH, stage 1 rows SH, stage 2
+// rows OH.
+template <int VS_, int EH_, int SH_, int OH_>
+struct FusedStrips {
+  static constexpr int VS = VS_, EH = EH_, SH = SH_, OH = OH_, NT = kR4R / VS * kR5Z;
+  static_assert(kR5Z == 64 && kR4R % VS == 0, "penalisation strips cover R4 rows x R5 columns");
+  static_assert(kR2R % EH == 0 && kR1R % SH == 0 && kFR % OH == 0, "strip heights");
+  static_assert((kR2R / EH) * kR2Z <= NT && (kR1R / SH) * kR1Z <= NT && (kFR / OH) * kFZ <= NT,
+                "one strip per thread");
+};
+// 256 threads: the least work overall (a strip of h rows evaluates h + 1 of
+// the radial ENO3 faces), four tiles on a CU (FP32: five).
+using FusedFull = FusedStrips<6, 5, 6, 4>;
+// Where all tiles of a launch run at once, a tile's time is its threads'
+// serial work, and shorter strips are faster although they do more of it:
+// 768 threads while every tile has a CU of its own, 512 while its tiles fit
+// on the CUs two (FP32: four) at a time.  us per step, 256 / 512 / 768
+// threads: FP64 256 x 128 (40 tiles) 37.0 / 34.0 / 32.5, 512 x 256 (160) 38.7 /
+// 35.8 / 34.6, 800 x 400 (375) 49.1 / 47.1 / 48.7, 1024 x 512 (608) 45.5 / 46.5 /
+// 49.6; FP32 512 x 256 31.3 / 28.3 / 27.2, 1024 x 512 40.8 / 38.7 / 40.7, 1200 x 600
+// (874) 56.8 / 55.2 / 57.8, 2048 x 1024 (2432) 62.5 / 63.3 / 70.8.
+using FusedSome = FusedStrips<3, 4, 3, 2>;
+using FusedFew = FusedStrips<2, 2, 2, 2>;
+constexpr int kCUs = 256;
 // LDS buffers and what they hold phase by phase.
 constexpr int kBufA = kR6R * kR6Z;  // psi (R6), then f (R4)
 constexpr int kBufC = kR4R * kR4Z;  // u_pen_z (R4), then stage-1 out (R1)
@@ -296,6 +315,7 @@ struct FusedLds {
   T *sri, *sinv, *sinv2;  // per R6 row: r_i, 1 / r_i, 1 / r_i^2
   double* srd;            // per R6 row: r_i (FP64, for the force)
   double* wpart;
+  double* force;  // the tile's force terms (strips other than FusedFull's)
   double* smax;  // slot maximum, then the step's dt, timer and reset flag
 };
 
@@ -306,13 +326,18 @@ struct FusedLds {
 // implicit-diffusion form of the drivers (flow_past_sphere.py:178-181), whose
 // tile output is the ENO3 result (the diffusion solve follows as its own
 // passes).
-template <typename T, bool IN, bool RK2 = true>
+template <typename T, class S, bool IN, bool RK2 = true>
 __device__ __forceinline__ void step_fused_tile(
     const T* __restrict__ psi, const T* __restrict__ chi, const T* __restrict__ wsrc,
     T* __restrict__ wdst, T* __restrict__ avg, const double* __restrict__ r,
     const double* __restrict__ wz, const double* __restrict__ wr, int kw, int nr, int nz, T dx,
     double* __restrict__ sc, const double* __restrict__ slots, double* __restrict__ partials,
     const RigidConfig& cfg, const FusedLds<T>& L, int i0, int j0, int tile) {
+  constexpr int kVS = S::VS, kEH = S::EH, kSH = S::SH, kOH = S::OH, kNT = S::NT;
+  // the force terms are summed in FusedFull's order whatever the strips, so
+  // that a case's force has the same bits alone and in a batch
+  using Full = FusedFull;
+  constexpr bool kStaged = !std::is_same_v<S, Full>;
   T(*sp)[kR6Z] = reinterpret_cast<T(*)[kR6Z]>(L.A);
   T(*sf)[kR4Z] = reinterpret_cast<T(*)[kR4Z]>(L.A);
   T(*sa)[kR2Z] = reinterpret_cast<T(*)[kR2Z]>(L.D);
@@ -323,18 +348,18 @@ __device__ __forceinline__ void step_fused_tile(
   const T* sinv = L.sinv;
   const T* sinv2 = L.sinv2;
   const int tid = threadIdx.x;
-  // penalisation strip of this thread: R5 column pb, R5 rows 6ps .. 6ps+7
+  // penalisation strip of this thread: R5 column pb, R5 rows VS ps .. VS ps + VS + 1
   const int pb = tid & 63, ps = tid >> 6;
   const int pj = j0 - 5 + pb;
   const bool pjin = IN || (pj >= 0 && pj < nz);
 
   // ---- 1. loads: psi tile, chi and stored omega of the strip, slots, rows
-  constexpr int NP = (kBufA + 255) / 256;
+  constexpr int NP = (kBufA + kNT - 1) / kNT;
   T vp[NP];
   const T* ptile = psi + ((i0 - 6) * nz + (j0 - 6));  // interior tiles only
 #pragma unroll
   for (int q = 0; q < NP; ++q) {
-    const int e = tid + q * 256;
+    const int e = tid + q * kNT;
     const int a = e / kR6Z, b = e % kR6Z;
     vp[q] = T(0);
     if constexpr (IN) {
@@ -388,7 +413,7 @@ __device__ __forceinline__ void step_fused_tile(
   }
 #pragma unroll
   for (int q = 0; q < NP; ++q) {
-    const int e = tid + q * 256;
+    const int e = tid + q * kNT;
     if (e < kBufA) L.A[e] = vp[q];
   }
   // Does the body reach this tile's R5 region?  Where chi = 0, Brinkman
@@ -470,7 +495,11 @@ __device__ __forceinline__ void step_fused_tile(
           const T base = (ds.reset != 0.0) ? T(0) : avg[c];
           avg[c] = base + p[0] * tdt;
         }
-        acc += (L.srd[q5 + 1] * double(vc[k])) * (double(pzv) - Ud);
+        const double term = (L.srd[q5 + 1] * double(vc[k])) * (double(pzv) - Ud);
+        if constexpr (kStaged)
+          L.force[(q5 - 5) * kFZ + pb - 5] = term;
+        else
+          acc += term;
       }
     }
     dz[k] = dzv;
@@ -484,6 +513,15 @@ __device__ __forceinline__ void step_fused_tile(
     }
   }
   __syncthreads();
+  if constexpr (kStaged) {
+    if (tid < Full::NT && pb >= 5 && pb < 5 + kFZ && (IN || pj < nz)) {
+#pragma unroll
+      for (int k = 1; k <= Full::VS; ++k) {
+        const int a = Full::VS * ps + k - 5;  // output row
+        if (a >= 0 && a < kFR && (IN || i0 + a < nr)) acc += L.force[a * kFZ + pb - 5];
+      }
+    }
+  }
 
   // ---- 3. f = taper(omega) + curl(u_pen - u) on the strip's R4 cells; the
   //         z neighbours of a strip column are the neighbouring lanes
@@ -521,12 +559,12 @@ __device__ __forceinline__ void step_fused_tile(
   // the tile's force sum leaves the registers before the ENO3 and RK2
   // phases (the same wave reduction the end of the kernel would make)
   acc = wave_sum(acc);
-  if ((tid & 63) == 0) L.wpart[tid >> 6] = acc;
+  if ((tid & 63) == 0 && tid < Full::NT) L.wpart[tid >> 6] = acc;
   if constexpr (!IN) {
     if (i0 == 0) {
       // rows -4..-1 of the ENO3 input are the axis mirror of rows 3..0
       // (f odd, u_z even, u_r odd: advect_vorticity_via_eno3.py:28-33)
-      for (int e = tid; e < 4 * kR4Z; e += 256) {
+      for (int e = tid; e < 4 * kR4Z; e += kNT) {
         const int m = e / kR4Z, c = e % kR4Z;
         sf[3 - m][c] = -sf[4 + m][c];
         sx[3 - m][c] = sx[4 + m][c];
@@ -681,9 +719,13 @@ constexpr int kFusedWaves = 4;
 template <typename T>
 constexpr int kRaggedFusedWaves = sizeof(T) == 8 ? 4 : 7;
 
-// 256 threads, waves and LDS as kFusedWaves says.
-template <typename T, bool RK2>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFusedWaves<T>))) step_fused_kernel(
+// Waves and LDS as kFusedWaves says for 256 threads; with more, what one
+// workgroup (768) or two (512) on a CU need.
+template <class S, typename T>
+constexpr int kFusedTileWaves = S::NT == 768 ? 3 : kFusedWaves<T>;
+template <typename T, class S, bool RK2>
+__global__ void __launch_bounds__(S::NT)
+    __attribute__((amdgpu_waves_per_eu(kFusedTileWaves<S, T>))) step_fused_kernel(
     const T* __restrict__ psi, const T* __restrict__ chi, const T* __restrict__ wsrc,
     T* __restrict__ wdst, T* __restrict__ avg, const double* __restrict__ r,
     const double* __restrict__ wz, const double* __restrict__ wr, int kw, int nr, int nz, T dx,
@@ -693,6 +735,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFused
   __shared__ T sri[kR6R], sinv[kR6R], sinv2[kR6R];
   __shared__ double srd[kR6R];
   __shared__ double wpart[4];
+  __shared__ double force[std::is_same_v<S, FusedFull> ? 1 : kFR * kFZ];
   __shared__ double smax[4];
   const int cb = blockIdx.z;  // case of a batch
   const RigidConfig& cfg = cfgs[cb];
@@ -705,7 +748,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFused
   sc += (int64_t)cb * AXS_RIGID_SCALARS;
   slots += (int64_t)cb * kSlotsPerCase;
   partials += (int64_t)cb * gridDim.x * gridDim.y;
-  const FusedLds<T> L{bufA, bufC, bufD, sri, sinv, sinv2, srd, wpart, smax};
+  const FusedLds<T> L{bufA, bufC, bufD, sri, sinv, sinv2, srd, wpart, force, smax};
   // XCD-aware tile order: workgroups are dealt to the 8 XCDs round-robin by
   // linear id; give each XCD a contiguous band of tiles so a tile's halo
   // rows are still in that XCD's L2 when its neighbours read them.
@@ -719,10 +762,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFused
   const bool interior = i0 - 6 >= m && i0 + kFR + 6 <= nr - m && j0 - 6 >= m &&
                         j0 + kFZ + 6 <= nz - m;
   if (interior)
-    step_fused_tile<T, true, RK2>(psi, chi, wsrc, wdst, avg, r, wz, wr, kw, nr, nz, dx, sc, slots,
+    step_fused_tile<T, S, true, RK2>(psi, chi, wsrc, wdst, avg, r, wz, wr, kw, nr, nz, dx, sc, slots,
                              partials, cfg, L, i0, j0, tile);
   else
-    step_fused_tile<T, false, RK2>(psi, chi, wsrc, wdst, avg, r, wz, wr, kw, nr, nz, dx, sc, slots,
+    step_fused_tile<T, S, false, RK2>(psi, chi, wsrc, wdst, avg, r, wz, wr, kw, nr, nz, dx, sc, slots,
                               partials, cfg, L, i0, j0, tile);
 }
 
@@ -747,19 +790,19 @@ step_fused_ragged_kernel(const T* __restrict__ psi, const T* __restrict__ chi,
   const int cb = G.case0 + cl;
   const int nr = G.nr, nz = G.nz;
   const int64_t fo = G.cell0 + (int64_t)cl * nr * nz;
-  const FusedLds<T> L{bufA, bufC, bufD, sri, sinv, sinv2, srd, wpart, smax};
+  const FusedLds<T> L{bufA, bufC, bufD, sri, sinv, sinv2, srd, wpart, nullptr, smax};
   const int j0 = (tile % G.fz) * kFZ, i0 = (tile / G.fz) * kFR;
   const int m = kw > 1 ? kw : 1;
   const bool interior = i0 - 6 >= m && i0 + kFR + 6 <= nr - m && j0 - 6 >= m &&
                         j0 + kFZ + 6 <= nz - m;
   double* part = partials + G.part0 + (int64_t)cl * G.ftiles;
   if (interior)
-    step_fused_tile<T, true>(psi + fo, chi + fo, wsrc + fo, wdst + fo, avg ? avg + fo : nullptr,
+    step_fused_tile<T, FusedFull, true>(psi + fo, chi + fo, wsrc + fo, wdst + fo, avg ? avg + fo : nullptr,
                              G.r, G.kill_wz, G.kill_wr, kw, nr, nz, T(G.dx),
                              sc + (int64_t)cb * AXS_RIGID_SCALARS,
                              slots + (int64_t)cb * kSlotsPerCase, part, cfgs[cb], L, i0, j0, tile);
   else
-    step_fused_tile<T, false>(psi + fo, chi + fo, wsrc + fo, wdst + fo, avg ? avg + fo : nullptr,
+    step_fused_tile<T, FusedFull, false>(psi + fo, chi + fo, wsrc + fo, wdst + fo, avg ? avg + fo : nullptr,
                               G.r, G.kill_wz, G.kill_wr, kw, nr, nz, T(G.dx),
                               sc + (int64_t)cb * AXS_RIGID_SCALARS,
                               slots + (int64_t)cb * kSlotsPerCase, part, cfgs[cb], L, i0, j0, tile);
@@ -844,12 +887,24 @@ hipError_t launch_step_fused(const T* psi, const T* chi, const T* wsrc, T* wdst,
                              int nz, T dx, double* sc, const double* slots, double* partials,
                              const RigidConfig* cfgs, int batch, hipStream_t s, bool rk2) {
   const dim3 grid(ceil_div(nz, kFZ), ceil_div(nr, kFR), batch);
-  if (rk2)
-    step_fused_kernel<T, true><<<grid, 256, 0, s>>>(psi, chi, wsrc, wdst, avg, r, wz, wr, kw, nr,
-                                                    nz, dx, sc, slots, partials, cfgs);
+  const auto launch = [&](auto strips, auto with_rk2) {
+    using S = decltype(strips);
+    step_fused_kernel<T, S, decltype(with_rk2)::value><<<grid, S::NT, 0, s>>>(
+        psi, chi, wsrc, wdst, avg, r, wz, wr, kw, nr, nz, dx, sc, slots, partials, cfgs);
+  };
+  const auto launch_for = [&](auto strips) {
+    if (rk2)
+      launch(strips, std::true_type());
+    else
+      launch(strips, std::false_type());
+  };
+  const int64_t tiles = (int64_t)grid.x * grid.y * batch;
+  if (tiles <= kCUs)
+    launch_for(FusedFew());
+  else if (tiles <= (sizeof(T) == 8 ? 2 : 4) * kCUs)
+    launch_for(FusedSome());
   else
-    step_fused_kernel<T, false><<<grid, 256, 0, s>>>(psi, chi, wsrc, wdst, avg, r, wz, wr, kw, nr,
-                                                     nz, dx, sc, slots, partials, cfgs);
+    launch_for(FusedFull());
   return hipGetLastError();
 }
 
