@@ -280,7 +280,7 @@ def time_implicit(sizes=((256, 128), (1024, 512), (2048, 1024)), reps=20):
     step = DST-I rows, radial tridiagonal solves, DST-I rows.  256 x 128 is
     the torus-streaming grid that uses it; dt = dx^2 / 4 / nu
     (flow_past_sphere.py:90).  The DST-I rows run as (nz + 1)-point DFTs
-    (Stockham when nz + 1 factors into 2, 3 and 5, else chirp-z); the parity
+    (Stockham when nz + 1 factors into primes up to 13, else chirp-z); the parity
     tests check the result against the oracle."""
     import torch
 
@@ -307,8 +307,8 @@ def time_implicit(sizes=((256, 128), (1024, 512), (2048, 1024)), reps=20):
         res[f"{nz}x{nr}"] = dict(us_per_step=round(us, 2),
                                  mcell_steps_per_s=round(nr * nz / us, 2))
     return dict(unit="us per implicit step (drop-in, fields resident)", sizes=res,
-                note="DST-I rows as (nz + 1)-point DFTs in LDS (chirp-z when nz + 1 is not "
-                     "2,3,5-smooth)")
+                note="DST-I rows as (nz + 1)-point DFTs in LDS (chirp-z when nz + 1 has "
+                     "a prime factor above 13)")
 
 
 def time_potential(sizes=((256, 128), (2048, 1024)), reps=20):
@@ -414,8 +414,8 @@ def time_serving(n_requests, steps, max_active=32, seed=0, precision="f32", open
         closed_loop_wall_s=round(t_closed, 3),
         closed_loop_mcell_steps_per_s=round(cells / t_closed / 1e6, 2),
         failed_requests=failed + s["failed"],
-        # steps whose extrapolation loop outran the queued sweeps and was
-        # finished by the one-workgroup tail (results unchanged)
+        # steps whose extrapolation loop took the given number of sweeps or
+        # more (results do not depend on it)
         lsq_tail_steps=int(sum(r["lsq_unconverged"] for r in recs + recs2)),
         queued_lsq_sweeps=srv.last_batch_info[1] if srv.last_batch_info else None,
         precision=precision,
