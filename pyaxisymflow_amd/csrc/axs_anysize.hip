@@ -484,7 +484,7 @@ static void allow_large_lds() {
       (const void*)any_dct3_rows_kernel<double, P>, (const void*)any_dct3_rows_kernel<float, P>, \
       (const void*)any_rfft_rows_kernel<P>, (const void*)any_irfft_rows_kernel<P>,               \
       (const void*)any_dst1_rows_kernel<P>
-#define AXS_ANY_BATCH_KERNELS(P)                                                                    \
+#define AXS_ANY_BATCH_KERNELS(P)                                                                  \
   (const void*)soft_batch_dct2_kernel<double, P>, (const void*)soft_batch_dct3_kernel<double, P>, \
       (const void*)soft_batch_dct2_kernel<float, P>, (const void*)soft_batch_dct3_kernel<float, P>
     const void* ks[] = {(const void*)any_bhat_kernel<1>,  (const void*)any_bhat_kernel<2>,
@@ -597,8 +597,8 @@ template <typename B>
 hipError_t launch_soft_batch_dct2(const SoftCaseT<B>* cases, const SoftBatchDims& d,
                                   hipStream_t s) {
   const dim3 grid(d.max_nr, d.ncase);
-  AXS_ANY_BATCH_PER(d.any_per,
-                              (soft_batch_dct2_kernel<B, P><<<grid, d.any_nth, d.any_lds, s>>>(cases)));
+  AXS_ANY_BATCH_PER(
+      d.any_per, (soft_batch_dct2_kernel<B, P><<<grid, d.any_nth, d.any_lds, s>>>(cases)));
   return hipGetLastError();
 }
 
@@ -606,8 +606,8 @@ template <typename B>
 hipError_t launch_soft_batch_dct3(const SoftCaseT<B>* cases, const SoftBatchDims& d,
                                   hipStream_t s) {
   const dim3 grid(d.max_nr, d.ncase);
-  AXS_ANY_BATCH_PER(d.any_per,
-                              (soft_batch_dct3_kernel<B, P><<<grid, d.any_nth, d.any_lds, s>>>(cases)));
+  AXS_ANY_BATCH_PER(
+      d.any_per, (soft_batch_dct3_kernel<B, P><<<grid, d.any_nth, d.any_lds, s>>>(cases)));
   return hipGetLastError();
 }
 
