@@ -429,7 +429,7 @@ __device__ __forceinline__ double& packed_y(Cplx<double>* z, int m) {
 // Orthonormal DST-I rows (sqrt(2 / (N + 1)) S), its own inverse; a has
 // length M = nz + 1, em[k] = e^{-i pi k / M} for k <= nz.
 template <int PER>
-__global__ void __launch_bounds__(1024) any_dst1_rows_kernel(
+__device__ __forceinline__ void any_dst1_rows_body(
     const double* __restrict__ src, double* __restrict__ dst, int nz, AnyDftArgs a,
     const Cplx<double>* __restrict__ em, double norm) {
   extern __shared__ unsigned char smem_raw[];
@@ -457,6 +457,22 @@ __global__ void __launch_bounds__(1024) any_dst1_rows_kernel(
     // -Im(Y_k) / 2 with Y_k = s / 2 - i ed / 2
     out[k - 1] = (ed.x - s.y) * norm;
   }
+}
+template <int PER>
+__global__ void __launch_bounds__(1024) any_dst1_rows_kernel(
+    const double* __restrict__ src, double* __restrict__ dst, int nz, AnyDftArgs a,
+    const Cplx<double>* __restrict__ em, double norm) {
+  any_dst1_rows_body<PER>(src, dst, nz, a, em, norm);
+}
+// At most 80 scalar registers: a SIMD has 800, and a wave takes them in
+// steps of 16 with 16 more for the trap handler, so 81 leave seven waves
+// instead of eight and a CU one row of 1024 threads instead of two (a step at
+// 2000 x 1024: 37 us a row pass with 81, 29 with 80).
+template <>
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80)))
+any_dst1_rows_kernel<1>(const double* __restrict__ src, double* __restrict__ dst, int nz,
+                        AnyDftArgs a, const Cplx<double>* __restrict__ em, double norm) {
+  any_dst1_rows_body<1>(src, dst, nz, a, em, norm);
 }
 
 // Every kernel above may take more than the default 64 KiB of dynamic LDS
