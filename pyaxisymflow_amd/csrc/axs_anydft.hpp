@@ -37,9 +37,13 @@ struct AnyDftArgs {
 // Host owner of one length's device tables.
 struct AnyDft {
   AnyDftArgs args{};
-  // the length-L FFT's launch shape: nth threads, PER of fft_lds (plus
-  // kFftWide)
-  int nth = 64, per = 1;
+  // the length-L FFT's launch shape (nth threads, PER of fft_lds plus
+  // kFftWide) for many rows, and for rows that each have a CU to themselves
+  struct Shape {
+    int nth = 64, per = 1;
+  };
+  Shape many, few;
+  const Shape& shape(int rows) const { return rows <= kCUs ? few : many; }
   std::vector<void*> owned;  // device tables
   // primes: 13, or 5 for a batch's rows (any_dft_length)
   hipError_t init(int N, int primes = 13);

@@ -114,6 +114,36 @@ static void allow_large_lds();
 // bytes of dynamic LDS every any-kernel may take (raised by allow_large_lds)
 static int g_any_lds_limit = 65536;
 
+// Threads of a row of more than 1920 points when there are many: the PER that
+// keeps the most threads in flight on a CU (rows by its 160 KiB of LDS and by
+// the waves per SIMD that the registers of PER = 1, 2, 4 and of the wide
+// radices allow), the smallest where that is equal, but PER = 4 where it
+// holds more rows than PER = 2.  Whole multiples of 256 threads: a row's
+// waves spread evenly over the four SIMDs, where 5 or 6 waves leave room for
+// one row less than their number says.  us per step of 1024 rows, sine rows
+// of L points (a quarter, half, three quarters, all of 1024 threads): 2160
+// (chirp-z) 134 / 134 / 134 / 138, 384 threads 137; 2560 (direct) - / 106 / 96 /
+// 120, 320 threads 136; 2880 123 / 104 / 105 / 105; 3456 - / 140 / 168 / 153;
+// cosine rows of 1250 points (chirp-z, 2500) 169 / 160 / 139 / 179, 384
+// threads 192.
+static int long_row_threads(const AnyDftArgs& a, bool wide) {
+  const size_t lds = sizeof(Cplx<double>) * (size_t)a.L * (a.stage ? 2 : 1);
+  const int in_lds = (int)((size_t)160 * 1024 / lds);
+  int nth = 0, rows = 0;
+  for (int p : {1, 2, 4}) {
+    const int t = (fft_threads(a, p, wide) + 255) / 256 * 256;
+    if (t > 1024) continue;
+    const int waves = wide || p == 4 ? 4 : p == 2 ? 6 : 7;  // per SIMD
+    const int r = std::min(in_lds, waves / (t / 256));
+    const int n = r == 1 ? 1024 : t;
+    if (r * n > rows * nth || (p == 4 && r * n == rows * nth && r > rows)) {
+      nth = n;
+      rows = r;
+    }
+  }
+  return nth;
+}
+
 hipError_t AnyDft::init(int N, int primes) {
   allow_large_lds();
   bool blue = false;
@@ -128,31 +158,23 @@ hipError_t AnyDft::init(int N, int primes) {
   args.stage = 2 * sizeof(Cplx<double>) * (size_t)L <= 65536 ? 1 : 0;
   radices_of(L, primes, &args.fp);
   const bool wide = fft_wide(args);
-  nth = std::max(64, (L / (wide ? 4 : 2) + 63) / 64 * 64);
-  if (nth >= 1024) {
-    // long rows: the butterflies per thread that keep the most rows in flight
-    // on a CU (its 160 KiB of LDS; the threads that the registers of PER = 1,
-    // 2, 4 and of the wide radices allow), the fewest where that is equal
-    // (1351 x 680, FFTs of 2880 points: 264 -> 188 us per step with 512
-    // threads, three rows on a CU, instead of 640; stokes 1501 x 700:
-    // 182 -> 116 us)
-    const size_t lds = sizeof(Cplx<double>) * (size_t)L * (args.stage ? 2 : 1);
-    const int in_lds = (int)((size_t)160 * 1024 / lds);
-    int most = 0;
-    for (int p : {1, 2, 4}) {
-      const int t = fft_threads(args, p, wide);
-      const int threads = wide || p == 4 ? 1024 : p == 2 ? 1536 : 2048;
-      const int rows = std::min(in_lds, threads / t);
-      if (t <= 1024 && rows > most) {
-        most = rows;
-        nth = std::min(1024, threads / rows / 64 * 64);
-      }
+  many.nth = std::max(64, (L / (wide ? 4 : 2) + 63) / 64 * 64);
+  if (many.nth >= 1024) many.nth = long_row_threads(args, wide);
+  if (!many.nth) return hipErrorInvalidValue;
+  many.nth = std::max(many.nth, fft_threads(args, 4, wide));
+  many.per = fft_per(args, many.nth, wide);
+  few = many;
+  if (L > 1920 && !wide) {
+    // a row alone on its CU: the fewest butterflies per thread (160 rows:
+    // sine rows of 3456 points 51 us with 512 threads by 4, 45 with 1024 by
+    // 2; of 2880 points 41 and 38)
+    for (int p : {4, 2, 1}) {
+      const int t = (fft_threads(args, p, false) + 255) / 256 * 256;
+      if (t <= 1024) few = Shape{p == 2 ? t : 1024, p};
     }
-    if (!most) return hipErrorInvalidValue;
   }
-  nth = std::max(nth, fft_threads(args, 4, wide));
-  per = fft_per(args, nth, wide);
-  if (wide) per |= kFftWide;
+  if (wide) many.per |= kFftWide;
+  if (wide) few.per |= kFftWide;
   std::vector<Cplx<double>> tw(L);
   for (int t = 0; t < L; ++t) {
     const double ang = -2.0 * M_PI * (double)t / (double)L;
@@ -184,12 +206,12 @@ hipError_t AnyDft::init(int N, int primes) {
   owned.push_back(d_bhat);
   const size_t shm = lds_bytes<double>();
   // chirp-z lengths hold radices up to 5 only
-  if (per == 1)
-    any_bhat_kernel<1><<<1, nth, shm, 0>>>(d_bhat, args);
-  else if (per == 2)
-    any_bhat_kernel<2><<<1, nth, shm, 0>>>(d_bhat, args);
+  if (many.per == 1)
+    any_bhat_kernel<1><<<1, many.nth, shm, 0>>>(d_bhat, args);
+  else if (many.per == 2)
+    any_bhat_kernel<2><<<1, many.nth, shm, 0>>>(d_bhat, args);
   else
-    any_bhat_kernel<4><<<1, nth, shm, 0>>>(d_bhat, args);
+    any_bhat_kernel<4><<<1, many.nth, shm, 0>>>(d_bhat, args);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if ((e = hipDeviceSynchronize()) != hipSuccess) return e;
   args.chirp = d_chirp;
@@ -569,12 +591,14 @@ hipError_t launch_any_dct2_rows(const StokesPlan& pl, const T* src, T* tapered, 
   const StepFinalize f = fin ? *fin : StepFinalize{};
   const dim3 grid(pl.nr + (f.partials ? 1 : 0), batch);
   const size_t shm = D.lds_bytes<T>();
-  const int nth = D.nth;
+  // the completed step's force is summed in an order that depends on the
+  // threads: one shape for a case alone and in a batch
+  const AnyDft::Shape h = D.shape(f.partials ? pl.nr : pl.nr * batch);
   if (taper)
-    AXS_ANY_PER(D.per, (any_dct2_rows_kernel<T, P, true><<<grid, nth, shm, s>>>(
+    AXS_ANY_PER(h.per, (any_dct2_rows_kernel<T, P, true><<<grid, h.nth, shm, s>>>(
                        src, tapered, dst, rscale, wz, wr, pl.nr, pl.nz, w, tb, f)));
   else
-    AXS_ANY_PER(D.per, (any_dct2_rows_kernel<T, P, false><<<grid, nth, shm, s>>>(
+    AXS_ANY_PER(h.per, (any_dct2_rows_kernel<T, P, false><<<grid, h.nth, shm, s>>>(
                        src, nullptr, dst, rscale, nullptr, nullptr, pl.nr, pl.nz, 0, tb, f)));
   return hipGetLastError();
 }
@@ -584,7 +608,8 @@ hipError_t launch_any_dct3_rows(const StokesPlan& pl, const T* src, T* dst, int 
                                 hipStream_t s) {
   const AnyDft& D = *pl.any;
   const AnyDctTables tb{D.args, pl.ge2, pl.e1, pl.e2, pl.any_half ? 1 : 0};
-  AXS_ANY_PER(D.per, (any_dct3_rows_kernel<T, P><<<dim3(rows, batch), D.nth, D.lds_bytes<T>(), s>>>(
+  const AnyDft::Shape h = D.shape(rows * batch);
+  AXS_ANY_PER(h.per, (any_dct3_rows_kernel<T, P><<<dim3(rows, batch), h.nth, D.lds_bytes<T>(), s>>>(
                      src, dst, rows, pl.nz, tb)));
   return hipGetLastError();
 }
@@ -593,10 +618,11 @@ hipError_t launch_any_rfft_rows(const StokesPlan& pl, const double* src, double*
                                 const double* rscale, int rows, bool inverse, hipStream_t s) {
   const AnyDft& D = *pl.any;
   const size_t shm = D.lds_bytes<double>();
+  const AnyDft::Shape h = D.shape(rows);
   if (inverse)
-    AXS_ANY_PER(D.per, (any_irfft_rows_kernel<P><<<rows, D.nth, shm, s>>>(src, dst, pl.nz, D.args)));
+    AXS_ANY_PER(h.per, (any_irfft_rows_kernel<P><<<rows, h.nth, shm, s>>>(src, dst, pl.nz, D.args)));
   else
-    AXS_ANY_PER(D.per, (any_rfft_rows_kernel<P><<<rows, D.nth, shm, s>>>(src, dst, rscale, pl.nz,
+    AXS_ANY_PER(h.per, (any_rfft_rows_kernel<P><<<rows, h.nth, shm, s>>>(src, dst, rscale, pl.nz,
                                                                       D.args)));
   return hipGetLastError();
 }
@@ -604,7 +630,8 @@ hipError_t launch_any_rfft_rows(const StokesPlan& pl, const double* src, double*
 hipError_t launch_any_dst1_rows(const AnyDft& D, const Cplx<double>* em, const double* src,
                                 double* dst, int rows, int nz, hipStream_t s) {
   const double norm = std::sqrt(2.0 / (double)(nz + 1)) / 4.0;
-  AXS_ANY_PER(D.per, (any_dst1_rows_kernel<P><<<rows, D.nth, D.lds_bytes<double>(), s>>>(
+  const AnyDft::Shape h = D.shape(rows);
+  AXS_ANY_PER(h.per, (any_dst1_rows_kernel<P><<<rows, h.nth, D.lds_bytes<double>(), s>>>(
                      src, dst, nz, D.args, em, norm)));
   return hipGetLastError();
 }

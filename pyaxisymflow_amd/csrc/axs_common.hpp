@@ -14,6 +14,8 @@
 
 namespace axs {
 
+constexpr int kCUs = 256;  // compute units of the chip
+
 // Thread-local last-error string reported by axs_last_error().
 void set_error(const std::string& msg);
 void clear_error();

@@ -296,7 +296,6 @@ using FusedFull = FusedStrips<6, 5, 6, 4>;
 // (874) 56.8 / 55.2 / 57.8, 2048 x 1024 (2432) 62.5 / 63.3 / 70.8.
 using FusedSome = FusedStrips<3, 4, 3, 2>;
 using FusedFew = FusedStrips<2, 2, 2, 2>;
-constexpr int kCUs = 256;
 // LDS buffers and what they hold phase by phase.
 constexpr int kBufA = kR6R * kR6Z;  // psi (R6), then f (R4)
 constexpr int kBufC = kR4R * kR4Z;  // u_pen_z (R4), then stage-1 out (R1)
