@@ -62,11 +62,75 @@ static bool radices_of(int M, int primes, FftPlanArgs* p) {
   return m == 1;
 }
 
-// The chirp-z length is the smallest smooth one without a lone radix 2 (that
-// stage has the most butterflies and does the least), unless that is more
-// than 1 / 16 longer than the smallest of all: 4500 points instead of 4320 for
-// N = 2049, 284 -> 202 us per implicit step at 2048 x 1024; 1125 instead of
-// 1080 for 513, 33 -> 31 us at 512 x 256.  Factors 7, 11 and 13 are radices of
+// The FFT twiddles are staged in LDS only while the doubled footprint still
+// lets two workgroups share a CU (longer rows lose more to occupancy than the
+// LDS twiddles save).
+static int stages_twiddles(int L) { return 2 * sizeof(Cplx<double>) * (size_t)L <= 65536 ? 1 : 0; }
+
+// Threads of a row of more than 1920 points when there are many: the PER that
+// keeps the most threads in flight on a CU (rows by its 160 KiB of LDS and by
+// the waves per SIMD that the registers of PER = 1, 2, 4 and of the wide
+// radices allow), the smallest where that is equal, but PER = 4 where it
+// holds more rows than PER = 2.  Whole multiples of 256 threads: a row's
+// waves spread evenly over the four SIMDs, where 5 or 6 waves leave room for
+// one row less than their number says.  us per step of 1024 rows, sine rows
+// of L points (a quarter, half, three quarters, all of 1024 threads): 2160
+// (chirp-z) 134 / 134 / 134 / 138, 384 threads 137; 2560 (direct) - / 106 / 96 /
+// 120, 320 threads 136; 2880 123 / 104 / 105 / 105; 3456 - / 140 / 168 / 153;
+// cosine rows of 1250 points (chirp-z, 2500) 169 / 160 / 139 / 179, 384
+// threads 192.
+struct LongRow {
+  int nth, rows;  // threads; rows in flight on a CU
+};
+static LongRow long_row(const AnyDftArgs& a, bool wide) {
+  const size_t lds = sizeof(Cplx<double>) * (size_t)a.L * (a.stage ? 2 : 1);
+  const int in_lds = (int)((size_t)160 * 1024 / lds);
+  int nth = 0, rows = 0;
+  for (int p : {1, 2, 4}) {
+    const int t = (fft_threads(a, p, wide) + 255) / 256 * 256;
+    if (t > 1024) continue;
+    const int waves = wide || p == 4 ? 4 : p == 2 ? 6 : 7;  // per SIMD
+    const int r = std::min(in_lds, waves / (t / 256));
+    const int n = r == 1 ? 1024 : t;
+    if (r * n > rows * nth || (p == 4 && r * n == rows * nth && r > rows)) {
+      nth = n;
+      rows = r;
+    }
+  }
+  return {nth, rows};
+}
+
+// Whether chirp-z rows of l points, a length without a lone radix 2, are
+// faster than rows of the L < l that is the shortest.  A stage costs about the
+// same in any radix, so a length with fewer stages is, if its waves spread
+// over the four SIMDs as well (us per implicit step of 1024 rows: 1125 points
+// 71, 1080 79; 1875 108, 1800 121; but 1280 94, 1250 83, equal stages, and
+// 1600 128, 1536 120, thirteen waves for twelve).  Of more than 1920 points
+// the radix 2 also sets the butterflies per thread and the rows in flight:
+// 2160 points 134, 2048 167; 3375 182, 3200 203; 5120 280, 5000 343; but 6912
+// 485, 6750 444, equal in all three.
+static bool better_length(int l, int L) {
+  AnyDftArgs a, b;
+  a.L = l;
+  b.L = L;
+  a.stage = stages_twiddles(l);
+  b.stage = stages_twiddles(L);
+  radices_of(l, 5, &a.fp);
+  radices_of(L, 5, &b.fp);
+  const bool fewer = a.fp.nstages < b.fp.nstages;
+  if (L <= 1920) {
+    const int wl = (l / 2 + 63) / 64, wL = (L / 2 + 63) / 64;
+    return fewer && (wl == wL || wl % 4 == 0);
+  }
+  const LongRow A = long_row(a, false), B = long_row(b, false);
+  return fewer || A.rows > B.rows || fft_per(a, A.nth, false) < fft_per(b, B.nth, false);
+}
+
+// The chirp-z length is the smallest smooth one, or one up to 1 / 16 longer
+// without its lone radix 2 (that stage has the most butterflies and does the
+// least) where that is faster: 4500 points instead of 4320 for N = 2049, 284 ->
+// 202 us per implicit step at 2048 x 1024; 1125 instead of 1080 for 513, 33 ->
+// 31 us at 512 x 256.  Factors 7, 11 and 13 are radices of
 // their own where the chirp-z form would do too (rows of 770, 385 = 5 x 7 x 11
 // points instead of two FFTs of 800: 68.6 -> 62.3 us per step of 770 x 386;
 // 113 -> 72 us at 1001 x 500); the longest rows stay those it holds.  A
@@ -84,7 +148,8 @@ int any_dft_length(int N, bool* bluestein, int primes) {
   if (bluestein) *bluestein = true;
   if (primes == 5) return L;
   for (int l = L; l <= std::min(L + L / 16, kAnyMaxL); ++l)
-    if (radices_of(l, 5, &p) && __builtin_ctz(l) % 2 == 0) return l;
+    if (radices_of(l, 5, &p) && __builtin_ctz(l) % 2 == 0 && (l == L || better_length(l, L)))
+      return l;
   return L;
 }
 
@@ -114,36 +179,6 @@ static void allow_large_lds();
 // bytes of dynamic LDS every any-kernel may take (raised by allow_large_lds)
 static int g_any_lds_limit = 65536;
 
-// Threads of a row of more than 1920 points when there are many: the PER that
-// keeps the most threads in flight on a CU (rows by its 160 KiB of LDS and by
-// the waves per SIMD that the registers of PER = 1, 2, 4 and of the wide
-// radices allow), the smallest where that is equal, but PER = 4 where it
-// holds more rows than PER = 2.  Whole multiples of 256 threads: a row's
-// waves spread evenly over the four SIMDs, where 5 or 6 waves leave room for
-// one row less than their number says.  us per step of 1024 rows, sine rows
-// of L points (a quarter, half, three quarters, all of 1024 threads): 2160
-// (chirp-z) 134 / 134 / 134 / 138, 384 threads 137; 2560 (direct) - / 106 / 96 /
-// 120, 320 threads 136; 2880 123 / 104 / 105 / 105; 3456 - / 140 / 168 / 153;
-// cosine rows of 1250 points (chirp-z, 2500) 169 / 160 / 139 / 179, 384
-// threads 192.
-static int long_row_threads(const AnyDftArgs& a, bool wide) {
-  const size_t lds = sizeof(Cplx<double>) * (size_t)a.L * (a.stage ? 2 : 1);
-  const int in_lds = (int)((size_t)160 * 1024 / lds);
-  int nth = 0, rows = 0;
-  for (int p : {1, 2, 4}) {
-    const int t = (fft_threads(a, p, wide) + 255) / 256 * 256;
-    if (t > 1024) continue;
-    const int waves = wide || p == 4 ? 4 : p == 2 ? 6 : 7;  // per SIMD
-    const int r = std::min(in_lds, waves / (t / 256));
-    const int n = r == 1 ? 1024 : t;
-    if (r * n > rows * nth || (p == 4 && r * n == rows * nth && r > rows)) {
-      nth = n;
-      rows = r;
-    }
-  }
-  return nth;
-}
-
 hipError_t AnyDft::init(int N, int primes) {
   allow_large_lds();
   bool blue = false;
@@ -153,13 +188,11 @@ hipError_t AnyDft::init(int N, int primes) {
   args.N = N;
   args.L = L;
   args.bluestein = blue ? 1 : 0;
-  // staged only while the doubled footprint still lets two workgroups share
-  // a CU (longer rows lose more to occupancy than the LDS twiddles save)
-  args.stage = 2 * sizeof(Cplx<double>) * (size_t)L <= 65536 ? 1 : 0;
+  args.stage = stages_twiddles(L);
   radices_of(L, primes, &args.fp);
   const bool wide = fft_wide(args);
   many.nth = std::max(64, (L / (wide ? 4 : 2) + 63) / 64 * 64);
-  if (many.nth >= 1024) many.nth = long_row_threads(args, wide);
+  if (many.nth >= 1024) many.nth = long_row(args, wide).nth;
   if (!many.nth) return hipErrorInvalidValue;
   many.nth = std::max(many.nth, fft_threads(args, 4, wide));
   many.per = fft_per(args, many.nth, wide);
