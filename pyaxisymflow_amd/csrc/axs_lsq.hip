@@ -268,7 +268,8 @@ static hipError_t launch_fill_u32(unsigned* p, int n, unsigned v, hipStream_t s)
 // is its 8-neighbour distance from the known set within the target set,
 // whatever the values are.  The loop then splits into three launches:
 //   levels  one workgroup per case walks the fronts on bit rows in LDS and
-//           lists the cells front by front;
+//           lists the cells front by front (the first fronts of a large solid
+//           are launches of their own: kLsqLargeRadius);
 //   factor  one thread per listed cell: its window, the cells of it known
 //           before its front, and the factored normal matrix, none of which
 //           depends on the values;
@@ -309,20 +310,45 @@ __device__ __forceinline__ unsigned lsq_dilate(const unsigned* known, int row, i
   return d;
 }
 
-// Lists the cells of `bits`, whose lowest is cell `base`, as front `level`.
-__device__ __forceinline__ void lsq_emit(const LsqWork& w, unsigned bits, unsigned base, int level,
-                                         unsigned* s_n) {
-  // the counter's address made to look divergent: on a uniform address the
-  // compiler adds the lanes up one by one in a loop before its one atomic
-  int zero;
-  asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
-  unsigned pos = atomicAdd(s_n + zero, (unsigned)__popc(bits));
+// The same on words in global memory, every load issued at once (a word outside
+// the rows reads its neighbour and counts as 0).
+__device__ __forceinline__ unsigned lsq_dilate_at(const unsigned* known, int row, int c, int rows,
+                                                  int wc) {
+  unsigned m[9];
+#pragma unroll
+  for (int n = 0; n < 9; ++n) {
+    const int r = min(max(row + n / 3 - 1, 0), rows - 1), q = min(max(c + n % 3 - 1, 0), wc - 1);
+    m[n] = known[(int64_t)r * wc + q];
+  }
+  unsigned d = 0u;
+#pragma unroll
+  for (int n = 0; n < 3; ++n) {
+    const int r = row + n - 1;
+    const unsigned mid = m[3 * n + 1];
+    const unsigned left = c > 0 ? m[3 * n] >> 31 : 0u, right = c + 1 < wc ? m[3 * n + 2] << 31 : 0u;
+    if (r >= 0 && r < rows) d |= mid | (mid << 1) | (mid >> 1) | left | right;
+  }
+  return d;
+}
+
+// Lists the cells of `bits`, whose lowest is cell `base`, as front `level`,
+// from entry `pos` on.
+__device__ __forceinline__ void lsq_list_bits(const LsqWork& w, unsigned bits, unsigned base,
+                                              int level, unsigned pos) {
   while (bits) {
     const unsigned cell = base + (unsigned)__ffs((int)bits) - 1u;
     bits &= bits - 1u;
     w.list[pos++] = LsqEntry{(int)cell, level};
     w.lev[cell] = level;
   }
+}
+__device__ __forceinline__ void lsq_emit(const LsqWork& w, unsigned bits, unsigned base, int level,
+                                         unsigned* s_n) {
+  // the counter's address made to look divergent: on a uniform address the
+  // compiler adds the lanes up one by one in a loop before its one atomic
+  int zero;
+  asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+  lsq_list_bits(w, bits, base, level, atomicAdd(s_n + zero, (unsigned)__popc(bits)));
 }
 
 // Block barrier that orders LDS accesses alone: the global stores of a
@@ -332,31 +358,55 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// The fronts of one case, by one workgroup of kLsqThreads.  zone[1]: the
-// last physical row with a target cell (-1: none); the doubled rows with
-// target cells are nr - 1 - zone[1] .. nr + zone[1].
+// The fronts of one case, by one workgroup of kLsqThreads, after the first
+// `done` of them (0 or kLsqFrontLaunches: lsq_front_levels_body has listed
+// those).  zone[1]: the last physical row with a target cell (-1: none); the
+// doubled rows with target cells are nr - 1 - zone[1] .. nr + zone[1].
 __device__ __forceinline__ void lsq_levels_body(const LsqWork& w, int nr, int nz,
-                                                const int* __restrict__ zone) {
+                                                const int* __restrict__ zone, int done) {
   __shared__ unsigned sk[kLsqLdsWords];
   __shared__ int s_w0, s_w1;
-  __shared__ unsigned s_n;
+  __shared__ unsigned s_n, s_m;
   const int tid = threadIdx.x;
+  unsigned n = 0u;
+  int level = 0;
+  for (; level < done; ++level) {  // uniform
+    const unsigned c = w.cnt[level];
+    if (!c) break;
+    n += c;
+    if (tid == 0) w.off[level + 1] = (int)n;
+  }
+  if (tid == 0) w.off[0] = 0;
+  if (level < done) {  // a front of the launches found nothing: all are listed
+    if (tid == 0) {
+      w.head[0] = n;
+      w.head[1] = (unsigned)level;
+    }
+    return;
+  }
   const int z1 = zone[1];
   const int W = (nz + 31) / 32, r0 = nr - 1 - z1, rows = 2 * (z1 + 1);
   if (tid == 0) {
     s_w0 = W;
     s_w1 = -1;
-    s_n = 0u;
+    s_n = n;
+    s_m = 0u;
   }
   __syncthreads();
-  // word columns with target cells
+  // word columns with target cells, from the box's rows of words as they
+  // lie (whole groups of four; a row's words beyond nz are 0)
+  const int G = w.wstride / 4, ng = rows * G;
+  const uint4* tb4 = reinterpret_cast<const uint4*>(w.tb + (int64_t)r0 * w.wstride);
+  const uint4* kb4 = reinterpret_cast<const uint4*>(w.kb + (int64_t)r0 * w.wstride);
   int lo = W, hi = -1;
-  for (int q = tid; q < rows * W; q += kLsqThreads) {
-    const int r = (int)((unsigned)q / (unsigned)W), c = q - r * W;
-    if (w.tb[(int64_t)(r0 + r) * w.wstride + c]) {
-      lo = min(lo, c);
-      hi = max(hi, c);
-    }
+#pragma unroll 4
+  for (int q = tid; q < ng; q += kLsqThreads) {
+    const uint4 t = tb4[q];
+    const int c = (int)((unsigned)q % (unsigned)G) * 4;
+    const unsigned any =
+        (t.x ? 1u : 0u) | (t.y ? 2u : 0u) | (t.z ? 4u : 0u) | (t.w ? 8u : 0u);
+    lo = any ? min(lo, c + __ffs((int)any) - 1) : lo;
+    hi = any ? max(hi, c + 31 - __clz((int)any)) : hi;
   }
   if (hi >= 0) {
     atomicMin(&s_w0, lo);
@@ -364,8 +414,6 @@ __device__ __forceinline__ void lsq_levels_body(const LsqWork& w, int nr, int nz
   }
   __syncthreads();
   const int w0 = s_w0, wc = max(0, s_w1 - s_w0 + 1), nw = rows * wc;
-  unsigned n = 0u;
-  int level = 0;
   // A front's cells join the known ones only after every thread has read
   // the known words (first barrier), and are read by the next front after
   // all have joined (second barrier); s_n moves between the second and the
@@ -415,26 +463,51 @@ __device__ __forceinline__ void lsq_levels_body(const LsqWork& w, int nr, int nz
       lds_barrier();
     }
   } else {
-    // a box too large for LDS: the same walk on the case's global words
-    // (todo and f words are each read and written by one thread only)
-    for (int q = tid; q < nw; q += kLsqThreads) {
-      const int r = q / wc;
-      const int64_t g = (int64_t)(r0 + r) * w.wstride + w0 + (q - r * wc);
-      const unsigned k = w.kb[g];
-      w.kw[q] = k;
-      w.tw[q] = w.tb[g] & ~k;
+    // A box too large for LDS: the same walk over a list of the words that
+    // hold cells to find, and the known words in global memory (kb itself:
+    // the next step's mirror writes these rows again).  A front costs the
+    // band's words instead of the box's: 129 us a step instead of 380 for a
+    // solid of radius 410 cells on 1024 x 512.  Four list entries at a time,
+    // so that their loads are in flight together.  A word's entries of tw and
+    // fw belong to one thread.
+#pragma unroll 4
+    for (int q = tid; q < ng; q += kLsqThreads) {
+      const uint4 t = tb4[q], k = kb4[q];
+      const int r = (int)((unsigned)q / (unsigned)G), c = (q - r * G) * 4;
+      const unsigned todo[4] = {t.x & ~k.x, t.y & ~k.y, t.z & ~k.z, t.w & ~k.w};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (!todo[u]) continue;
+        const unsigned i = atomicAdd(&s_m, 1u);
+        w.wl[i] = (unsigned)(r0 + r) << 16 | (unsigned)(c + u);  // 2 nr <= 8192
+        w.tw[i] = todo[u];
+      }
     }
     __syncthreads();
+    const int m = (int)s_m;
+    constexpr int kU = 4;
     for (;;) {
-      for (int q = tid; q < nw; q += kLsqThreads) {
-        const unsigned todo = w.tw[q];
-        if (!todo) continue;
-        const int r = q / wc, c = q - r * wc;
-        const unsigned f = lsq_dilate(w.kw, r, c, rows, wc) & todo;
-        w.fw[q] = f;
-        if (f)
-          lsq_emit(w, f, (unsigned)(r0 + r) * (unsigned)nz + (unsigned)(w0 + c) * 32u, level + 1,
-                   &s_n);
+      for (int b = tid; b < m; b += kU * kLsqThreads) {
+        unsigned at[kU], todo[kU], f[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          const int i = min(b + u * kLsqThreads, m - 1);
+          at[u] = w.wl[i];
+          todo[u] = w.tw[i];
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+          f[u] = lsq_dilate_at(w.kb + (int64_t)r0 * w.wstride, (int)(at[u] >> 16) - r0,
+                               (int)(at[u] & 0xffffu), rows, w.wstride) & todo[u];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          const int i = b + u * kLsqThreads;
+          if (i >= m) continue;
+          w.fw[i] = f[u];
+          if (f[u])
+            lsq_emit(w, f[u], (at[u] >> 16) * (unsigned)nz + (at[u] & 0xffffu) * 32u, level + 1,
+                     &s_n);
+        }
       }
       __syncthreads();
       const unsigned now = s_n;
@@ -442,21 +515,71 @@ __device__ __forceinline__ void lsq_levels_body(const LsqWork& w, int nr, int nz
       n = now;
       ++level;
       if (tid == 0) w.off[level] = (int)n;
-      for (int q = tid; q < nw; q += kLsqThreads) {
-        const unsigned todo = w.tw[q];
-        if (!todo) continue;
-        const unsigned f = w.fw[q];
+#pragma unroll 4
+      for (int i = tid; i < m; i += kLsqThreads) {
+        const unsigned f = w.fw[i];
         if (!f) continue;
-        w.kw[q] |= f;
-        w.tw[q] = todo & ~f;
+        const unsigned at = w.wl[i];
+        w.kb[(int64_t)(at >> 16) * w.wstride + (at & 0xffffu)] |= f;
+        w.tw[i] &= ~f;
       }
       __syncthreads();
     }
   }
   if (tid == 0) {
-    w.off[0] = 0;
     w.head[0] = n;
     w.head[1] = (unsigned)level;
+  }
+}
+
+// Front `front` (from 0) of a case by many workgroups of 256 threads, four
+// words each, this one the blk-th: from one buffer of known words into the
+// other, the cells found listed after the fronts before it.  cnt[i] holds the
+// cells of front i (cleared before the step's first); a front after one that
+// found nothing does nothing.
+__device__ __forceinline__ void lsq_front_levels_body(const LsqWork& w, int nr, int nz,
+                                                      const int* __restrict__ zone, int front,
+                                                      int blk) {
+  __shared__ unsigned s_n, s_at;
+  const int tid = threadIdx.x;
+  const int z1 = zone[1], r0 = nr - 1 - z1, rows = 2 * (z1 + 1);
+  const int G = w.wstride / 4, ng = rows * G;
+  if (blk * 256 >= ng || (front > 0 && w.cnt[front - 1] == 0u)) return;  // uniform
+  unsigned base = 0u;
+  for (int i = 0; i < front; ++i) base += w.cnt[i];
+  const int64_t o = (int64_t)r0 * w.wstride;
+  const unsigned* in = ((front & 1) ? w.kb2 : w.kb) + o;
+  unsigned* out = ((front & 1) ? w.kb : w.kb2) + o;
+  if (tid == 0) s_n = 0u;
+  __syncthreads();
+  const int q = blk * 256 + tid;
+  const int r = (int)((unsigned)q / (unsigned)G), c = (q - r * G) * 4;
+  unsigned f[4] = {0u, 0u, 0u, 0u};
+  unsigned n = 0u, pos = 0u;
+  if (q < ng) {
+    const uint4 k = reinterpret_cast<const uint4*>(in)[q];
+    const uint4 t = reinterpret_cast<const uint4*>(w.tb + o)[q];
+    const unsigned kw[4] = {k.x, k.y, k.z, k.w}, tw[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const unsigned todo = tw[u] & ~kw[u];
+      if (todo) f[u] = lsq_dilate_at(in, r, c + u, rows, w.wstride) & todo;
+      n += (unsigned)__popc(f[u]);
+    }
+    reinterpret_cast<uint4*>(out)[q] =
+        make_uint4(kw[0] | f[0], kw[1] | f[1], kw[2] | f[2], kw[3] | f[3]);
+  }
+  if (n) pos = atomicAdd(&s_n, n);
+  __syncthreads();
+  if (tid == 0 && s_n) s_at = base + atomicAdd(w.cnt + front, s_n);
+  __syncthreads();
+  if (!n) return;
+  pos += s_at;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    lsq_list_bits(w, f[u], (unsigned)(r0 + r) * (unsigned)nz + (unsigned)(c + u) * 32u, front + 1,
+                  pos);
+    pos += (unsigned)__popc(f[u]);
   }
 }
 
@@ -645,8 +768,14 @@ __device__ __forceinline__ void lsq_solve_body(const LsqWork& w, double* e, bool
 }
 
 __global__ void __launch_bounds__(kLsqThreads) lsq_levels_kernel(LsqWork w, int nr, int nz,
-                                                                 const int* __restrict__ zone) {
-  lsq_levels_body(w, nr, nz, zone);
+                                                                 const int* __restrict__ zone,
+                                                                 int done) {
+  lsq_levels_body(w, nr, nz, zone, done);
+}
+__global__ void __launch_bounds__(256) lsq_front_levels_kernel(LsqWork w, int nr, int nz,
+                                                               const int* __restrict__ zone,
+                                                               int front) {
+  lsq_front_levels_body(w, nr, nz, zone, front, blockIdx.x);
 }
 __global__ void __launch_bounds__(256) lsq_factor_kernel(LsqWork w, const double* __restrict__ ex,
                                                          const double* __restrict__ ey,
@@ -669,11 +798,21 @@ __global__ void __launch_bounds__(kLsqSolveThreads) lsq_solve_kernel(LsqWork w, 
 // 5,000).
 constexpr int kLsqFactorBlocks = 64;
 
+// Workgroups of a front of lsq_front_levels_body over a doubled grid.
+static int lsq_front_blocks(int nr, int nz) {
+  return (int)ceil_div((int64_t)2 * nr * (lsq_words(nz) / 4), 256);
+}
+
 hipError_t launch_lsq_fronts(const LsqWork& w, double* e1d, double* e2d, const double* z, int nr,
-                             int nz, const int* zone, hipStream_t s) {
-  lsq_levels_kernel<<<1, kLsqThreads, 0, s>>>(w, nr, nz, zone);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+                             int nz, const int* zone, bool large, hipStream_t s) {
+  const int done = large ? kLsqFrontLaunches : 0;
+  hipError_t e;
+  for (int k = 0; k < done; ++k) {
+    lsq_front_levels_kernel<<<lsq_front_blocks(nr, nz), 256, 0, s>>>(w, nr, nz, zone, k);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  lsq_levels_kernel<<<1, kLsqThreads, 0, s>>>(w, nr, nz, zone, done);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
   lsq_factor_kernel<<<kLsqFactorBlocks, 256, 0, s>>>(w, e1d, e2d, z, 2 * nr, nz);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   lsq_solve_kernel<<<2, kLsqSolveThreads, 0, s>>>(w, e1d, e2d, z, 2 * nr, nz);
@@ -684,9 +823,15 @@ hipError_t launch_lsq_fronts(const LsqWork& w, double* e1d, double* e2d, const d
 // kLsqFactorBlocks workgroups (factor) per case.
 template <typename B>
 __global__ void __launch_bounds__(kLsqThreads) soft_batch_lsq_levels_kernel(
-    const SoftCaseT<B>* __restrict__ cs) {
+    const SoftCaseT<B>* __restrict__ cs, int done) {
   const SoftCaseT<B>& C = cs[blockIdx.x];
-  lsq_levels_body(C.lw, C.nr, C.nz, C.zone);
+  lsq_levels_body(C.lw, C.nr, C.nz, C.zone, done);
+}
+template <typename B>
+__global__ void __launch_bounds__(256) soft_batch_lsq_front_levels_kernel(
+    const SoftCaseT<B>* __restrict__ cs, int front) {
+  const SoftCaseT<B>& C = cs[blockIdx.y];
+  lsq_front_levels_body(C.lw, C.nr, C.nz, C.zone, front, blockIdx.x);
 }
 template <typename B>
 __global__ void __launch_bounds__(256) soft_batch_lsq_factor_kernel(
@@ -705,9 +850,15 @@ __global__ void __launch_bounds__(kLsqSolveThreads) soft_batch_lsq_solve_kernel(
 template <typename B>
 hipError_t launch_soft_batch_lsq(const SoftCaseT<B>* cases, const SoftBatchDims& d,
                                  hipStream_t s) {
-  soft_batch_lsq_levels_kernel<B><<<d.ncase, kLsqThreads, 0, s>>>(cases);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  const int done = d.large_solid ? kLsqFrontLaunches : 0;
+  hipError_t e;
+  for (int k = 0; k < done; ++k) {
+    soft_batch_lsq_front_levels_kernel<B>
+        <<<dim3(lsq_front_blocks(d.max_nr, d.max_nz), d.ncase), 256, 0, s>>>(cases, k);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  soft_batch_lsq_levels_kernel<B><<<d.ncase, kLsqThreads, 0, s>>>(cases, done);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
   soft_batch_lsq_factor_kernel<B><<<dim3(kLsqFactorBlocks, d.ncase), 256, 0, s>>>(cases);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   soft_batch_lsq_solve_kernel<B><<<dim3(2, d.ncase), kLsqSolveThreads, 0, s>>>(cases);

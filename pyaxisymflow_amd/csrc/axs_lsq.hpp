@@ -14,9 +14,14 @@ struct LsqEntry {
 // the target cells; the values are extrapolated in place.
 struct LsqWork {
   // bit rows of wstride words, 32 cells a word: cells known before the
-  // extrapolation, and target cells (the known ones among them)
+  // extrapolation (a walk outside LDS adds those it finds), and target cells
+  // (the known ones among them)
   unsigned *kb, *tb;
-  unsigned *kw, *tw, *fw;  // fronts of a box that does not fit in LDS
+  unsigned* kb2;  // the known cells after every other front of the launches
+  unsigned* cnt;  // cells of each front of the launches (cleared by the step's dt pass)
+  // a box that does not fit in LDS: the words with cells to find (row << 16 |
+  // word of the row), their cells not found yet and found by this front
+  unsigned *wl, *tw, *fw;
   int wstride;
   int* lev;       // 0 known, else the front that fits the cell; kLsqNever: none has yet
   LsqEntry* list; // cells to fit, front after front
@@ -28,6 +33,19 @@ struct LsqWork {
 };
 
 constexpr int kLsqNever = 0x7fffffff;
+
+// A solid whose radius is this many cells or more is large: the first
+// kLsqFrontLaunches fronts of a step (a stiff solid's loop takes 9 to 13) are
+// found by launches of many workgroups, the others by one.  About there
+// one workgroup's walk no longer fits in LDS; us a step, one workgroup / the
+// launches: radius 205 cells (512 x 256) 52 / -, 410 (1024 x 512) 129 (380 on the
+// whole box) / 92, 1638 (4096 x 2048) 511 (4918) / 136.
+constexpr double kLsqLargeRadius = 224.0;
+constexpr int kLsqFrontLaunches = 12;
+static_assert(kLsqFrontLaunches % 2 == 0, "the known cells end in kb");
+__host__ __device__ constexpr bool lsq_large(double r_ball, double dx) {
+  return r_ball >= kLsqLargeRadius * dx;
+}
 
 // Words per bit row: whole 256-column workgroups of the mirror pass.
 __host__ __device__ constexpr int lsq_words(int nz) { return (nz + 255) / 256 * 8; }
@@ -43,6 +61,6 @@ __host__ __device__ constexpr int lsq_factor_cap(int64_t n) { return int(n / 16 
 // bit for bit, in three launches.  z: coordinates of both axes.  zone[1]:
 // the last physical row with a target cell, -1 if none.
 hipError_t launch_lsq_fronts(const LsqWork& w, double* e1d, double* e2d, const double* z, int nr,
-                             int nz, const int* zone, hipStream_t s);
+                             int nz, const int* zone, bool large, hipStream_t s);
 
 }  // namespace axs

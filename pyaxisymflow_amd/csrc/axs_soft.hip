@@ -102,7 +102,8 @@ __device__ __forceinline__ void soft_dt_body(double* __restrict__ sc, double* __
 }
 
 __global__ void soft_dt_kernel(double* __restrict__ sc, double* __restrict__ slots,
-                               int* __restrict__ zone, SoftConfig cfg) {
+                               int* __restrict__ zone, unsigned* __restrict__ cnt, SoftConfig cfg) {
+  if (threadIdx.x < kLsqFrontLaunches) cnt[threadIdx.x] = 0u;
   if (threadIdx.x == 0) {  // an empty target zone for the mirror to record
     zone[0] = cfg.nr;
     zone[1] = -1;
@@ -385,13 +386,14 @@ struct SoftStepperT {
     lw.wstride = lsq_words(cfg.nz);
     lw.fcap = lsq_factor_cap((int64_t)nd);
     const size_t wb = sizeof(unsigned) * 2 * (size_t)cfg.nr * lw.wstride;
-    for (unsigned** f : {&lw.kb, &lw.tb, &lw.kw, &lw.tw, &lw.fw})
+    for (unsigned** f : {&lw.kb, &lw.kb2, &lw.tb, &lw.wl, &lw.tw, &lw.fw})
       if ((e = alloc(f, wb)) != hipSuccess) return e;
     if ((e = alloc(&lw.lev, nd * sizeof(int))) != hipSuccess) return e;
     if ((e = alloc(&lw.list, nd * sizeof(LsqEntry))) != hipSuccess) return e;
     const size_t fronts = (size_t)lsq_max_fronts((int64_t)nd) + 1;
     if ((e = alloc(&lw.off, fronts * sizeof(int))) != hipSuccess) return e;
     if ((e = alloc(&lw.head, 2 * sizeof(unsigned))) != hipSuccess) return e;
+    if ((e = alloc(&lw.cnt, kLsqFrontLaunches * sizeof(unsigned))) != hipSuccess) return e;
     if ((e = alloc(&lw.win, nd * sizeof(unsigned))) != hipSuccess) return e;
     if ((e = alloc(&lw.fac, 9 * (size_t)lw.fcap * D8)) != hipSuccess) return e;
     // every row: the first step a case takes here visits the whole grid
@@ -451,7 +453,7 @@ struct SoftStepperT {
     const int mb = std::min<int64_t>(ceil_div(n, 256), 1024);
     soft_velocity_max_kernel<<<mb, 256, 0, s>>>(buf.u_z, buf.u_r, n, slots);
     AXS_TRY_LAUNCH();
-    soft_dt_kernel<<<1, 64, 0, s>>>(sc, slots, zone, cfg);
+    soft_dt_kernel<<<1, 64, 0, s>>>(sc, slots, zone, lw.cnt, cfg);
     AXS_TRY_LAUNCH();
     AXS_TRY_STEP(launch_eno3_refmap<double>(buf.eta1, buf.eta2, buf.u_z, buf.u_r, e1n, e2n, nr,
                                             nz, Scalar<double>{0.0, sc + kSsDtByDx}, s));
@@ -468,7 +470,8 @@ struct SoftStepperT {
         buf.phi, buf.char_func, cfg.moll_zone, buf.eta1, buf.eta2, e1d, e2d, lw, zone, nr, nz,
         cfg.extrap_zone);
     AXS_TRY_LAUNCH();
-    AXS_TRY_STEP(launch_lsq_fronts(lw, e1d, e2d, buf.z, nr, nz, zone, s));
+    AXS_TRY_STEP(launch_lsq_fronts(lw, e1d, e2d, buf.z, nr, nz, zone,
+                                   lsq_large(cfg.r_ball, cfg.dx), s));
     soft_lsq_back_kernel<<<ceil_div(n, 256), 256, 0, s>>>(buf.eta1, buf.eta2, e1d, e2d, buf.phi,
                                                           cfg.extrap_zone, n);
     AXS_TRY_LAUNCH();
@@ -568,6 +571,7 @@ using SoftStepper = SoftStepperT<double>;
 template <typename B>
 __global__ void soft_batch_dt_kernel(const SoftCaseT<B>* __restrict__ cs) {
   const SoftCaseT<B>& C = cs[blockIdx.x];
+  if (threadIdx.x < kLsqFrontLaunches) C.lw.cnt[threadIdx.x] = 0u;
   if (threadIdx.x == 0) {  // the last step's zone kept, an empty one to record
     C.zone[2] = C.zone[0];
     C.zone[3] = C.zone[1];
@@ -775,6 +779,7 @@ struct SoftBatchT {
       const SoftStepperT<B>& S = *c.st;
       h_cases.push_back(describe(S, need));
       const StokesPlan& P = *S.plan;
+      dims.large_solid |= lsq_large(S.cfg.r_ball, S.cfg.dx);
       dims.max_nr = std::max(dims.max_nr, P.nr);
       dims.max_nz = std::max(dims.max_nz, P.nz);
       dims.max_chunks = std::max(dims.max_chunks, (int)ceil_div(P.nz, P.tri_K));

@@ -81,6 +81,7 @@ using SoftCase = SoftCaseT<double>;
 struct SoftBatchDims {
   int ncase = 0, max_nr = 0, max_nz = 0, max_chunks = 0;
   int any_nth = 64, any_per = 1;
+  bool large_solid = false;  // some case's solid is large (lsq_large)
   size_t any_lds = 0, tri_lds = 0;
   const uint32_t* cell_blocks = nullptr;
   int ncell_blocks = 0;
