@@ -275,7 +275,8 @@ static hipError_t launch_fill_u32(unsigned* p, int n, unsigned v, hipStream_t s)
 //           depends on the values;
 //   solve   one workgroup per case and component takes the fronts in order
 //           (a block barrier between them): window values in, right-hand
-//           side, back substitution, value out.
+//           side, back substitution, value out (a large solid's first
+//           fronts by many workgroups, a launch each).
 // One launch per sweep was bound by a fit's latency (flags, window, a 3 x 3
 // elimination with nine divisions, its pivoted rows in scratch memory): 17
 // us a sweep for twelve cases of 130 to 490 rows, paid for every queued
@@ -739,14 +740,16 @@ __device__ __forceinline__ LsqRecord lsq_record(const LsqWork& w, int k) {
 // and is not used) and writes its own cell.  A thread's first record of the
 // next front is loaded before this front's barrier, so that the front after
 // starts with its window's values.
+// The first `done` fronts are those of lsq_front_solve_body.
 __device__ __forceinline__ void lsq_solve_body(const LsqWork& w, double* e, bool second,
-                                               const double* __restrict__ g, int n0, int n1) {
+                                               const double* __restrict__ g, int n0, int n1,
+                                               int done) {
   const int levels = (int)w.head[1], total = (int)w.head[0];
   const int tid = threadIdx.x, nth = blockDim.x;
-  if (total == 0) return;
-  int begin = 0, end = w.off[1], next = levels > 1 ? w.off[2] : end;
-  LsqRecord r = lsq_record(w, min(tid, total - 1));
-  for (int level = 1; level <= levels; ++level) {
+  if (levels <= done) return;
+  int begin = w.off[done], end = w.off[done + 1], next = levels > done + 1 ? w.off[done + 2] : end;
+  LsqRecord r = lsq_record(w, min(begin + tid, total - 1));
+  for (int level = done + 1; level <= levels; ++level) {
     const LsqRecord r1 = lsq_record(w, min(end + tid, total - 1));
     const int after = level + 2 <= levels ? w.off[level + 2] : next;
     for (int k = begin + tid; k < end; k += nth) {
@@ -764,6 +767,25 @@ __device__ __forceinline__ void lsq_solve_body(const LsqWork& w, double* e, bool
     begin = end;
     end = next;
     next = after;
+  }
+}
+
+// One component's fits of front `front` (from 0) by many workgroups: cells
+// idx, idx + stride, ... of it.
+__device__ __forceinline__ void lsq_front_solve_body(const LsqWork& w, double* e, bool second,
+                                                     const double* __restrict__ g, int n0, int n1,
+                                                     int front, int idx, int stride) {
+  if ((int)w.head[1] <= front) return;
+  const int end = w.off[front + 1];
+  for (int k = w.off[front] + idx; k < end; k += stride) {
+    LsqRecord r = lsq_record(w, k);
+    const int j = r.cell / n1, i = r.cell - j * n1;
+    const LsqWindow v = lsq_unpack(r.win, r.f.m0, r.f.m1);
+    const bool nan = second ? v.nan_y : v.nan_x;
+    if (k < w.fcap)
+      lsq_fit_window(v, nan, r.f, e, g, n0, n1, j, i);
+    else
+      lsq_fit_unfactored(v, nan, e, g, n0, n1, j, i);
   }
 }
 
@@ -790,8 +812,14 @@ constexpr int kLsqSolveThreads = 512;
 __global__ void __launch_bounds__(kLsqSolveThreads) lsq_solve_kernel(LsqWork w, double* ex,
                                                                      double* ey,
                                                                      const double* __restrict__ g,
-                                                                     int n0, int n1) {
-  lsq_solve_body(w, blockIdx.x ? ey : ex, blockIdx.x != 0, g, n0, n1);
+                                                                     int n0, int n1, int done) {
+  lsq_solve_body(w, blockIdx.x ? ey : ex, blockIdx.x != 0, g, n0, n1, done);
+}
+__global__ void __launch_bounds__(256) lsq_front_solve_kernel(LsqWork w, double* ex, double* ey,
+                                                              const double* __restrict__ g, int n0,
+                                                              int n1, int front) {
+  lsq_front_solve_body(w, blockIdx.y ? ey : ex, blockIdx.y != 0, g, n0, n1, front,
+                       blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
 // A band's cells, one per thread at a time (a 256-row case lists about
@@ -815,7 +843,11 @@ hipError_t launch_lsq_fronts(const LsqWork& w, double* e1d, double* e2d, const d
   if ((e = hipGetLastError()) != hipSuccess) return e;
   lsq_factor_kernel<<<kLsqFactorBlocks, 256, 0, s>>>(w, e1d, e2d, z, 2 * nr, nz);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  lsq_solve_kernel<<<2, kLsqSolveThreads, 0, s>>>(w, e1d, e2d, z, 2 * nr, nz);
+  for (int k = 0; k < done; ++k) {
+    lsq_front_solve_kernel<<<dim3(kLsqFactorBlocks, 2), 256, 0, s>>>(w, e1d, e2d, z, 2 * nr, nz, k);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  lsq_solve_kernel<<<2, kLsqSolveThreads, 0, s>>>(w, e1d, e2d, z, 2 * nr, nz, done);
   return hipGetLastError();
 }
 
@@ -842,9 +874,16 @@ __global__ void __launch_bounds__(256) soft_batch_lsq_factor_kernel(
 }
 template <typename B>
 __global__ void __launch_bounds__(kLsqSolveThreads) soft_batch_lsq_solve_kernel(
-    const SoftCaseT<B>* __restrict__ cs) {
+    const SoftCaseT<B>* __restrict__ cs, int done) {
   const SoftCaseT<B>& C = cs[blockIdx.y];
-  lsq_solve_body(C.lw, blockIdx.x ? C.e2d : C.e1d, blockIdx.x != 0, C.z, 2 * C.nr, C.nz);
+  lsq_solve_body(C.lw, blockIdx.x ? C.e2d : C.e1d, blockIdx.x != 0, C.z, 2 * C.nr, C.nz, done);
+}
+template <typename B>
+__global__ void __launch_bounds__(256) soft_batch_lsq_front_solve_kernel(
+    const SoftCaseT<B>* __restrict__ cs, int front) {
+  const SoftCaseT<B>& C = cs[blockIdx.z];
+  lsq_front_solve_body(C.lw, blockIdx.y ? C.e2d : C.e1d, blockIdx.y != 0, C.z, 2 * C.nr, C.nz,
+                       front, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
 template <typename B>
@@ -861,7 +900,12 @@ hipError_t launch_soft_batch_lsq(const SoftCaseT<B>* cases, const SoftBatchDims&
   if ((e = hipGetLastError()) != hipSuccess) return e;
   soft_batch_lsq_factor_kernel<B><<<dim3(kLsqFactorBlocks, d.ncase), 256, 0, s>>>(cases);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  soft_batch_lsq_solve_kernel<B><<<dim3(2, d.ncase), kLsqSolveThreads, 0, s>>>(cases);
+  for (int k = 0; k < done; ++k) {
+    soft_batch_lsq_front_solve_kernel<B>
+        <<<dim3(kLsqFactorBlocks, 2, d.ncase), 256, 0, s>>>(cases, k);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  soft_batch_lsq_solve_kernel<B><<<dim3(2, d.ncase), kLsqSolveThreads, 0, s>>>(cases, done);
   return hipGetLastError();
 }
 

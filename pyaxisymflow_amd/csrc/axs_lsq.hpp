@@ -36,10 +36,11 @@ constexpr int kLsqNever = 0x7fffffff;
 
 // A solid whose radius is this many cells or more is large: the first
 // kLsqFrontLaunches fronts of a step (a stiff solid's loop takes 9 to 13) are
-// found by launches of many workgroups, the others by one.  About there
-// one workgroup's walk no longer fits in LDS; us a step, one workgroup / the
-// launches: radius 205 cells (512 x 256) 52 / -, 410 (1024 x 512) 129 (380 on the
-// whole box) / 92, 1638 (4096 x 2048) 511 (4918) / 136.
+// found, and fitted, by launches of many workgroups, the others by one.  About
+// there one workgroup's walk no longer fits in LDS; us a step, one workgroup /
+// the launches: radius 205 cells (512 x 256) walk 52 / -, fits 71 / -; 410
+// (1024 x 512) 129 (380 on the whole box) / 92, 123 / 62; 1638 (4096 x 2048)
+// 511 (4918) / 136, 684 / 70.
 constexpr double kLsqLargeRadius = 224.0;
 constexpr int kLsqFrontLaunches = 12;
 static_assert(kLsqFrontLaunches % 2 == 0, "the known cells end in kb");
