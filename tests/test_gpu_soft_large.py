@@ -118,8 +118,9 @@ def step_us(nz, r_ball):
 
 
 # one workgroup that walked the whole box at every front: 2.83 at 1024, now 1.78; fits
-# of a front by one workgroup per component: 1.96 at 2048, now 1.51
-@pytest.mark.parametrize("nz,bar", [(1024, 2.2), (2048, 1.72)])
+# of a front by one workgroup per component: 1.96 at 2048, now 1.51; two
+# atomics on one line by every segment of the target rows: 1.46 at 4096, now 1.19
+@pytest.mark.parametrize("nz,bar", [(1024, 2.2), (2048, 1.72), (4096, 1.32)])
 def test_a_large_solid_costs_little_more(nz, bar):
     large, small = step_us(nz, 0.4), step_us(nz, 0.05)
     print(f"nz {nz}: {large:.0f} and {small:.0f} us per step", flush=True)
