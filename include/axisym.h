@@ -479,10 +479,11 @@ axs_status axs_soft_batch_remove(axs_soft_batch* b, int case_id);
 /* Queues nsteps steps of every case on `stream` (use_graph: captured after
  * each change of the case set, replayed). */
 axs_status axs_soft_batch_run(axs_soft_batch* b, int nsteps, int use_graph, void* stream);
-/* Cases, the most extrapolation sweeps a step has taken + 4 rounded up to 4
- * (at least 12), graph launches and captures so far (any pointer may be
- * null). */
-axs_status axs_soft_batch_info(const axs_soft_batch* b, int* ncase, int* queued_sweeps,
+/* Cases, the most extrapolation sweeps that fitted cells in one step of any
+ * case (as of the last run that has finished on its stream; 0 before), graph
+ * launches and captures so far (any pointer may be null).  Reads host memory
+ * alone and waits for nothing. */
+axs_status axs_soft_batch_info(const axs_soft_batch* b, int* ncase, int* most_sweeps,
                                int64_t* graph_launches, int64_t* captures);
 axs_status axs_soft_batch_destroy(axs_soft_batch* b);
 

@@ -286,11 +286,11 @@ __global__ void soft_lsq_back_kernel(double* __restrict__ e1, double* __restrict
 // queue > 0: steps whose loop takes `queue` sweeps or more are counted.
 __device__ __forceinline__ void soft_finalize_body(double* __restrict__ sc,
                                                    const unsigned* __restrict__ head, int queue,
-                                                   unsigned* __restrict__ need) {
+                                                   unsigned* __restrict__ most) {
   const unsigned used = head[1];  // sweeps that fitted cells
   if (queue > 0 && used >= (unsigned)queue) sc[kSsLsqUnconverged] = sc[kSsLsqUnconverged] + 1.0;
   sc[kSsLsqSweeps] = double(used);
-  if (need) atomicMax(need, used + 1u);  // sweeps the reference's loop takes
+  if (most) atomicMax(most, used);
   sc[kSsT] = sc[kSsT] + sc[kSsDt];
   sc[kSsIt] = sc[kSsIt] + 1.0;
 }
@@ -629,7 +629,13 @@ template <typename B>
 __global__ void soft_batch_finalize_kernel(const SoftCaseT<B>* __restrict__ cs) {
   if (threadIdx.x != 0) return;
   const SoftCaseT<B>& C = cs[blockIdx.x];
-  soft_finalize_body(C.scalars, C.lw.head, 0, C.need);
+  soft_finalize_body(C.scalars, C.lw.head, 0, C.most_sweeps);
+}
+
+// Ends a run: the most sweeps of a step so far, to the host's copy.
+__global__ void soft_batch_publish_kernel(const unsigned* __restrict__ most,
+                                          unsigned* __restrict__ host) {
+  *host = *most;
 }
 
 // Many soft cases stepped together: each pass of the step is one launch over
@@ -649,7 +655,9 @@ struct SoftBatchT {
   SoftCaseT<B>* d_cases = nullptr;
   std::vector<SoftCaseT<B>> h_cases;
   SoftBatchDims dims{};
-  unsigned* need = nullptr;  // most sweeps an extrapolation loop has taken (device)
+  // most sweeps that fitted cells in a step: on the device, and pinned as of
+  // the last finished run
+  unsigned *most = nullptr, *most_host = nullptr;
   static constexpr int kChunkSteps = 8;
   hipGraph_t graph = nullptr, chunk_graph = nullptr;
   hipGraphExec_t graph_exec = nullptr, chunk_exec = nullptr;
@@ -666,8 +674,12 @@ struct SoftBatchT {
     max_cases = cap;
     hipError_t e = hipMalloc(reinterpret_cast<void**>(&d_cases), sizeof(SoftCaseT<B>) * cap);
     if (e != hipSuccess) return e;
-    if ((e = hipMalloc(reinterpret_cast<void**>(&need), sizeof(unsigned))) != hipSuccess) return e;
-    if ((e = hipMemset(need, 0, sizeof(unsigned))) != hipSuccess) return e;
+    if ((e = hipMalloc(reinterpret_cast<void**>(&most), sizeof(unsigned))) != hipSuccess) return e;
+    if ((e = hipMemset(most, 0, sizeof(unsigned))) != hipSuccess) return e;
+    if ((e = hipHostMalloc(reinterpret_cast<void**>(&most_host), sizeof(unsigned),
+                           hipHostMallocDefault)) != hipSuccess)
+      return e;
+    *most_host = 0u;
     return hipMalloc(reinterpret_cast<void**>(&d_rcnt), 3 * sizeof(unsigned));
   }
 
@@ -686,14 +698,15 @@ struct SoftBatchT {
     (void)hipDeviceSynchronize();
     drop_graphs();
     for (Entry& c : cases) delete c.st;
-    if (need) (void)hipFree(need);
+    if (most) (void)hipFree(most);
+    if (most_host) (void)hipHostFree(most_host);
     if (d_cases) (void)hipFree(d_cases);
     if (d_blocks) (void)hipFree(d_blocks);
     if (d_rlist) (void)hipFree(d_rlist);
     if (d_rcnt) (void)hipFree(d_rcnt);
   }
 
-  static SoftCaseT<B> describe(const SoftStepperT<B>& S, unsigned* need) {
+  static SoftCaseT<B> describe(const SoftStepperT<B>& S, unsigned* most) {
     SoftCaseT<B> C{};
     const SoftConfig& g = S.cfg;
     C.nr = g.nr;
@@ -746,7 +759,7 @@ struct SoftBatchT {
     C.tr = S.tr;
     C.rw = S.rw;
     C.lw = S.lw;
-    C.need = need;
+    C.most_sweeps = most;
     C.zone = S.zone;
     const StokesPlan& P = *S.plan;
     C.any = P.any->args;
@@ -780,7 +793,7 @@ struct SoftBatchT {
     }
     for (const Entry& c : cases) {
       const SoftStepperT<B>& S = *c.st;
-      h_cases.push_back(describe(S, need));
+      h_cases.push_back(describe(S, most));
       const StokesPlan& P = *S.plan;
       dims.large_solid |= lsq_large(S.cfg.r_ball, S.cfg.dx);
       dims.max_nr = std::max(dims.max_nr, P.nr);
@@ -946,6 +959,13 @@ struct SoftBatchT {
     hipError_t e;
     if (table_dirty && (e = refresh()) != hipSuccess) return e;
     if (cases.empty() || nsteps == 0) return hipSuccess;
+    if ((e = steps(nsteps, use_graph, s)) != hipSuccess) return e;
+    soft_batch_publish_kernel<<<1, 1, 0, s>>>(most, most_host);
+    return hipGetLastError();
+  }
+
+  hipError_t steps(int nsteps, bool use_graph, hipStream_t s) {
+    hipError_t e;
     if (!use_graph) {
       for (int q = 0; q < nsteps; ++q)
         if ((e = enqueue_step(s)) != hipSuccess) return e;
@@ -1155,18 +1175,12 @@ axs_status axs_soft_batch_run(axs_soft_batch* bt, int nsteps, int use_graph, voi
   return AXS_OK;
 }
 
-axs_status axs_soft_batch_info(const axs_soft_batch* bt, int* ncase, int* queued_sweeps,
+axs_status axs_soft_batch_info(const axs_soft_batch* bt, int* ncase, int* most_sweeps,
                                int64_t* graph_launches, int64_t* captures) {
   AXS_CHECK_ARG(bt, "null batch");
-  if (queued_sweeps) {
-    unsigned need = 0u;
-    AXS_HIP(bt->with([&](const auto& b) {
-      return hipMemcpy(&need, b.need, sizeof(unsigned), hipMemcpyDeviceToHost);
-    }));
-    *queued_sweeps = std::max(12, (int)((need + 4u + 3u) / 4u * 4u));
-  }
   bt->with([&](const auto& b) {
     if (ncase) *ncase = (int)b.cases.size();
+    if (most_sweeps) *most_sweeps = (int)__atomic_load_n(b.most_host, __ATOMIC_RELAXED);
     if (graph_launches) *graph_launches = b.chunk_launches + b.step_launches;
     if (captures) *captures = b.captures;
     return 0;

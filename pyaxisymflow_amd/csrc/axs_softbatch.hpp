@@ -57,7 +57,7 @@ struct SoftCaseT {
   ReinitWork rw;
   int reinit_tile_base;  // the case's first entry in the batch's reinit tile table
   LsqWork lw;
-  unsigned* need;
+  unsigned* most_sweeps;  // the batch's: most sweeps that fitted cells in a step
   // rows [zone[0], zone[1]] hold the step's extrapolation target zone,
   // [zone[2], zone[3]] the previous step's
   int* zone;

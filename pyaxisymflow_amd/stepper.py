@@ -870,9 +870,10 @@ class SoftSphereBatch:
         self.stream.synchronize()
 
     def info(self):
-        """(cases, an upper figure for the extrapolation sweeps of a step,
-        graph launches, graph captures).  The sweeps figure is the most any
-        step has taken + 4, rounded up to 4, and at least 12."""
+        """(cases, the most extrapolation sweeps that fitted cells in one
+        step of any case, graph launches, graph captures).  The sweeps are as
+        of the last ``step`` call that has finished on the batch's stream;
+        nothing is waited for."""
         n, q = ctypes.c_int(), ctypes.c_int()
         g, c = ctypes.c_int64(), ctypes.c_int64()
         _lib.call("axs_soft_batch_info", self._h, ctypes.byref(n), ctypes.byref(q),
