@@ -352,7 +352,7 @@ axs_status axs_rigid_stepper_create(const axs_rigid_config* cfg, const axs_rigid
  * batch = 1.
  *
  * Uneven batches: cases may also differ in nr, nz and dx when none has a
- * moving body, every nz <= 1024, and the cases come in at most 16 runs of
+ * moving body, every nz even and <= 1024, and the cases come in at most 16 runs of
  * one grid.  Every pass is then one launch over all cases.  Fields hold
  * case q's nr_q * nz_q elements after those of cases 0..q-1; r holds each
  * case's nr_q radii back to back, kill_wz each case's 2 kill_width

@@ -306,10 +306,12 @@ static bool same_grid(const RigidConfig& a, const RigidConfig& b) {
   return a.nr == b.nr && a.nz == b.nz && a.dx == b.dx;
 }
 
-// Radix plan of the half-length transform (radices 4, 2, 3, 5); false if
-// nz / 2 has another prime factor.
+// Radix plan of the half-length transform (radices 4, 2, 3, 5); false if nz
+// is odd (its rows would be taken as nz - 1 columns) or nz / 2 has another
+// prime factor.
 static bool fft_args(int nz, FftPlanArgs& fp) {
   fp = FftPlanArgs{};
+  if (nz % 2) return false;
   fp.M = nz / 2;
   int m = fp.M;
   for (int rdx : {4, 2, 3, 5})
@@ -754,8 +756,8 @@ axs_status axs_rigid_batch_create(const axs_rigid_config* cfgs, int batch,
     AXS_CHECK_ARG(runs <= kMaxRaggedGroups,
                   "a batch of uneven grids takes at most 16 runs of one grid (order the cases)");
     for (int q = 0; q < batch; ++q)
-      AXS_CHECK_ARG(cfgs[q].nz <= 1024 && cfgs[q].nr <= 4096,
-                    "a batch of uneven grids takes nz <= 1024 and nr <= 4096");
+      AXS_CHECK_ARG(cfgs[q].nz <= 1024 && cfgs[q].nz % 2 == 0 && cfgs[q].nr <= 4096,
+                    "a batch of uneven grids takes even nz <= 1024 and nr <= 4096");
   }
   if (c0.implicit_diffusion) {
     AXS_CHECK_ARG(!uneven && c0.precision == AXS_F64,

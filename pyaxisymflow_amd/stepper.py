@@ -351,7 +351,8 @@ class UnevenBatchStepper(_Checkpoint):
 
     ``cases`` is a list of dicts, each with the case's grid -- ``nz``,
     ``nr``, ``z_len`` and optionally ``r_len`` -- and the per-case arguments
-    of ``RigidBodyStepper`` (no ``moving_body``; nz <= 1024).  Cases are
+    of ``RigidBodyStepper`` (no ``moving_body``; with more than one grid even
+    nz <= 1024, nz / 2 a product of twos, threes and fives).  Cases are
     stored grouped by grid (at most 16 grids); accessors take the caller's
     case index and return that case's (nr, nz) arrays.  Every case keeps its
     own t, dt and force history.
