@@ -38,7 +38,9 @@ struct AnyDftArgs {
 struct AnyDft {
   AnyDftArgs args{};
   // the length-L FFT's launch shape (nth threads, PER of fft_lds plus
-  // kFftWide) for many rows, and for rows that each have a CU to themselves
+  // kFftWide) for many rows, and for rows that each have a CU to themselves;
+  // by the rows of one case, also in a batch: a row's rounding depends on PER,
+  // and the order of the force sum on the threads
   struct Shape {
     int nth = 64, per = 1;
   };

@@ -624,9 +624,7 @@ hipError_t launch_any_dct2_rows(const StokesPlan& pl, const T* src, T* tapered, 
   const StepFinalize f = fin ? *fin : StepFinalize{};
   const dim3 grid(pl.nr + (f.partials ? 1 : 0), batch);
   const size_t shm = D.lds_bytes<T>();
-  // the completed step's force is summed in an order that depends on the
-  // threads: one shape for a case alone and in a batch
-  const AnyDft::Shape h = D.shape(f.partials ? pl.nr : pl.nr * batch);
+  const AnyDft::Shape h = D.shape(pl.nr);
   if (taper)
     AXS_ANY_PER(h.per, (any_dct2_rows_kernel<T, P, true><<<grid, h.nth, shm, s>>>(
                        src, tapered, dst, rscale, wz, wr, pl.nr, pl.nz, w, tb, f)));
@@ -641,7 +639,7 @@ hipError_t launch_any_dct3_rows(const StokesPlan& pl, const T* src, T* dst, int 
                                 hipStream_t s) {
   const AnyDft& D = *pl.any;
   const AnyDctTables tb{D.args, pl.ge2, pl.e1, pl.e2, pl.any_half ? 1 : 0};
-  const AnyDft::Shape h = D.shape(rows * batch);
+  const AnyDft::Shape h = D.shape(rows);
   AXS_ANY_PER(h.per, (any_dct3_rows_kernel<T, P><<<dim3(rows, batch), h.nth, D.lds_bytes<T>(), s>>>(
                      src, dst, rows, pl.nz, tb)));
   return hipGetLastError();
@@ -661,10 +659,10 @@ hipError_t launch_any_rfft_rows(const StokesPlan& pl, const double* src, double*
 }
 
 hipError_t launch_any_dst1_rows(const AnyDft& D, const Cplx<double>* em, const double* src,
-                                double* dst, int rows, int nz, hipStream_t s) {
+                                double* dst, int rows, int batch, int nz, hipStream_t s) {
   const double norm = std::sqrt(2.0 / (double)(nz + 1)) / 4.0;
   const AnyDft::Shape h = D.shape(rows);
-  AXS_ANY_PER(h.per, (any_dst1_rows_kernel<P><<<rows, h.nth, D.lds_bytes<double>(), s>>>(
+  AXS_ANY_PER(h.per, (any_dst1_rows_kernel<P><<<rows * batch, h.nth, D.lds_bytes<double>(), s>>>(
                      src, dst, nz, D.args, em, norm)));
   return hipGetLastError();
 }

@@ -80,10 +80,9 @@ hipError_t ImplicitPlan::init(int nr, int nz, double dx, double nu_dt_, int batc
 }
 
 hipError_t ImplicitPlan::launch(double* omega, int batch, hipStream_t s) {
-  const int rows = tri.nr * batch;
-  hipError_t e = launch_any_dst1_rows(dst, em, omega, tri.spec, rows, tri.nz, s);
+  hipError_t e = launch_any_dst1_rows(dst, em, omega, tri.spec, tri.nr, batch, tri.nz, s);
   if (e == hipSuccess) e = launch_tridiag<double>(tri, tri.spec, s, batch);
-  if (e == hipSuccess) e = launch_any_dst1_rows(dst, em, tri.spec, omega, rows, tri.nz, s);
+  if (e == hipSuccess) e = launch_any_dst1_rows(dst, em, tri.spec, omega, tri.nr, batch, tri.nz, s);
   return e;
 }
 

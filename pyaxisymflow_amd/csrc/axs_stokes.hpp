@@ -126,10 +126,10 @@ hipError_t launch_any_dct3_rows(const StokesPlan& pl, const T* src, T* dst, int 
                                 hipStream_t s);
 hipError_t launch_any_rfft_rows(const StokesPlan& pl, const double* src, double* dst,
                                 const double* rscale, int rows, bool inverse, hipStream_t s);
-// Orthonormal DST-I of `rows` rows of nz (D of length nz + 1, em[k] =
-// e^{-i pi k / (nz + 1)}, k <= nz); src and dst must not alias.
+// Orthonormal DST-I of `rows` rows of nz of each of `batch` cases (D of length
+// nz + 1, em[k] = e^{-i pi k / (nz + 1)}, k <= nz); src and dst must not alias.
 hipError_t launch_any_dst1_rows(const AnyDft& D, const Cplx<double>* em, const double* src,
-                                double* dst, int rows, int nz, hipStream_t s);
+                                double* dst, int rows, int batch, int nz, hipStream_t s);
 // Largest nz a plan takes: the half-length transforms cover nz <= 8192 with
 // nz / 2 2,3,5-smooth; the any-length ones need their FFT length <= kAnyMaxL.
 bool stokes_nz_supported(int nz);

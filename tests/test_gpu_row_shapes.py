@@ -10,6 +10,7 @@ compute unit, of 3375 against 3125 points 1.13 (1.41), of 4000 against 4096
 points 0.97 (1.09)."""
 import time
 
+import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -44,3 +45,32 @@ def test_long_rows_take_what_their_length_explains(monkeypatch, nr, points, othe
     a, b = step_us(points, nr), step_us(other, nr)
     print(f"{nr} rows: {points} points {a:.1f} us, {other} points {b:.1f} us", flush=True)
     assert a / b < bar
+
+
+@pytest.mark.parametrize("implicit", [False, True])
+def test_a_case_keeps_its_bits_in_a_batch(implicit):
+    """96 rows alone, 384 in a batch of four: rows of 2518 points (cosine, FFTs of
+    2700) and of 1258 (sine, the same) have one shape for few rows and another
+    for many, and a row's rounding depends on it."""
+    from pyaxisymflow_amd import workloads
+    from pyaxisymflow_amd.stepper import RigidBatchStepper, RigidBodyStepper
+
+    nz, nr = (1258, 96) if implicit else (2518, 96)
+    args = []
+    for seed in (0, 1):
+        sp = workloads.case_spec(seed)
+        sp.update(nz=nz, nr=nr)
+        a = workloads.rigid_case_args(sp, workloads.case_inputs(sp, nz, nr)[1])
+        if implicit:
+            a.update(nu=1e-3, implicit_diffusion=True)
+        args.append(a)
+    cases = [args[q % 2] for q in range(4)]
+    print(f"{nz} x {nr}, implicit {implicit}", flush=True)
+    many = RigidBatchStepper(nz, nr, 1.0, cases, r_len=nr / nz)
+    many.step(4)
+    for q in (0, 3):
+        one = RigidBodyStepper(nz, nr, 1.0, r_len=nr / nz, **cases[q])
+        one.step(4)
+        assert np.isfinite(one.vorticity()).all()
+        assert np.array_equal(many.vorticity(q), one.vorticity())
+        assert np.array_equal(many.drag_history(q), one.drag_history())
