@@ -13,9 +13,9 @@ two Poisson routes (exact vs the reference's eig route) differ by 1.1e-7 in
 omega after 12 steps.  Bars: after one step every field within 1e-12
 relative L2 (dt within 1e-12); after 12 steps every field no further from
 the oracle's exact route than twice the oracle's exact-vs-eig spread.  The
-smooth Heaviside's sin() is the device's, within an ulp of numpy's.  A
-loop longer than the queued extrapolation sweeps, finished by one
-workgroup, gives the same bits as one that fits in them.
+smooth Heaviside's sin() is the device's, within an ulp of numpy's.  The
+extrapolation of a deformed solid, whose loop is long, is the oracle's loop
+bit for bit, sweep count included.
 """
 import numpy as np
 import pytest
@@ -72,7 +72,7 @@ def test_soft_one_step_matches_oracle():
           "sweeps", gpu.lsq_sweeps_last(), flush=True)
     assert gpu.steps_done() == 1
     assert abs(gpu.dt() - cpu.dts[-1]) <= 1e-12 * cpu.dts[-1]
-    assert gpu.lsq_unconverged() == 0 and gpu.lsq_sweeps_last() >= 1
+    assert gpu.lsq_sweeps_last() >= 1
     for k, v in errs.items():
         assert v < 1e-12, k
 
@@ -94,7 +94,6 @@ def test_soft_12_steps_within_oracle_route_spread():
         print(f"soft {steps} steps {k}: gpu {got:.2e} oracle routes {spread:.2e}", flush=True)
         assert got <= 2 * spread + 1e-14, k
     assert abs(gpu.time() - exact.t) <= 1e-12 * exact.t
-    assert gpu.lsq_unconverged() == 0
 
 
 def test_soft_graph_equals_eager():
@@ -115,40 +114,59 @@ def test_soft_graph_equals_eager():
     assert np.array_equal(a.scalars(), b.scalars())
 
 
-@pytest.mark.parametrize("queued", [4, 5])
-def test_soft_tail_finishes_the_loop(queued):
-    """With fewer queued sweeps than the loop needs (18-19 here), the
-    one-workgroup tail carries the loop on: every field and scalar but the
-    tail-step counter equals the run with the default 48, bit for bit, for
-    an even and an odd count (the result returns to the right buffer set)."""
+@pytest.mark.parametrize("sweeps,counted", [(4, 10), (64, 0)])
+def test_soft_lsq_sweeps_only_counts_steps(sweeps, counted):
+    """``lsq_sweeps`` counts the steps whose loop takes that many sweeps or
+    more (8 to 19 here) and changes nothing else."""
     from pyaxisymflow_amd.stepper import SoftSphereStepper
 
-    a = SoftSphereStepper(grid_size_z=128, lsq_sweeps=queued)
+    a = SoftSphereStepper(grid_size_z=128, lsq_sweeps=sweeps)
     b = SoftSphereStepper(grid_size_z=128)
     a.step(10)
     b.step(10)
-    assert a.lsq_unconverged() == 10 and b.lsq_unconverged() == 0
-    assert a.lsq_sweeps_last() == b.lsq_sweeps_last() > queued
+    assert a.lsq_unconverged() == counted
+    assert 4 <= a.lsq_sweeps_last() == b.lsq_sweeps_last() < 64
     assert np.array_equal(a.vorticity(), b.vorticity())
     assert np.array_equal(a.phi(), b.phi())
     ea, eb = a.eta(), b.eta()
     assert np.array_equal(ea[0], eb[0]) and np.array_equal(ea[1], eb[1])
 
 
-def test_soft_growing_queue_equals_fixed():
-    """The default stepper starts with 12 queued sweeps and grows the queue
-    (re-capturing its graphs) as steps need more; over 200 steps every field
-    equals a stepper with a fixed queue of 64, bit for bit."""
+def test_soft_long_loop_is_the_oracle_s():
+    """A soft solid (G = 0.1) after 800 steps, whose loop takes more sweeps
+    than the first steps': from the GPU's own state before and velocity and
+    dt of the next step, the oracle's reference-map ENO3, pin, reinit and
+    sweep loop give the same phi, eta and sweep count."""
+    from oracle import kernels as K
+    from oracle.lsq import extrapolate_using_least_squares_till_first_order
+    from oracle.reinit import distance
     from pyaxisymflow_amd.stepper import SoftSphereStepper
 
-    a = SoftSphereStepper(grid_size_z=128, G=0.1)
-    b = SoftSphereStepper(grid_size_z=128, G=0.1, lsq_sweeps=64)
-    for _ in range(4):
-        a.step(50)
-        b.step(50)
-    assert b.lsq_unconverged() == 0
-    assert a.lsq_sweeps_last() == b.lsq_sweeps_last()
-    assert np.array_equal(a.vorticity(), b.vorticity())
-    assert np.array_equal(a.phi(), b.phi())
-    ea, eb = a.eta(), b.eta()
-    assert np.array_equal(ea[0], eb[0]) and np.array_equal(ea[1], eb[1])
+    cpu = SoftSphereCase(grid_size_z=128, G=0.1, solver="exact")
+    gpu = SoftSphereStepper(grid_size_z=128, G=0.1)
+    gpu.step(1)
+    first = gpu.lsq_sweeps_last()
+    gpu.step(800)
+    e1, e2 = gpu.eta()
+    old = gpu.phi()
+    gpu.step(1)
+    u_z, u_r = gpu.velocity()
+    dx = cpu.dx
+    K.advect_refmap_via_eno3(e1, e2, u_z, u_r, gpu.dt(), dx)
+    pinned = -np.sqrt((e1 - cpu.Z_cm) ** 2 + (e2 - cpu.R_cm) ** 2) + cpu.r_ball
+    phi = np.where(old > -3 * dx, pinned, old)
+    d, masked = distance(phi, dx, cpu.reinit_band)
+    phi = np.where(masked, phi, d)
+    assert np.array_equal(gpu.phi(), phi)
+    # extrapolate_eta_using_least_squares_unb.py:19-30 on the doubled grid
+    chi = 0 * phi
+    K.smooth_Heaviside(chi, phi, cpu.moll_zone)
+    a, b = (chi > 0.5) * e1, (chi > 0.5) * e2
+    level = -np.concatenate([phi[::-1], phi])
+    a, b = np.concatenate([a[::-1], a]), np.concatenate([-b[::-1], b])
+    sweeps = extrapolate_using_least_squares_till_first_order(
+        (level < 0).astype(np.int16), (level < cpu.extrap_zone).astype(np.int16), a, b, cpu.z,
+        cpu.z)
+    g1, g2 = gpu.eta()
+    assert np.array_equal(g1, a[cpu.nr:]) and np.array_equal(g2, b[cpu.nr:])
+    assert gpu.lsq_sweeps_last() == sweeps > first

@@ -67,7 +67,6 @@ def test_batch_case_one_step_matches_oracle():
     sc = case.scalars()
     assert case.steps_done() == 1
     assert abs(sc[1] - cpu.dts[-1]) <= 1e-12 * cpu.dts[-1]
-    assert case.lsq_unconverged() == 0
     for k, v in errs.items():
         assert v < 1e-12, k
 
@@ -88,7 +87,6 @@ def test_batch_long_rows_one_step_match_oracle(precision, bar):
         errs = {k: rel_l2(np.asarray(g[k], np.float64), c[k]) for k in c}
         print(f"soft batch {precision} nz {nz}: " + " ".join(f"{k} {v:.2e}" for k, v in errs.items()),
               flush=True)
-        assert case.lsq_unconverged() == 0
         for k, v in errs.items():
             assert v < bar, (nz, k)
 
@@ -114,7 +112,6 @@ def test_batch_case_12_steps_within_oracle_route_spread():
         print(f"soft batch {steps} steps {k}: gpu {got:.2e} oracle routes {spread:.2e}", flush=True)
         assert got <= 2 * spread + 1e-14, k
     assert abs(case.time() - exact.t) <= 1e-12 * exact.t
-    assert case.lsq_unconverged() == 0
 
 
 @pytest.mark.parametrize("precision", ["f64", "f32"])
@@ -168,8 +165,8 @@ def test_batch_join_leave_between_runs():
     b.step(9)
     _assert_same_bits(a, x, "join/leave")
     assert late.steps_done() == 9 and x.steps_done() == 14
-    n, queued, launches, captures = b.info()
-    print(f"soft batch info: cases {n} queued sweeps {queued} graph launches {launches} "
+    n, sweeps, launches, captures = b.info()
+    print(f"soft batch info: cases {n} most sweeps {sweeps} graph launches {launches} "
           f"captures {captures}", flush=True)
     assert n == 2 and captures >= 2
 
