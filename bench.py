@@ -396,7 +396,6 @@ def time_serving(n_requests, steps, max_active=32, seed=0, precision="f32", open
         return dict(closed_loop_wall_s=round(t_closed, 3),
                     closed_loop_mcell_steps_per_s=round(cells / t_closed / 1e6, 2),
                     capacity_requests_per_s=round(capacity, 3),
-                    lsq_tail_steps=int(sum(r["lsq_unconverged"] for r in recs)),
                     failed_requests=failed, precision=precision)
     rate = 0.8 * capacity
     open_set = request_set(n_requests, seed=seed, rate=rate, steps=steps)
@@ -414,10 +413,8 @@ def time_serving(n_requests, steps, max_active=32, seed=0, precision="f32", open
         closed_loop_wall_s=round(t_closed, 3),
         closed_loop_mcell_steps_per_s=round(cells / t_closed / 1e6, 2),
         failed_requests=failed + s["failed"],
-        # steps whose extrapolation loop took the given number of sweeps or
-        # more (results do not depend on it)
-        lsq_tail_steps=int(sum(r["lsq_unconverged"] for r in recs + recs2)),
-        queued_lsq_sweeps=srv.last_batch_info[1] if srv.last_batch_info else None,
+        # most extrapolation sweeps that fitted cells in a step of the last run
+        most_lsq_sweeps=srv.last_batch_info[1] if srv.last_batch_info else None,
         precision=precision,
     )
 
