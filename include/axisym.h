@@ -446,8 +446,9 @@ axs_status axs_soft_stepper_run(axs_soft_stepper* st, int nsteps, int use_graph,
  * gives the same bits alone and in any mix.  Cases join (add) and leave
  * (remove) between runs; both wait for the device to finish queued work.
  * The configuration and buffers are those of axs_soft_stepper_create
- * (lsq_sweeps and lsq_grow are not used); the buffers must stay valid until the case is
- * removed.  At most 1024 cases; nz up to 4096 (nr up to 2048). */
+ * (lsq_sweeps and lsq_grow are not used); the buffers must stay valid until
+ * the case is removed.  At most 1024 cases; every nr up to 1281 (nz = 2 nr; the
+ * radial pass keeps a grid's coefficients in LDS, taller ones are refused). */
 typedef struct axs_soft_batch axs_soft_batch;
 axs_status axs_soft_batch_create(int max_cases, axs_soft_batch** out);
 axs_status axs_soft_batch_add(axs_soft_batch* b, const axs_soft_config* cfg,

@@ -7,11 +7,12 @@
 // approach to the computation of discrete Fourier transform", IEEE Trans.
 // Audio Electroacoust. 18(4), 1970): with w_n = e^{-i pi n^2 / N},
 //   X_k = sum_n v_n e^{-2 pi i n k / N} = w_k sum_n (v_n w_n) conj(w_{k-n}),
-// a circular convolution of 2,3,5-smooth length L >= 2N - 1, computed by two length-L FFTs and a pointwise product with
-// bhat = FFT_L(b) / L, b_m = conj(w_m) for |m| < N (m taken mod L), which
-// the plan computes once on the device.  The chirp angle is reduced as
-// pi (n^2 mod 2N) / N on the host so that it stays exact for large n.  The
-// inverse direction (exponent +1) uses conj(w) and conj(bhat_{-k}).
+// a circular convolution of 2,3,5-smooth length L >= 2N - 1, computed by two
+// length-L FFTs and a pointwise product with bhat = FFT_L(b) / L, b_m =
+// conj(w_m) for |m| < N (m taken mod L), which the plan computes once on the
+// device.  The chirp angle is reduced as pi (n^2 mod 2N) / N on the host so
+// that it stays exact for large n.  The inverse direction (exponent +1) uses
+// conj(w) and conj(bhat_{-k}).
 #pragma once
 
 #include "axs_fft.hpp"
@@ -55,9 +56,11 @@ struct AnyDft {
 };
 
 // Radices 7, 8, 11 and 13 are kept out of the kernels of plans without them:
-// with them a row's kernel takes 112-128 registers instead of 48-74 at
-// PER <= 2, which halves the waves in flight (the implicit step at 1024 x 512,
-// chirp-z rows of 1025: 92 us with them, 70 without).
+// with them an FP64 row's kernel takes 112-128 registers, four waves per
+// SIMD; without, 46-54 at PER = 1 (eight; seven where it takes more than 80
+// scalar ones) and 74 at PER = 2 (six; the inverse cosine rows 120 and four),
+// 128 at PER = 4.  The implicit step at 1024 x 512, chirp-z rows of 1025: 92 us
+// with them, 70 without.
 constexpr int kFftWide = 8;
 inline bool fft_wide(const AnyDftArgs& a) {
   for (int s = 0; s < a.fp.nstages; ++s)
@@ -101,7 +104,8 @@ template <typename T, int PER>
 __device__ __forceinline__ void any_fft(Cplx<T>* work, const AnyDftArgs& a, int sgn, int tid,
                                         int nth) {
   if (a.stage)
-    fft_lds<T, PER & 7, (PER & kFftWide) != 0>(work, a.fp, static_cast<const Cplx<T>*>(work + a.L), sgn, tid, nth);
+    fft_lds<T, PER & 7, (PER & kFftWide) != 0>(
+        work, a.fp, static_cast<const Cplx<T>*>(work + a.L), sgn, tid, nth);
   else
     fft_lds<T, PER & 7, (PER & kFftWide) != 0>(work, a.fp, a.tw, sgn, tid, nth);
 }

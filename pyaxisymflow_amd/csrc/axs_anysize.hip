@@ -70,8 +70,9 @@ static int stages_twiddles(int L) { return 2 * sizeof(Cplx<double>) * (size_t)L 
 // Threads of a row of more than 1920 points when there are many: the PER that
 // keeps the most threads in flight on a CU (rows by its 160 KiB of LDS and by
 // the waves per SIMD that the registers of PER = 1, 2, 4 and of the wide
-// radices allow), the smallest where that is equal, but PER = 4 where it
-// holds more rows than PER = 2.  Whole multiples of 256 threads: a row's
+// radices allow; the inverse cosine rows at PER = 2 hold four, not six), the
+// smallest where that is equal, but PER = 4 where it holds more rows than
+// PER = 2.  Whole multiples of 256 threads: a row's
 // waves spread evenly over the four SIMDs, where 5 or 6 waves leave room for
 // one row less than their number says.  us per step of 1024 rows, sine rows
 // of L points (a quarter, half, three quarters, all of 1024 threads): 2160

@@ -806,8 +806,9 @@ __global__ void __launch_bounds__(256) lsq_factor_kernel(LsqWork w, const double
   lsq_factor_body(w, ex, ey, g, n0, n1, blockIdx.x * blockDim.x + threadIdx.x,
                   gridDim.x * blockDim.x);
 }
-// 512 threads: a front has a few hundred cells, and two records in flight
-// need more than the 128 registers that 1024 threads would leave.
+// 512 threads: a front has a few hundred cells, and the barrier after it
+// costs more with 1024 (256 x 128: 19 us a step, 23 with 1024; the widest
+// fronts that are left to it, a solid of 205 cells' radius: 74, 71).
 constexpr int kLsqSolveThreads = 512;
 __global__ void __launch_bounds__(kLsqSolveThreads) lsq_solve_kernel(LsqWork w, double* ex,
                                                                      double* ey,
@@ -823,7 +824,8 @@ __global__ void __launch_bounds__(256) lsq_front_solve_kernel(LsqWork w, double*
 }
 
 // A band's cells, one per thread at a time (a 256-row case lists about
-// 5,000).
+// 5,000).  The factor pass takes 238 registers, one wave per SIMD: a
+// workgroup has its CU alone, and twelve cases' 768 run three to a CU in turn.
 constexpr int kLsqFactorBlocks = 64;
 
 // Workgroups of a front of lsq_front_levels_body over a doubled grid.

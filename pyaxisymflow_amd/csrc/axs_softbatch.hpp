@@ -35,7 +35,7 @@ enum : int {
   kSsMaxU,            // max(|u_z| + |u_r|)
   kSsIt,              // step counter
   kSsLsqSweeps,       // sweeps that fitted cells in the last step
-  kSsLsqUnconverged,  // steps whose last allowed sweep still fitted cells
+  kSsLsqUnconverged,  // steps whose loop took lsq_sweeps sweeps or more (single case, no lsq_grow)
   kSsFreqTimer,       // streaming: time since the cycle timer last reset
   kSsUwall,           // streaming: tethered core's velocity U_0 cos(omega t)
   kSsZtether,         // streaming: tethered core's centre Z_cm + e r_ball sin(omega t)

@@ -748,6 +748,7 @@ class SoftSphereStepper(_Checkpoint):
         return int(self.scalars()[SS_LSQ_SWEEPS])
 
     def lsq_unconverged(self):
+        """Steps whose loop took ``lsq_sweeps`` sweeps or more (0 without it)."""
         return int(self.scalars()[SS_LSQ_UNCONVERGED])
 
     def __del__(self):
@@ -807,6 +808,7 @@ class _SoftCaseView(_Checkpoint):
         return int(self.scalars()[SS_IT])
 
     def lsq_unconverged(self):
+        """0: a batch counts no steps (SoftSphereStepper's ``lsq_sweeps``)."""
         return int(self.scalars()[SS_LSQ_UNCONVERGED])
 
 
