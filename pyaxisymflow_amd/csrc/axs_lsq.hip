@@ -394,20 +394,30 @@ __device__ __forceinline__ void lsq_levels_body(const LsqWork& w, int nr, int nz
     s_m = 0u;
   }
   __syncthreads();
-  // word columns with target cells, from the box's rows of words as they
-  // lie (whole groups of four; a row's words beyond nz are 0)
+  // word columns with target cells: a word per thread, or, of more rows than
+  // fit in LDS whole, groups of four words as they lie (a row's words beyond
+  // nz are 0)
   const int G = w.wstride / 4, ng = rows * G;
   const uint4* tb4 = reinterpret_cast<const uint4*>(w.tb + (int64_t)r0 * w.wstride);
   const uint4* kb4 = reinterpret_cast<const uint4*>(w.kb + (int64_t)r0 * w.wstride);
   int lo = W, hi = -1;
+  if (rows * W <= kLsqLdsWords) {
+    for (int q = tid; q < rows * W; q += kLsqThreads) {
+      const int r = (int)((unsigned)q / (unsigned)W), c = q - r * W;
+      if (w.tb[(int64_t)(r0 + r) * w.wstride + c]) {
+        lo = min(lo, c);
+        hi = max(hi, c);
+      }
+    }
+  } else {
 #pragma unroll 4
-  for (int q = tid; q < ng; q += kLsqThreads) {
-    const uint4 t = tb4[q];
-    const int c = (int)((unsigned)q % (unsigned)G) * 4;
-    const unsigned any =
-        (t.x ? 1u : 0u) | (t.y ? 2u : 0u) | (t.z ? 4u : 0u) | (t.w ? 8u : 0u);
-    lo = any ? min(lo, c + __ffs((int)any) - 1) : lo;
-    hi = any ? max(hi, c + 31 - __clz((int)any)) : hi;
+    for (int q = tid; q < ng; q += kLsqThreads) {
+      const uint4 t = tb4[q];
+      const int c = (int)((unsigned)q % (unsigned)G) * 4;
+      const unsigned any = (t.x ? 1u : 0u) | (t.y ? 2u : 0u) | (t.z ? 4u : 0u) | (t.w ? 8u : 0u);
+      lo = any ? min(lo, c + __ffs((int)any) - 1) : lo;
+      hi = any ? max(hi, c + 31 - __clz((int)any)) : hi;
+    }
   }
   if (hi >= 0) {
     atomicMin(&s_w0, lo);
