@@ -59,7 +59,8 @@ __host__ __device__ constexpr int lsq_factor_cap(int64_t n) { return int(n / 16 
 
 // Extrapolates (e1d, e2d) of a case whose known cells are all targets: the
 // reference's loop (core/src/extrapolate_using_least_squares.hpp:142-446),
-// bit for bit, in three launches.  z: coordinates of both axes.  zone[1]:
+// bit for bit, in three launches (and 2 kLsqFrontLaunches more of a large
+// solid).  z: coordinates of both axes.  zone[1]:
 // the last physical row with a target cell, -1 if none.
 hipError_t launch_lsq_fronts(const LsqWork& w, double* e1d, double* e2d, const double* z, int nr,
                              int nz, const int* zone, bool large, hipStream_t s);
