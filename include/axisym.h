@@ -477,6 +477,10 @@ axs_status axs_soft_batch_create_f32(int max_cases, axs_soft_batch** out);
 axs_status axs_soft_batch_add_f32(axs_soft_batch* b, const axs_soft_config* cfg,
                                   const axs_soft_buffers_f32* bufs, int* case_id);
 axs_status axs_soft_batch_remove(axs_soft_batch* b, int case_id);
+/* To be called after the caller has written another state into the buffers of
+ * a case (waits for queued work): a step visits the rows of the case's last
+ * zone and a margin, and after this its next step visits every row. */
+axs_status axs_soft_batch_state_loaded(axs_soft_batch* b, int case_id);
 /* Queues nsteps steps of every case on `stream` (use_graph: captured after
  * each change of the case set, replayed). */
 axs_status axs_soft_batch_run(axs_soft_batch* b, int nsteps, int use_graph, void* stream);

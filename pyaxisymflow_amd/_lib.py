@@ -185,6 +185,7 @@ SIGNATURES = {
     "axs_soft_batch_add_f32": [_P, ctypes.POINTER(SoftConfig), ctypes.POINTER(SoftBuffersF32),
                                _P],
     "axs_soft_batch_remove": [_P, _I],
+    "axs_soft_batch_state_loaded": [_P, _I],
     "axs_soft_batch_run": [_P, _I, _I, _P],
     "axs_soft_batch_info": [_P, _P, _P, _P, _P],
     "axs_soft_batch_destroy": [_P],

@@ -343,6 +343,14 @@ struct SoftStepperT {
   // single-case step keeps zone[1] alone, the zone's last row
   int* zone = nullptr;
 
+  // The zone a case starts with, and has again once another state is loaded:
+  // every row, so that its next step in a batch visits the whole grid (its
+  // flags and values are written nowhere else before it).
+  hipError_t all_rows() {
+    const int rows[4] = {0, cfg.nr - 1, 0, cfg.nr - 1};
+    return hipMemcpy(zone, rows, sizeof(rows), hipMemcpyHostToDevice);
+  }
+
   template <typename P>
   hipError_t alloc(P** p, size_t bytes) {
     void* q = nullptr;
@@ -399,13 +407,8 @@ struct SoftStepperT {
     if ((e = alloc(&lw.cnt, kLsqFrontLaunches * sizeof(unsigned))) != hipSuccess) return e;
     if ((e = alloc(&lw.win, nd * sizeof(unsigned))) != hipSuccess) return e;
     if ((e = alloc(&lw.fac, 9 * (size_t)lw.fcap * D8)) != hipSuccess) return e;
-    // every row: the first step a case takes here visits the whole grid
-    // (its flags and values are written nowhere else before it), also when
-    // its state was loaded from another run
-    const int all_rows[4] = {0, cfg.nr - 1, 0, cfg.nr - 1};
-    if ((e = alloc(&zone, sizeof(all_rows))) != hipSuccess) return e;
-    if ((e = hipMemcpy(zone, all_rows, sizeof(all_rows), hipMemcpyHostToDevice)) != hipSuccess)
-      return e;
+    if ((e = alloc(&zone, 4 * sizeof(int))) != hipSuccess) return e;
+    if ((e = all_rows()) != hipSuccess) return e;
     if ((e = alloc(&slots, D8 * kSlotsPerCase)) != hipSuccess) return e;
     // scratch the reference allocates once and never fully rewrites
     // (gradient and tau scratch keep zeros where they are never written)
@@ -882,6 +885,15 @@ struct SoftBatchT {
     return hipSuccess;
   }
 
+  hipError_t state_loaded(int id) {
+    for (const Entry& c : cases) {
+      if (c.id != id) continue;
+      hipError_t e = hipDeviceSynchronize();  // queued steps record their zones
+      return e == hipSuccess ? c.st->all_rows() : e;
+    }
+    return hipErrorInvalidValue;
+  }
+
   hipError_t remove(int id) {
     for (size_t k = 0; k < cases.size(); ++k) {
       if (cases[k].id != id) continue;
@@ -1155,15 +1167,25 @@ axs_status axs_soft_batch_add_f32(axs_soft_batch* bt, const axs_soft_config* c,
   return soft_batch_add(bt->f, c, b, case_id);
 }
 
-axs_status axs_soft_batch_remove(axs_soft_batch* bt, int case_id) {
-  AXS_CHECK_ARG(bt, "null batch");
-  const bool known = bt->with([&](const auto& b) {
+static bool has_case(const axs_soft_batch* bt, int case_id) {
+  return bt->with([&](const auto& b) {
     for (const auto& c : b.cases)
       if (c.id == case_id) return true;
     return false;
   });
-  AXS_CHECK_ARG(known, "no such case in the batch");
+}
+
+axs_status axs_soft_batch_remove(axs_soft_batch* bt, int case_id) {
+  AXS_CHECK_ARG(bt, "null batch");
+  AXS_CHECK_ARG(has_case(bt, case_id), "no such case in the batch");
   AXS_HIP(bt->with([&](auto& b) { return b.remove(case_id); }));
+  return AXS_OK;
+}
+
+axs_status axs_soft_batch_state_loaded(axs_soft_batch* bt, int case_id) {
+  AXS_CHECK_ARG(bt, "null batch");
+  AXS_CHECK_ARG(has_case(bt, case_id), "no such case in the batch");
+  AXS_HIP(bt->with([&](auto& b) { return b.state_loaded(case_id); }));
   return AXS_OK;
 }
 

@@ -112,7 +112,8 @@ __device__ __forceinline__ SoftBlock soft_block(const uint32_t* __restrict__ t) 
 
 // Rows of a case that the passes after the mirror (copy back, stress,
 // stress divergence) visit: the extrapolation's target
-// zone, recorded by the mirror pass of the same step, and kZoneMargin rows
+// zone, recorded by the mirror pass of the same step, the previous step's
+// (its stress is cleared where the zone has left), and kZoneMargin rows
 // either side; every row in the case's first step.  Beyond them the
 // reference map is zero (the copy back zeroes it outside the target zone,
 // and one step's ENO3 spreads it by two rows while the zone moves by less
@@ -123,12 +124,13 @@ constexpr int kZoneMargin = 6;
 template <class CaseT>
 __device__ __forceinline__ bool zone_row(const CaseT& C, int i) {
   if (C.scalars[kSsIt] == 0.0) return true;
-  return i >= C.zone[0] - kZoneMargin && i <= C.zone[1] + kZoneMargin;
+  return i >= min(C.zone[0], C.zone[2]) - kZoneMargin &&
+         i <= max(C.zone[1], C.zone[3]) + kZoneMargin;
 }
 // The passes before the mirror (reference-map ENO3, pin, the mirror
 // itself) go by the previous step's zone, two rows wider: the zone moves by
-// less than a row per step.  A case's zone starts as every row, so its first
-// step in a batch visits the whole grid even when its state was loaded.
+// less than a row per step.  A case's zone starts as every row, and is every
+// row again once a state was loaded (axs_soft_batch_state_loaded).
 template <class CaseT>
 __device__ __forceinline__ bool prev_zone_row(const CaseT& C, int i) {
   if (C.scalars[kSsIt] == 0.0) return true;

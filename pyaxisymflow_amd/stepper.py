@@ -776,6 +776,11 @@ class _SoftCaseView(_Checkpoint):
     def synchronize(self):
         self._batch.synchronize()
 
+    def load_state(self, state):
+        super().load_state(state)
+        if self._batch.cases.get(getattr(self, "id", None)) is self:
+            _lib.call("axs_soft_batch_state_loaded", self._batch._h, int(self.id))
+
     def _host(self, t):
         self._batch.synchronize()
         return t.cpu().numpy()

@@ -10,6 +10,10 @@ bit as that one does.
 * Soft sphere (single stepper, 128 x 64): 17 steps, checkpoint, 12 more.
 * Soft batch, FP32 bulk: a case checkpointed inside a three-case batch
   resumes in a batch of its own and matches the case left in the mix.
+* Soft batch: a case that has stepped takes a later state, whose solid
+  reaches more than 8 rows further out, and an earlier one (the passes of a
+  batch step visit the rows of the last step's solid and 8 more), and goes on
+  as a case of a new batch that takes the same state does.
 * Uneven batch (three grids, FP32): 13 steps, checkpoint, 9 more; the set-up
   layout searches are pinned (they time their candidates, and two steppers
   may pick different layouts, whose round-off differs).
@@ -110,6 +114,36 @@ def test_soft_batch_case_resumes_in_another_batch():
     assert case.steps_done() == moved.steps_done() == 16
     for k, v in case.state().items():
         assert np.array_equal(v, moved.state()[k]), k
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_soft_batch_case_that_has_stepped_takes_another_state(precision):
+    from pyaxisymflow_amd.stepper import SoftSphereBatch
+
+    params = dict(grid_size_z=256, G=0.1)
+
+    def zone(state):  # rows of the extrapolation's target zone, 8 dx around the solid
+        return int(np.flatnonzero((-state["phi"] < 8 / 256).any(axis=1))[-1])
+
+    run = SoftSphereBatch(max_cases=1, precision=precision)
+    case = run.add(**params)
+    run.step(2)
+    early = case.state()
+    run.step(600)
+    late = case.state()
+    print("last rows of the zone:", zone(early), zone(late), flush=True)
+    assert zone(late) > zone(early) + 10
+    for first, then in ((early, late), (late, early)):
+        case.load_state(first)
+        run.step(3)
+        case.load_state(then)
+        run.step(3)
+        fresh = SoftSphereBatch(max_cases=1, precision=precision)
+        new = fresh.add(**params)
+        new.load_state(then)
+        fresh.step(3)
+        for k, v in new.state().items():
+            assert np.array_equal(case.state()[k], v), k
 
 
 def test_wrong_state_is_refused():
